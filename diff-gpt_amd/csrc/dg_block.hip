@@ -276,10 +276,30 @@ __global__ __launch_bounds__(256) void attn_res_norm_split_kernel(const AttnResA
   }
 }
 
-// sigmoid as ATen evaluates it: 1 / (1 + exp(-x)) in fp32
-__device__ __forceinline__ float sigmoid_f32(float x) {
+// sigmoid rounded to T.  fp32: as ATen evaluates it, 1 / (1 + exp(-x)).  16-bit
+// types: the hardware exp2 and reciprocal (a few units of 2^-22, far below the
+// rounding to T that follows) in place of expf and a correctly rounded divide,
+// which at about 40 VALU instructions per element bounded the gate over a
+// prefill's rows (see gate_vec_kernel).
+template <typename T>
+__device__ __forceinline__ float sigmoid_rt(float x) {
 #pragma clang fp contract(off)
-  return 1.0f / (1.0f + expf(-x));
+  if constexpr (sizeof(T) == 4) {
+    return 1.0f / (1.0f + expf(-x));
+  } else {
+    return rt<T>(__builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x * -1.44269504f)));
+  }
+}
+
+// One SwiGLU element with the torch sequence's roundings (swi_glu.py:15-19).
+// clamp(max=limit) / clamp(-limit, limit) select existing values: exact.
+template <typename T>
+__device__ __forceinline__ float swiglu_value(float gate, float lin, float alpha, float limit) {
+#pragma clang fp contract(off)
+  gate = fminf(gate, limit);
+  lin = fminf(fmaxf(lin, -limit), limit);
+  const float s = sigmoid_rt<T>(rt<T>(alpha * gate));
+  return rt<T>(gate * s) * rt<T>(lin + 1.0f);
 }
 
 struct RowsArgs {
@@ -300,7 +320,7 @@ __global__ __launch_bounds__(256) void gate_kernel(const RowsArgs a) {
   const int64_t r = idx / a.N;
   const int c = (int)(idx - r * a.N);
   const float y = to_f32(static_cast<const T*>(a.x)[r * a.x_ld + c]);
-  const float s = rt<T>(sigmoid_f32(to_f32(static_cast<const T*>(a.g)[r * a.g_ld + c])));
+  const float s = sigmoid_rt<T>(to_f32(static_cast<const T*>(a.g)[r * a.g_ld + c]));
   static_cast<T*>(a.out)[r * a.out_ld + c] = from_f32<T>(y * s);
 }
 
@@ -312,14 +332,94 @@ __global__ __launch_bounds__(256) void swiglu_kernel(const RowsArgs a) {
   const int64_t r = idx / a.N;
   const int j = (int)(idx - r * a.N);
   const T* xr = static_cast<const T*>(a.x) + r * a.x_ld;
-  const float alpha = a.p0, limit = a.p1;
-  // clamp(max=limit) / clamp(-limit, limit) select existing values: exact
-  const float gate = fminf(to_f32(xr[2 * j]), limit);
-  const float lin = fminf(fmaxf(to_f32(xr[2 * j + 1]), -limit), limit);
-  const float s = rt<T>(sigmoid_f32(rt<T>(alpha * gate)));
-  const float gs = rt<T>(gate * s);
-  const float l1 = rt<T>(lin + 1.0f);
-  static_cast<T*>(a.out)[r * a.out_ld + j] = from_f32<T>(gs * l1);
+  static_cast<T*>(a.out)[r * a.out_ld + j] =
+      from_f32<T>(swiglu_value<T>(to_f32(xr[2 * j]), to_f32(xr[2 * j + 1]), a.p0, a.p1));
+}
+
+// gate_kernel and swiglu_kernel over rows of whole 16-byte vectors of their
+// input (aligned; the host checks): same values, same bits.  A thread takes U
+// vectors, 256 apart, all loaded before the first is used; the row and column
+// of the first come from one 32-bit division, those of the next by adding the
+// row and column steps of 256 vectors (drow, dcol).  One element per thread,
+// with a 64-bit division each and 2-byte accesses, ran at 2.3 TB/s: the gate of
+// 262144 bf16 rows of 512 (805 MB) took 348 us, here 172 (4.7 TB/s, a large copy's
+// rate).
+struct VecRowsArgs {
+  RowsArgs a;
+  uint32_t vectors, cols;  // vectors in all, and per row
+  uint32_t drow, dcol;     // 256 / cols, 256 % cols
+};
+
+template <typename T, int U>
+__global__ __launch_bounds__(256) void gate_vec_kernel(const VecRowsArgs v) {
+#pragma clang fp contract(off)
+  constexpr int E = 16 / (int)sizeof(T);
+  const RowsArgs& a = v.a;
+  const uint32_t idx = blockIdx.x * (256u * U) + threadIdx.x;
+  uint32_t r = idx / v.cols, c = idx - r * v.cols;
+  RowRegs<T, E> y[U], g[U];
+  T* o[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    o[u] = nullptr;
+    if (idx + 256u * u < v.vectors) {
+      load_row<T, E>(y[u], static_cast<const T*>(a.x) + (int64_t)r * a.x_ld + c * E);
+      load_row<T, E>(g[u], static_cast<const T*>(a.g) + (int64_t)r * a.g_ld + c * E);
+      o[u] = static_cast<T*>(a.out) + (int64_t)r * a.out_ld + c * E;
+    }
+    r += v.drow;
+    c += v.dcol;
+    if (c >= v.cols) {
+      c -= v.cols;
+      ++r;
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    if (o[u] == nullptr) continue;
+    float x[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) x[e] = elem<T, E>(y[u], e) * sigmoid_rt<T>(elem<T, E>(g[u], e));
+    RowRegs<T, E> p;
+    pack_row<T, E>(p, x);
+    store_row<T, E>(o[u], p);
+  }
+}
+
+template <typename T, int U>
+__global__ __launch_bounds__(256) void swiglu_vec_kernel(const VecRowsArgs v) {
+#pragma clang fp contract(off)
+  constexpr int E = 16 / (int)sizeof(T);  // input elements: E / 2 outputs
+  const RowsArgs& a = v.a;
+  const uint32_t idx = blockIdx.x * (256u * U) + threadIdx.x;
+  uint32_t r = idx / v.cols, c = idx - r * v.cols;
+  RowRegs<T, E> x[U];
+  T* o[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    o[u] = nullptr;
+    if (idx + 256u * u < v.vectors) {
+      load_row<T, E>(x[u], static_cast<const T*>(a.x) + (int64_t)r * a.x_ld + c * E);
+      o[u] = static_cast<T*>(a.out) + (int64_t)r * a.out_ld + c * (E / 2);
+    }
+    r += v.drow;
+    c += v.dcol;
+    if (c >= v.cols) {
+      c -= v.cols;
+      ++r;
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    if (o[u] == nullptr) continue;
+    float h[E / 2];
+#pragma unroll
+    for (int e = 0; e < E / 2; ++e)
+      h[e] = swiglu_value<T>(elem<T, E>(x[u], 2 * e), elem<T, E>(x[u], 2 * e + 1), a.p0, a.p1);
+    RowRegs<T, E / 2> p;
+    pack_row<T, E / 2>(p, h);
+    store_row<T, E / 2>(o[u], p);
+  }
 }
 
 template <typename T>
@@ -720,7 +820,7 @@ __global__ __launch_bounds__(256) void block_out_kernel(const BlockOutArgs a) {
 
   // 1) gate (gate_kernel's arithmetic)
 #pragma unroll
-  for (int i = 0; i < CH; ++i) y[i] = y[i] * rt<T>(sigmoid_f32(gl[i]));
+  for (int i = 0; i < CH; ++i) y[i] = y[i] * sigmoid_rt<T>(gl[i]);
   store_vec<T, CH>(ga + gr * LDC + gc0, y);
   __syncthreads();
   // 2) c_proj, then the partial sum
@@ -758,10 +858,7 @@ __global__ __launch_bounds__(256) void block_out_kernel(const BlockOutArgs a) {
     float hv[2];
 #pragma unroll
     for (int q = 0; q < 2; ++q) {
-      const float gate = fminf(rt<T>(acc[2 * q]), a.limit);
-      const float lin = fminf(fmaxf(rt<T>(acc[2 * q + 1]), -a.limit), a.limit);
-      const float s = rt<T>(sigmoid_f32(rt<T>(a.alpha * gate)));
-      hv[q] = rt<T>(gate * s) * rt<T>(lin + 1.0f);
+      hv[q] = swiglu_value<T>(rt<T>(acc[2 * q]), rt<T>(acc[2 * q + 1]), a.alpha, a.limit);
     }
     store_vec<T, 2>(hh + c * LDH + 8 * t + 2 * g, hv);
   }
@@ -939,6 +1036,51 @@ int launch_lm_head(const LmHeadArgs& a, hipStream_t s) {
     return check_launch(#K);                                                                  \
   } while (0)
 
+// Vectors per thread of the vector row kernels: 4 (64 bytes in flight per
+// input and lane) once the launch still fills the chip with them -- 1024
+// workgroups, 4 per CU -- else 1, so that a decode step's few rows spread over
+// as many CUs as they can.
+constexpr int64_t kVecRowsDeep = 4 * 256 * 1024;
+
+// The vector form of a row op whose input rows hold `in_cols` elements: K<T, U>
+// when they are whole 16-byte vectors (fewer than 2^31 in all) and every row
+// pointed to is aligned (out_align bytes for the output); false otherwise.
+bool vec_rows(const RowsArgs& a, int dtype, int64_t in_cols, int64_t out_align, VecRowsArgs& v) {
+  if (dtype == DG_F64) return false;
+  const int64_t es = dtype_bytes(dtype);
+  auto rows = [&](const void* p, int64_t ld, int64_t n) {
+    return p == nullptr || ((reinterpret_cast<uintptr_t>(p) % (uintptr_t)n) == 0 && (ld * es) % n == 0);
+  };
+  const int64_t cols = in_cols * es / 16;
+  if ((in_cols * es) % 16 != 0 || cols > 0x7fffffffLL || a.M > 0x7fffffffLL / cols) return false;
+  if (!rows(a.x, a.x_ld, 16) || !rows(a.g, a.g_ld, 16) || !rows(a.out, a.out_ld, out_align)) return false;
+  // the last workgroup counts past the end
+  if (a.M * cols > 0x7fffffffLL - 4 * 256) return false;
+  v.a = a;
+  v.vectors = (uint32_t)(a.M * cols);
+  v.cols = (uint32_t)cols;
+  v.drow = 256u / v.cols;
+  v.dcol = 256u % v.cols;
+  return true;
+}
+
+#define DG_LAUNCH_VEC_ROWS(K, dtype, v, s)                                                        \
+  do {                                                                                            \
+    const bool deep_ = (int64_t)(v).vectors >= kVecRowsDeep;                                      \
+    const unsigned blocks_ = ((v).vectors + (deep_ ? 1023u : 255u)) / (deep_ ? 1024u : 256u);     \
+    if ((dtype) == DG_F32) {                                                                      \
+      if (deep_) hipLaunchKernelGGL((K<float, 4>), dim3(blocks_), dim3(256), 0, (s), (v));        \
+      else hipLaunchKernelGGL((K<float, 1>), dim3(blocks_), dim3(256), 0, (s), (v));              \
+    } else if ((dtype) == DG_BF16) {                                                              \
+      if (deep_) hipLaunchKernelGGL((K<bf16_t, 4>), dim3(blocks_), dim3(256), 0, (s), (v));       \
+      else hipLaunchKernelGGL((K<bf16_t, 1>), dim3(blocks_), dim3(256), 0, (s), (v));             \
+    } else {                                                                                      \
+      if (deep_) hipLaunchKernelGGL((K<f16_t, 4>), dim3(blocks_), dim3(256), 0, (s), (v));        \
+      else hipLaunchKernelGGL((K<f16_t, 1>), dim3(blocks_), dim3(256), 0, (s), (v));              \
+    }                                                                                             \
+    return check_launch(#K);                                                                      \
+  } while (0)
+
 bool dtype_ok(int dtype) { return dtype == DG_F32 || dtype == DG_BF16 || dtype == DG_F16; }
 // the row kernels with float64 forms (dg_attn_res_norm, dg_gate, dg_swiglu, dg_softcap)
 bool dtype_ok_f64(int dtype) { return dtype_ok(dtype) || dtype == DG_F64; }
@@ -995,7 +1137,10 @@ extern "C" int dg_gate(int64_t M, int C, int dtype, const void* y, int64_t y_ld,
   RowsArgs a{};
   a.x = y; a.g = g; a.out = out;
   a.x_ld = y_ld; a.g_ld = g_ld; a.out_ld = out_ld; a.M = M; a.N = C;
-  DG_LAUNCH_ROWS(gate_kernel, dtype, a, static_cast<hipStream_t>(stream));
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  VecRowsArgs v;
+  if (vec_rows(a, dtype, C, 16, v)) DG_LAUNCH_VEC_ROWS(gate_vec_kernel, dtype, v, s);
+  DG_LAUNCH_ROWS(gate_kernel, dtype, a, s);
 }
 
 extern "C" int dg_swiglu(int64_t M, int N, int dtype, const void* x, int64_t x_ld, void* out,
@@ -1010,7 +1155,10 @@ extern "C" int dg_swiglu(int64_t M, int N, int dtype, const void* x, int64_t x_l
   a.x_ld = x_ld; a.out_ld = out_ld; a.M = M; a.N = N;
   a.p0 = (float)alpha; a.p1 = (float)limit;
   a.d0 = alpha; a.d1 = limit;
-  DG_LAUNCH_ROWS(swiglu_kernel, dtype, a, static_cast<hipStream_t>(stream));
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  VecRowsArgs v;
+  if (vec_rows(a, dtype, 2 * (int64_t)N, 8, v)) DG_LAUNCH_VEC_ROWS(swiglu_vec_kernel, dtype, v, s);
+  DG_LAUNCH_ROWS(swiglu_kernel, dtype, a, s);
 }
 
 extern "C" int dg_softcap(int64_t M, int N, int dtype, const void* x, int64_t x_ld, void* out,

@@ -1,0 +1,62 @@
+"""The vector forms of the row kernels around attention (dg_block.hip) against
+their general forms on the same values, at the sizes where a vector form can go
+wrong: rows whose vector count does not divide the workgroup, one row, launches
+with one and with four vectors per thread, and a last workgroup that is partly
+empty.  The general form runs on rows one element off their alignment."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+TDT = {"f32": torch.float32, "bf16": torch.bfloat16, "f16": torch.float16}
+
+
+def _rows(M, C, dtype, dev, seed, offset, scale=3.0):
+    """(M, C) values that depend on the seed alone, rows ``offset`` elements off a
+    16-byte boundary (the row stride is a multiple of 16 bytes)."""
+    g = torch.Generator(device=dev).manual_seed(seed)
+    x = (torch.randn(M, C, generator=g, device=dev) * scale).to(dtype)
+    wide = torch.zeros(M, C + 8, dtype=dtype, device=dev)
+    wide[:, offset : offset + C] = x
+    return wide[:, offset : offset + C]
+
+
+SHAPES = [(1, 8), (3, 24), (1, 512), (37, 200), (4100, 64), (131075, 64), (2051, 4104)]
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("M,C", SHAPES, ids=lambda v: str(v))
+def test_gate_and_swiglu_vector_rows_equal_the_general_form(dev, dtype, M, C):
+    from diff_gpt import _native
+
+    dt = TDT[dtype]
+    got, ref = (_rows(M, C, dt, dev, 1, off) for off in (0, 1))
+    ga, gb = (_rows(M, C, dt, dev, 2, off) for off in (0, 1))
+    _native.gate_(got, ga)
+    _native.gate_(ref, gb)
+    assert torch.equal(got, ref)
+    xa, xb = (_rows(M, C, dt, dev, 3, off) for off in (0, 1))
+    oa, ob = (torch.empty(M, C // 2, dtype=dt, device=dev) for _ in range(2))
+    _native.swiglu_(xa, oa, 1.702, 7.0)
+    _native.swiglu_(xb, ob, 1.702, 7.0)
+    assert torch.equal(oa, ob)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16", "f16"])
+def test_gate_limits(dev, dtype):
+    """sigmoid at infinities, NaN and arguments beyond exp's range: the values of
+    torch's own sequence within one rounding of the type (2^-7, 2^-10 or, for
+    fp32, 4 ulps of 2^-23, relative)."""
+    from diff_gpt import _native
+
+    g = torch.tensor([float("inf"), float("-inf"), float("nan"), 0.0, -0.0, 88.0, -86.0, 200.0, -200.0, 3e4, -3e4,
+                      1e-6, -1e-6, 1.5, -1.5, 9.0] * 4, dtype=TDT[dtype])
+    y = torch.full_like(g, 1.25)
+    got = y.to(dev).view(1, -1).clone()
+    _native.gate_(got, g.to(dev).view(1, -1))
+    ref = (y * torch.sigmoid(g)).view(1, -1)
+    tol = {"f32": 2.0**-21, "bf16": 2.0**-7, "f16": 2.0**-10}[dtype]
+    assert torch.equal(got.isnan().cpu(), ref.isnan())
+    d = (got.cpu().double() - ref.double()).abs().nan_to_num(0.0)
+    assert bool((d <= tol * ref.double().abs().nan_to_num(0.0) + torch.finfo(TDT[dtype]).tiny).all())
