@@ -38,6 +38,7 @@ struct AttnResArgs {
   void* out;
   int64_t out_ld, M;
   int nsrc, N;
+  int dup;  // 1 when source 1 is source 0 (same rows): read once
 };
 
 // round-trip through the storage dtype
@@ -77,8 +78,7 @@ __device__ __forceinline__ void load_slice(const T* p, int c0, int N, bool vec, 
 // Sources a lane loads into registers together, up front, to serve both
 // passes of the mixture (one round trip to memory for them, instead of one
 // per source and pass): about 32 registers of slices inside dg_block_out,
-// whose GEMM stages need the rest, and about 64 in attn_res_norm_kernel (at
-// n_embd 512, bf16, 10 sources took 21 us with 4 held).
+// whose GEMM stages need the rest, and about 64 in attn_res_norm_kernel.
 template <int CH>
 constexpr int res_held() {
   return CH <= 4 ? 8 : CH <= 8 ? 4 : CH <= 16 ? 2 : 1;
@@ -88,78 +88,136 @@ constexpr int res_held_norm() {
   return CH <= 4 ? 16 : CH <= 8 ? 8 : CH <= 16 ? 4 : CH <= 32 ? 2 : 1;
 }
 
-template <typename T, int NPAD, int CH>
+// The mixture's arithmetic on a lane's slices as they are stored, the same in
+// its three kernels (so they agree bit for bit), each intermediate rounded to
+// T where its torch tensor is.  16-bit types work on packed pairs: the squares
+// and the products with w by v_dot2_f32_{bf16,f16} (exact products, fp32
+// sums), each rounding by one conversion of a pair.
+
+// sum of the slice's squares
+template <typename T, int CH>
+__device__ __forceinline__ float slice_squares(const RowRegs<T, CH>& x) {
+  return slice_dot<T, CH>(x, x);
+}
+// sum of rt(x r) w over the slice: the normalised row against the pseudo-query
+template <typename T, int CH>
+__device__ __forceinline__ float slice_score(const RowRegs<T, CH>& x, float r, const RowRegs<T, CH>& w) {
+#pragma clang fp contract(off)
+  float v[CH];
+#pragma unroll
+  for (int i = 0; i < CH; ++i) v[i] = elem<T, CH>(x, i) * r;
+  RowRegs<T, CH> n;
+  pack_row<T, CH>(n, v);
+  return slice_dot<T, CH>(n, w);
+}
+// h += rt(p x)
+template <typename T, int CH>
+__device__ __forceinline__ void slice_add(float (&h)[CH], float p, const RowRegs<T, CH>& x) {
+#pragma clang fp contract(off)
+  float v[CH];
+#pragma unroll
+  for (int i = 0; i < CH; ++i) v[i] = p * elem<T, CH>(x, i);
+  RowRegs<T, CH> n;
+  pack_row<T, CH>(n, v);
+#pragma unroll
+  for (int i = 0; i < CH; ++i) h[i] = h[i] + elem<T, CH>(n, i);
+}
+// the slice at p (elements c0 .. of a row of N), zeros past N
+template <typename T, int CH>
+__device__ __forceinline__ void load_packed(RowRegs<T, CH>& r, const T* p, int c0, int N, bool vec) {
+  if (vec && c0 + CH <= N) {
+    load_row<T, CH>(r, p);
+  } else {
+    float v[CH];
+#pragma unroll
+    for (int i = 0; i < CH; ++i) v[i] = (c0 + i < N) ? to_f32(p[i]) : 0.f;
+    pack_row<T, CH>(r, v);
+  }
+}
+// Sum over the G lanes of a row.  G = 64: halves and 16-lane rows first, in
+// the order attn_res_norm_wave_kernel folds several sums at once.
+__device__ __forceinline__ float row16_sum(float v) {
+  v = v + dpp<kDppQuadXor1>(v);
+  v = v + dpp<kDppQuadXor2>(v);
+  v = v + dpp<kDppHalfMirror>(v);
+  return v + dpp<kDppMirror>(v);
+}
+template <int G>
+__device__ __forceinline__ float score_sum(float v) {
+  if constexpr (G == 64) {
+    float a, b;
+    pair32(v, a, b);
+    v = a + b;
+    pair16(v, a, b);
+    return row16_sum(a + b);
+  } else {
+    return group_sum_dpp<G>(v);
+  }
+}
+__device__ __forceinline__ float row_factor(float ss, int N) {
+#pragma clang fp contract(off)
+  return 1.0f / sqrtf(ss / (float)N + FLT_EPSILON);
+}
+
+// NS: the most sources of the instance (the launch's fit).
+template <typename T, int NPAD, int CH, int NS>
 __global__ __launch_bounds__(256) void attn_res_norm_kernel(const AttnResArgs a, const int vec) {
 #pragma clang fp contract(off)
   constexpr int G = NPAD / CH;
-  constexpr int HELD = res_held_norm<CH>();
+  constexpr int HELD = res_held_norm<CH>() < NS ? res_held_norm<CH>() : NS;
   static_assert(G >= 1 && G <= 64, "row mapping");
   constexpr int ROWS_PER_BLOCK = 256 / G;
   const int sub = threadIdx.x % G;
   const int64_t row = (int64_t)blockIdx.x * ROWS_PER_BLOCK + threadIdx.x / G;
   if (row >= a.M) return;  // whole lane groups leave together; no barriers
   const int c0 = sub * CH;
-  auto load = [&](int n, float (&x)[CH]) __attribute__((always_inline)) {
-    load_slice<T, CH>(static_cast<const T*>(a.src[n]) + row * a.ld[n] + c0, c0, a.N, vec, x);
+  auto load = [&](int n, RowRegs<T, CH>& x) __attribute__((always_inline)) {
+    load_packed<T, CH>(x, static_cast<const T*>(a.src[n]) + row * a.ld[n] + c0, c0, a.N, vec);
   };
-  float held[HELD][CH];
+  RowRegs<T, CH> held[HELD], w;
 #pragma unroll
   for (int n = 0; n < HELD; ++n)
     if (n < a.nsrc) load(n, held[n]);  // uniform; no use before all are issued
-  auto get = [&](int n, float (&x)[CH]) __attribute__((always_inline)) {
-    if (n < HELD) {
-#pragma unroll
-      for (int i = 0; i < CH; ++i) x[i] = held[n][i];
-    } else {
-      load(n, x);
-    }
+  auto get = [&](int n, RowRegs<T, CH>& x) __attribute__((always_inline)) {
+    if (n < HELD) x = held[n];
+    else load(n, x);
   };
-  float w[CH];
-  load_slice<T, CH>(static_cast<const T*>(a.w) + c0, c0, a.N, vec, w);
+  load_packed<T, CH>(w, static_cast<const T*>(a.w) + c0, c0, a.N, vec);
 
   // pass 1: score_n = rms_norm(V_n) . w, each rounded as its tensor is
-  float score[kMaxResSources];
+  float score[NS];
   float mx = -INFINITY;
 #pragma unroll
-  for (int n = 0; n < kMaxResSources; ++n) {
+  for (int n = 0; n < NS; ++n) {
     score[n] = -INFINITY;
     if (n >= a.nsrc) continue;  // uniform
-    float x[CH];
+    RowRegs<T, CH> x;
     get(n, x);
-    row_rms<CH, G>(x, a.N);
-    float prod[CH];
-#pragma unroll
-    for (int i = 0; i < CH; ++i) prod[i] = rt<T>(x[i]) * w[i];
-    float dot = tree_sum<CH>(prod);
-    dot = group_sum_dpp<G>(dot);
-    score[n] = rt<T>(dot);
+    const float r = row_factor(score_sum<G>(slice_squares<T, CH>(x)), a.N);
+    score[n] = rt<T>(score_sum<G>(slice_score<T, CH>(x, r, w)));
     mx = fmaxf(mx, score[n]);
   }
   // softmax over the sources (fp32 inside, rounded output)
-  float e[kMaxResSources];
   float sum = 0.f;
 #pragma unroll
-  for (int n = 0; n < kMaxResSources; ++n) {
-    e[n] = 0.f;
+  for (int n = 0; n < NS; ++n) {
     if (n >= a.nsrc) continue;
-    e[n] = expf(score[n] - mx);
-    sum += e[n];
+    score[n] = expf(score[n] - mx);
+    sum += score[n];
   }
-  // pass 2: h = sum_n rt(p_n * V_n), fp32 sum in source order, rounded
+  // pass 2: h = sum_n rt(p_n V_n), fp32 sum in source order, rounded
   float h[CH];
 #pragma unroll
   for (int i = 0; i < CH; ++i) h[i] = 0.f;
 #pragma unroll
-  for (int n = 0; n < kMaxResSources; ++n) {
+  for (int n = 0; n < NS; ++n) {
     if (n >= a.nsrc) continue;
-    const float p = rt<T>(e[n] / sum);
-    float x[CH];
+    RowRegs<T, CH> x;
     get(n, x);
-#pragma unroll
-    for (int i = 0; i < CH; ++i) h[i] = h[i] + rt<T>(p * x[i]);
+    slice_add<T, CH>(h, rt<T>(score[n] / sum), x);
   }
 #pragma unroll
-  for (int i = 0; i < CH; ++i) h[i] = (c0 + i < a.N) ? rt<T>(h[i]) : 0.f;
+  for (int i = 0; i < CH; ++i) h[i] = rt<T>(h[i]);
   row_rms<CH, G>(h, a.N);
   T* os = static_cast<T*>(a.out) + row * a.out_ld + c0;
   if (vec && c0 + CH <= a.N) {
@@ -171,11 +229,101 @@ __global__ __launch_bounds__(256) void attn_res_norm_kernel(const AttnResArgs a,
   }
 }
 
+// attn_res_norm_kernel for rows that fill a wave (G = 64 lanes of CH elements,
+// aligned) with at most NS sources, every one held in registers as loaded.
+// A row's sums fold together: each step of the cross-lane
+// reduction halves the number of registers (v_permlane32_swap hands the low
+// half of the wave one sum and the high half another, v_permlane16_swap the
+// same for rows of 16 lanes), so four sources cost the DPP steps of one, and
+// the four 16-lane rows then take the square roots, exponentials and
+// quotients of four sources at once.  Near HBM's rate at a prefill's sizes: 65536
+// bf16 rows of 512 with 6 sources, 5 of them distinct (403 MB), take 101 us
+// (4.0 TB/s), 28672 rows of 1024 with 4 (235 MB) 52 us (4.5 TB/s); one source at
+// a time, with its own reductions and fp32 copies in registers, they took 237
+// and 110.  NS = 4, 6, 8 or 12 sources and 96 registers of them: beyond either
+// the general form's.
+template <typename T, int CH, int NS>
+__global__ __launch_bounds__(256) void attn_res_norm_wave_kernel(const AttnResArgs a) {
+#pragma clang fp contract(off)
+  constexpr int NG = (NS + 3) / 4;  // groups of four sources
+  const int lane = threadIdx.x & 63;
+  const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (row >= a.M) return;  // whole waves leave; no barriers
+  const int c0 = lane * CH;
+  RowRegs<T, CH> v[NS], w;
+#pragma unroll
+  for (int n = 0; n < NS; ++n) {
+    if (n >= a.nsrc) {  // uniform
+#pragma unroll
+      for (int i = 0; i < RowRegs<T, CH>::WORDS; ++i) v[n].w[i] = 0u;
+    } else if (n == 1 && a.dup) {
+      v[1] = v[0];
+    } else {
+      load_row<T, CH>(v[n], static_cast<const T*>(a.src[n]) + row * a.ld[n] + c0);
+    }
+  }
+  load_row<T, CH>(w, static_cast<const T*>(a.w) + c0);
+  // the sums of sources 4k .. 4k + 3 in 16-lane rows 0, 2, 1, 3 of one register
+  auto fold4 = [](float s0, float s1, float s2, float s3) __attribute__((always_inline)) {
+    auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(s0), __float_as_uint(s1), false, false);
+    const float t0 = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    r = __builtin_amdgcn_permlane32_swap(__float_as_uint(s2), __float_as_uint(s3), false, false);
+    const float t1 = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    r = __builtin_amdgcn_permlane16_swap(__float_as_uint(t0), __float_as_uint(t1), false, false);
+    return row16_sum(__uint_as_float(r[0]) + __uint_as_float(r[1]));
+  };
+  auto of_source = [](const float (&x)[NG], int n) __attribute__((always_inline)) {
+    const int lane0 = 16 * (((n & 1) << 1) | ((n >> 1) & 1));
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x[n / 4]), lane0));
+  };
+  const int q = lane >> 4, in4 = ((q & 1) << 1) | (q >> 1);  // this 16-lane row's source of each four
+  float part[4 * NG], sc[NG];
+#pragma unroll
+  for (int n = 0; n < 4 * NG; ++n) part[n] = n < NS ? slice_squares<T, CH>(v[n < NS ? n : 0]) : 0.f;
+#pragma unroll
+  for (int k = 0; k < NG; ++k)
+    sc[k] = row_factor(fold4(part[4 * k], part[4 * k + 1], part[4 * k + 2], part[4 * k + 3]), a.N);
+#pragma unroll
+  for (int n = 0; n < NS; ++n) part[n] = slice_score<T, CH>(v[n], of_source(sc, n), w);
+  float mx = -INFINITY;
+#pragma unroll
+  for (int k = 0; k < NG; ++k) {
+    const float d = fold4(part[4 * k], part[4 * k + 1], part[4 * k + 2], part[4 * k + 3]);
+    sc[k] = 4 * k + in4 < a.nsrc ? rt<T>(d) : -INFINITY;
+    mx = fmaxf(mx, sc[k]);
+  }
+  {
+    float x, y;
+    pair16(mx, x, y);
+    mx = fmaxf(x, y);
+    pair32(mx, x, y);
+    mx = fmaxf(x, y);
+  }
+  float sum = 0.f;
+#pragma unroll
+  for (int k = 0; k < NG; ++k) sc[k] = expf(sc[k] - mx);
+#pragma unroll
+  for (int n = 0; n < NS; ++n)
+    if (n < a.nsrc) sum += of_source(sc, n);
+#pragma unroll
+  for (int k = 0; k < NG; ++k) sc[k] = rt<T>(sc[k] / sum);
+  float h[CH];
+#pragma unroll
+  for (int i = 0; i < CH; ++i) h[i] = 0.f;
+#pragma unroll
+  for (int n = 0; n < NS; ++n)
+    if (n < a.nsrc) slice_add<T, CH>(h, of_source(sc, n), v[n]);  // uniform
+#pragma unroll
+  for (int i = 0; i < CH; ++i) h[i] = rt<T>(h[i]);
+  row_rms<CH, 64>(h, a.N);
+  store_vec<T, CH>(static_cast<T*>(a.out) + row * a.out_ld + c0, h);
+}
+
 // attn_res_norm_kernel for few wide rows (one row per wave there, G = 64):
 // a workgroup of 4 waves takes one row, so a decode step's few hundred rows
 // keep four times the waves in flight and each wave's dependent chain of
 // per-source reductions is a quarter as long.  Wave w scores sources w,
-// w + 4, ... (each in the lane mapping, arithmetic and reduction tree of
+// w + 4, ... (each in the lane mapping, arithmetic and reduction order of
 // attn_res_norm_kernel, so each score has its bits); the scores meet in LDS;
 // every wave takes the softmax over them in source order; wave w forms the
 // weighted sum for a quarter of the columns (each column summed over the
@@ -200,12 +348,12 @@ __global__ __launch_bounds__(256) void attn_res_norm_split_kernel(const AttnResA
   const int wv = threadIdx.x >> 6;
   const int64_t row = blockIdx.x;  // the host launches one workgroup per row
   const int c0 = lane * CH;
-  float w[CH];
-  load_slice<T, CH>(static_cast<const T*>(a.w) + c0, c0, a.N, vec, w);
-  auto load = [&](int n, float (&x)[CH]) __attribute__((always_inline)) {
-    load_slice<T, CH>(static_cast<const T*>(a.src[n]) + row * a.ld[n] + c0, c0, a.N, vec, x);
+  RowRegs<T, CH> w;
+  load_packed<T, CH>(w, static_cast<const T*>(a.w) + c0, c0, a.N, vec);
+  auto load = [&](int n, RowRegs<T, CH>& x) __attribute__((always_inline)) {
+    load_packed<T, CH>(x, static_cast<const T*>(a.src[n]) + row * a.ld[n] + c0, c0, a.N, vec);
   };
-  float held[HELD][CH];
+  RowRegs<T, CH> held[HELD];
 #pragma unroll
   for (int j = 0; j < HELD; ++j)
     if (wv + 4 * j < a.nsrc) load(wv + 4 * j, held[j]);  // wave-uniform; no use before all are issued
@@ -214,23 +362,15 @@ __global__ __launch_bounds__(256) void attn_res_norm_split_kernel(const AttnResA
   for (int j = 0; j < kMaxResSources / 4; ++j) {
     const int n = wv + 4 * j;
     if (n >= a.nsrc) break;  // wave-uniform
-    float x[CH];
-    if (j < HELD) {
-#pragma unroll
-      for (int i = 0; i < CH; ++i) x[i] = held[j][i];
-    } else {
-      load(n, x);
-    }
-    row_rms<CH, G>(x, a.N);
-    float prod[CH];
-#pragma unroll
-    for (int i = 0; i < CH; ++i) prod[i] = rt<T>(x[i]) * w[i];
-    float dot = tree_sum<CH>(prod);
-    dot = group_sum_dpp<G>(dot);
-    if (lane == 0) sc[n] = rt<T>(dot);
+    RowRegs<T, CH> x;
+    if (j < HELD) x = held[j];
+    else load(n, x);
+    const float r = row_factor(score_sum<G>(slice_squares<T, CH>(x)), a.N);
+    const float score = rt<T>(score_sum<G>(slice_score<T, CH>(x, r, w)));
+    if (lane == 0) sc[n] = score;
   }
   __syncthreads();
-  // softmax over the sources (fp32 inside, rounded output), in source order
+  // softmax over the sources, in source order
   float mx = -INFINITY;
 #pragma unroll
   for (int n = 0; n < kMaxResSources; ++n)
@@ -559,8 +699,31 @@ int launch_res(const AttnResArgs& a, hipStream_t s) {
       return check_launch("attn_res_norm_split_kernel");
     }
   }
-  hipLaunchKernelGGL((attn_res_norm_kernel<T, NPAD, CH>), dim3((unsigned)blocks), dim3(256), 0, s, a,
-                     vec ? 1 : 0);
+  if constexpr (G == 64 && CH * (int)sizeof(T) >= 16) {
+    // rows that fill a wave, every source in registers (at most 96 of them)
+    if (vec && a.N == NPAD) {
+      constexpr int WORDS = RowRegs<T, CH>::WORDS;
+#define DG_RES_WAVE(NS)                                                                                         \
+  if constexpr (WORDS * NS <= 96) {                                                                             \
+    if (a.nsrc <= NS) {                                                                                         \
+      hipLaunchKernelGGL((attn_res_norm_wave_kernel<T, CH, NS>), dim3((unsigned)blocks), dim3(256), 0, s, a);   \
+      return check_launch("attn_res_norm_wave_kernel");                                                         \
+    }                                                                                                           \
+  }
+      DG_RES_WAVE(4)
+      DG_RES_WAVE(6)
+      DG_RES_WAVE(8)
+      DG_RES_WAVE(12)
+#undef DG_RES_WAVE
+    }
+  }
+  // the unrolled loops as long as the sources need (few in a shallow model)
+  if (a.nsrc <= 4)
+    hipLaunchKernelGGL((attn_res_norm_kernel<T, NPAD, CH, 4>), dim3((unsigned)blocks), dim3(256), 0, s, a,
+                       vec ? 1 : 0);
+  else
+    hipLaunchKernelGGL((attn_res_norm_kernel<T, NPAD, CH, kMaxResSources>), dim3((unsigned)blocks), dim3(256), 0, s,
+                       a, vec ? 1 : 0);
   return check_launch("attn_res_norm_kernel");
 }
 
@@ -1115,6 +1278,7 @@ extern "C" int dg_attn_res_norm(int64_t M, int C, int dtype, int nsrc, const voi
   a.M = M;
   a.nsrc = nsrc;
   a.N = C;
+  a.dup = nsrc > 1 && src[1] == src[0] && src_ld[1] == src_ld[0] ? 1 : 0;
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (dtype == DG_F64) {
     DG_REQUIRE((M + 3) / 4 <= 0x7fffffffLL, DG_EINVAL, "attn_res_norm: too many rows (%lld)", (long long)M);

@@ -388,7 +388,8 @@ DG_API int dg_copy4d(int dtype, const int64_t* shape, const void* src,
  * softmax over the sources, weighted sum) followed by rms_norm.py:5-7, for the
  * nsrc sources V_n = src[n] (rows of C elements, row stride src_ld[n]) in the
  * order block_attn_res stacks them (committed blocks, then the partial sum).
- * The RMSNorms give dg_rms_norm's bits for the same row.
+ * The RMSNorm of the mixture gives dg_rms_norm's bits for the same row (the
+ * sources' norms, inside their scores, sum in another order).
  * Supported: C <= 2048, 1 <= nsrc <= 32.
  */
 DG_API int dg_attn_res_norm(int64_t M, int C, int dtype, int nsrc, const void* const* src,

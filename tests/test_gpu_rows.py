@@ -60,3 +60,30 @@ def test_gate_limits(dev, dtype):
     assert torch.equal(got.isnan().cpu(), ref.isnan())
     d = (got.cpu().double() - ref.double()).abs().nan_to_num(0.0)
     assert bool((d <= tol * ref.double().abs().nan_to_num(0.0) + torch.finfo(TDT[dtype]).tiny).all())
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("C", [64, 256, 512, 1024, 2048])
+@pytest.mark.parametrize("n", [1, 2, 4, 5, 7, 8, 12, 13])
+def test_mixture_forms_agree(dev, dtype, C, n):
+    """Aligned full-width rows (every source held in registers where they fit),
+    rows off their alignment (the general form) and few rows (a workgroup per
+    row) give the same bits, with source 1 being source 0 itself or a copy of
+    it."""
+    from diff_gpt import _native
+
+    dt, M = TDT[dtype], 4099
+    aligned, shifted = ([_rows(M, C, dt, dev, 50 + i, off, 0.5 + 0.2 * i) for i in range(n)] for off in (0, 1))
+    if n > 1:
+        aligned[1], shifted[1] = aligned[0], shifted[0]
+    copied = [s.clone() for s in aligned]  # no two are the same rows
+    w = torch.randn(1, C, generator=torch.Generator(device=dev).manual_seed(9), device=dev).to(dt)
+    outs = []
+    for srcs in (aligned, shifted, copied):
+        out = torch.empty(M, C, dtype=dt, device=dev)
+        _native.attn_res_norm_(srcs, w, out)
+        outs.append(out)
+    few = torch.empty(33, C, dtype=dt, device=dev)
+    _native.attn_res_norm_([s[:33] for s in aligned], w, few)
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+    assert torch.equal(outs[0][:33], few)
