@@ -82,7 +82,8 @@ bool mfma_prefill_rope_applicable(int B, int H, int Tq, int Tk, int D, int dtype
 int mfma_prefill_rope(int B, int H, int Tq, int Tk, int D, int dtype, const void* q, const dg_stride3* q_st,
                       const void* freqs, const dg_stride3* f_st, int fdtype, int qknorm, int keys_normed,
                       const void* k, const dg_stride3* k_st, const void* v, const dg_stride3* v_st, void* y,
-                      const dg_stride3* y_st, float scale, hipStream_t s);
+                      const dg_stride3* y_st, float scale, const void* gate, const dg_stride3* g_st,
+                      hipStream_t s);
 
 // ---------------------------------------------------------------------------
 // Strided 4-D copy (exact), element size 2, 4 or 8 bytes.
@@ -213,11 +214,11 @@ extern "C" int dg_attention_grouped(int B, int H, int Tq, int Tk, int D, int dty
                        workspace, workspace_bytes, Tk, s);
 }
 
-extern "C" int dg_prefill_rope(int B, int H, int Tq, int Tk, int D, int dtype, const void* q,
-                               const dg_stride3* q_st, const void* freqs, const dg_stride3* f_st,
+static int prefill_rope_impl(int B, int H, int Tq, int Tk, int D, int dtype, const void* q,
+                             const dg_stride3* q_st, const void* freqs, const dg_stride3* f_st,
                                int freqs_dtype, int flags, const void* k, const dg_stride3* k_st,
                                const void* v, const dg_stride3* v_st, void* y, const dg_stride3* y_st,
-                               float scale, void* stream) {
+                               float scale, const void* gate, const dg_stride3* g_st, void* stream) {
   DG_REQUIRE(B >= 0 && H >= 0 && Tq >= 0 && Tk >= 0, DG_EINVAL, "prefill_rope: negative size");
   DG_REQUIRE(dtype == DG_F32 || dtype == DG_BF16 || dtype == DG_F16, DG_EUNSUPPORTED,
              "prefill_rope: dtype %d unsupported", dtype);
@@ -236,9 +237,35 @@ extern "C" int dg_prefill_rope(int B, int H, int Tq, int Tk, int D, int dtype, c
              DG_EUNSUPPORTED,
              "prefill_rope: not taken by the fused kernels (bf16/fp16/fp32, head_dim 64 or 128, Tq >= 16, "
              "16-byte aligned rows); use dg_rope_qknorm_append + dg_attention");
+  if (gate != nullptr) {
+    const int64_t n = 16 / dtype_bytes(dtype);
+    DG_REQUIRE(g_st != nullptr, DG_EINVAL, "prefill_rope_gate: NULL strides");
+    DG_REQUIRE((reinterpret_cast<uintptr_t>(gate) & 15) == 0 && g_st->b % n == 0 && g_st->t % n == 0 &&
+                   g_st->h % n == 0,
+               DG_EUNSUPPORTED, "prefill_rope_gate: gate rows must be 16-byte aligned");
+  }
   return mfma_prefill_rope(B, H, Tq, Tk, D, dtype, q, q_st, freqs, f_st, freqs_dtype, (flags & DG_QKNORM) != 0,
-                           (flags & DG_KEYS_NORMED) != 0, k, k_st, v, v_st, y, y_st, scale,
+                           (flags & DG_KEYS_NORMED) != 0, k, k_st, v, v_st, y, y_st, scale, gate, g_st,
                            static_cast<hipStream_t>(stream));
+}
+
+extern "C" int dg_prefill_rope(int B, int H, int Tq, int Tk, int D, int dtype, const void* q,
+                               const dg_stride3* q_st, const void* freqs, const dg_stride3* f_st,
+                               int freqs_dtype, int flags, const void* k, const dg_stride3* k_st,
+                               const void* v, const dg_stride3* v_st, void* y, const dg_stride3* y_st,
+                               float scale, void* stream) {
+  return prefill_rope_impl(B, H, Tq, Tk, D, dtype, q, q_st, freqs, f_st, freqs_dtype, flags, k, k_st, v, v_st, y,
+                           y_st, scale, nullptr, nullptr, stream);
+}
+
+extern "C" int dg_prefill_rope_gate(int B, int H, int Tq, int Tk, int D, int dtype, const void* q,
+                                    const dg_stride3* q_st, const void* freqs, const dg_stride3* f_st,
+                                    int freqs_dtype, int flags, const void* k, const dg_stride3* k_st,
+                                    const void* v, const dg_stride3* v_st, void* y, const dg_stride3* y_st,
+                                    float scale, const void* gate, const dg_stride3* g_st, void* stream) {
+  DG_REQUIRE((int64_t)B * H * Tq <= 0 || gate != nullptr, DG_EINVAL, "prefill_rope_gate: NULL gate");
+  return prefill_rope_impl(B, H, Tq, Tk, D, dtype, q, q_st, freqs, f_st, freqs_dtype, flags, k, k_st, v, v_st, y,
+                           y_st, scale, gate, g_st, stream);
 }
 
 extern "C" size_t dg_decode_attention_at_workspace_size(int B, int H, int max_keys, int D, int dtype) {

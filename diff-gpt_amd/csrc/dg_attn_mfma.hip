@@ -676,8 +676,20 @@ void prefill_mfma_kernel(const PrefillArgs a) {
   static_assert(32 * D <= C::TILE, "a stage array holds one wave's output rows");
   uint16_t* stg = wv == 0 ? ks0 : wv == 1 ? vs0 : wv == 2 ? ks1 : vs1;
   T* yb0 = static_cast<T*>(a.y) + b * a.yb + (int64_t)head * a.yh;
+  const int piece = lane % PPQ;
 #pragma unroll
   for (int qb = 0; qb < QW; ++qb) {
+    // the gate's rows in the store's layout, in flight while the output passes
+    // through LDS.  Applied here the gate costs its own read alone; as a launch
+    // of its own it reads and writes y once more (measured: attention and
+    // gate of 256 x 1024 rows of 8 x 64 in bf16, 350 + 172 us apart)
+    RowRegs<T, 8> gv[32 / RPS];
+    if (a.gate != nullptr) {  // uniform over the grid
+      const T* gb0 = static_cast<const T*>(a.gate) + b * a.gb + (int64_t)head * a.gh + 8 * piece;
+#pragma unroll
+      for (int p = 0; p < 32 / RPS; ++p)
+        load_row<T, 8>(gv[p], gb0 + (int64_t)min(qw + 32 * qb + p * RPS + lane / PPQ, a.Tq - 1) * a.gt);
+    }
     // rows past Tq carry finite values and are not stored
     const float inv = __builtin_amdgcn_rcpf(half_pair_sum(l[qb]));
 #pragma unroll
@@ -693,13 +705,14 @@ void prefill_mfma_kernel(const PrefillArgs a) {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    const int piece = lane % PPQ;
 #pragma unroll
     for (int p = 0; p < 32 / RPS; ++p) {
       const int row = p * RPS + lane / PPQ;
-      const u32x4_t val = *reinterpret_cast<const u32x4_t*>(stg + row * D + 8 * (piece ^ (row & (PPQ - 1))));
+      RowRegs<T, 8> val;
+      load_row<T, 8>(val, reinterpret_cast<const T*>(stg + row * D + 8 * (piece ^ (row & (PPQ - 1)))));
+      if (a.gate != nullptr) val = gate_row<T, 8>(val, gv[p]);
       const int qi = qw + 32 * qb + row;
-      if (qi < a.Tq) *reinterpret_cast<u32x4_t*>(yb0 + (int64_t)qi * a.yt + 8 * piece) = val;
+      if (qi < a.Tq) store_row<T, 8>(yb0 + (int64_t)qi * a.yt + 8 * piece, val);
     }
     if (qb + 1 < QW) {
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -828,8 +841,13 @@ int launch_rope_prefill(int D, bool f32, const PrefillArgs& a, hipStream_t s) {
 int mfma_prefill_rope(int B, int H, int Tq, int Tk, int D, int dtype, const void* q, const dg_stride3* q_st,
                       const void* freqs, const dg_stride3* f_st, int fdtype, int qknorm, int keys_normed,
                       const void* k, const dg_stride3* k_st, const void* v, const dg_stride3* v_st, void* y,
-                      const dg_stride3* y_st, float scale, hipStream_t s) {
+                      const dg_stride3* y_st, float scale, const void* gate, const dg_stride3* g_st,
+                      hipStream_t s) {
   PrefillArgs a = prefill_args(B, H, Tq, Tk, D, q, q_st, k, k_st, v, v_st, y, y_st, scale);
+  if (gate != nullptr) {
+    a.gate = gate;
+    a.gb = g_st->b; a.gt = g_st->t; a.gh = g_st->h;
+  }
   a.freqs = freqs;
   a.fb = f_st->b; a.ft = f_st->t; a.fh = f_st->h;
   a.qknorm = qknorm;

@@ -278,9 +278,20 @@ void prefill_mfma_f32_kernel(const PrefillArgs a) {
   // lane's query, so group g gives 4*NB consecutive dims
   const float inv = __builtin_amdgcn_rcpf(half_pair_sum(l));
   float* yrow = static_cast<float*>(a.y) + b * a.yb + (int64_t)qi * a.yt + (int64_t)head * a.yh;
+  const float* grow = a.gate == nullptr ? nullptr
+                                        : static_cast<const float*>(a.gate) + b * a.gb + (int64_t)qi * a.gt +
+                                              (int64_t)head * a.gh;
+  auto put = [&](int d, f32x4v_t w) __attribute__((always_inline)) {
+    if (grow != nullptr) {  // uniform over the grid
+      const f32x4v_t g = *reinterpret_cast<const f32x4v_t*>(grow + d);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) w[i] = w[i] * sigmoid_rt<float>(g[i]);
+    }
+    *reinterpret_cast<f32x4v_t*>(yrow + d) = w;
+  };
 #pragma unroll
   for (int g = 0; g < 4; ++g) {
-    float* dst = yrow + NB * (8 * g + 4 * hh);
+    const int d0 = NB * (8 * g + 4 * hh);
     if constexpr (NB == 2) {
 #pragma unroll
       for (int h2 = 0; h2 < 2; ++h2) {
@@ -289,7 +300,7 @@ void prefill_mfma_f32_kernel(const PrefillArgs a) {
         w[1] = o[1][4 * g + 2 * h2] * inv;
         w[2] = o[0][4 * g + 2 * h2 + 1] * inv;
         w[3] = o[1][4 * g + 2 * h2 + 1] * inv;
-        *reinterpret_cast<f32x4v_t*>(dst + 4 * h2) = w;
+        put(d0 + 4 * h2, w);
       }
     } else {
 #pragma unroll
@@ -297,7 +308,7 @@ void prefill_mfma_f32_kernel(const PrefillArgs a) {
         f32x4v_t w;
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) w[nb] = o[nb][4 * g + e] * inv;
-        *reinterpret_cast<f32x4v_t*>(dst + 4 * e) = w;
+        put(d0 + 4 * e, w);
       }
     }
   }

@@ -19,8 +19,8 @@
 // Every intermediate is rounded to the storage dtype where the torch op
 // sequence rounds it (each op returns a tensor of the input dtype; fp32
 // arithmetic inside, as ATen's opmath does), so bf16 results follow the same
-// rounding steps.  The RMSNorms use the lane mapping and reduction tree of
-// rms_norm_kernel, so they produce its bits for the same row.
+// rounding steps.  The RMSNorms of outputs use the lane mapping and
+// reduction tree of rms_norm_kernel, so they produce its bits for the same row.
 #include <float.h>
 
 #include <type_traits>
@@ -40,12 +40,6 @@ struct AttnResArgs {
   int nsrc, N;
   int dup;  // 1 when source 1 is source 0 (same rows): read once
 };
-
-// round-trip through the storage dtype
-template <typename T>
-__device__ __forceinline__ float rt(float x) {
-  return to_f32(from_f32<T>(x));
-}
 
 // RMSNorm of one row slice with rms_norm_kernel's arithmetic (squares summed
 // by tree_sum inside the lane, then the butterfly over the G lanes of the row,
@@ -239,8 +233,8 @@ __global__ __launch_bounds__(256) void attn_res_norm_kernel(const AttnResArgs a,
 // quotients of four sources at once.  Near HBM's rate at a prefill's sizes: 65536
 // bf16 rows of 512 with 6 sources, 5 of them distinct (403 MB), take 101 us
 // (4.0 TB/s), 28672 rows of 1024 with 4 (235 MB) 52 us (4.5 TB/s); one source at
-// a time, with its own reductions and fp32 copies in registers, they took 237
-// and 110.  NS = 4, 6, 8 or 12 sources and 96 registers of them: beyond either
+// a time, with its own reductions and fp32 copies in registers, the former took
+// 237.  NS = 4, 6, 8 or 12 sources and 96 registers of them: beyond either
 // the general form's.
 template <typename T, int CH, int NS>
 __global__ __launch_bounds__(256) void attn_res_norm_wave_kernel(const AttnResArgs a) {
@@ -416,21 +410,6 @@ __global__ __launch_bounds__(256) void attn_res_norm_split_kernel(const AttnResA
   }
 }
 
-// sigmoid rounded to T.  fp32: as ATen evaluates it, 1 / (1 + exp(-x)).  16-bit
-// types: the hardware exp2 and reciprocal (a few units of 2^-22, far below the
-// rounding to T that follows) in place of expf and a correctly rounded divide,
-// which at about 40 VALU instructions per element bounded the gate over a
-// prefill's rows (see gate_vec_kernel).
-template <typename T>
-__device__ __forceinline__ float sigmoid_rt(float x) {
-#pragma clang fp contract(off)
-  if constexpr (sizeof(T) == 4) {
-    return 1.0f / (1.0f + expf(-x));
-  } else {
-    return rt<T>(__builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x * -1.44269504f)));
-  }
-}
-
 // One SwiGLU element with the torch sequence's roundings (swi_glu.py:15-19).
 // clamp(max=limit) / clamp(-limit, limit) select existing values: exact.
 template <typename T>
@@ -517,12 +496,7 @@ __global__ __launch_bounds__(256) void gate_vec_kernel(const VecRowsArgs v) {
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     if (o[u] == nullptr) continue;
-    float x[E];
-#pragma unroll
-    for (int e = 0; e < E; ++e) x[e] = elem<T, E>(y[u], e) * sigmoid_rt<T>(elem<T, E>(g[u], e));
-    RowRegs<T, E> p;
-    pack_row<T, E>(p, x);
-    store_row<T, E>(o[u], p);
+    store_row<T, E>(o[u], gate_row<T, E>(y[u], g[u]));
   }
 }
 

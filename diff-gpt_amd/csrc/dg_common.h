@@ -75,6 +75,27 @@ __device__ __forceinline__ uint32_t pack_pair(float a, float b) {
   }
 }
 
+// round-trip through the storage dtype
+template <typename T>
+__device__ __forceinline__ float rt(float x) {
+  return to_f32(from_f32<T>(x));
+}
+
+// sigmoid rounded to T.  fp32: as ATen evaluates it, 1 / (1 + exp(-x)).  16-bit
+// types: the hardware exp2 and reciprocal (a few units of 2^-22, far below the
+// rounding to T that follows) in place of expf and a correctly rounded divide,
+// which at about 40 VALU instructions per element bounded the gate over a
+// prefill's rows (gate_vec_kernel).
+template <typename T>
+__device__ __forceinline__ float sigmoid_rt(float x) {
+#pragma clang fp contract(off)
+  if constexpr (sizeof(T) == 4) {
+    return 1.0f / (1.0f + expf(-x));
+  } else {
+    return rt<T>(__builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x * -1.44269504f)));
+  }
+}
+
 // ---------------------------------------------------------------------------
 // Vector loads of EPL consecutive elements (EPL*sizeof(T) bytes, naturally
 // aligned by the host-side checks) converted to fp32.
@@ -444,6 +465,19 @@ __device__ __forceinline__ float slice_dot(const RowRegs<T, EPL>& q, const RowRe
                                  __builtin_bit_cast(f16x2v_t, k.w[w]), d, false);
   }
   return d;
+}
+
+// A row slice times the sigmoid of its gate (mha.py:84), each rounded to T:
+// y * sigmoid(g) on the stored y.
+template <typename T, int EPL>
+__device__ __forceinline__ RowRegs<T, EPL> gate_row(const RowRegs<T, EPL>& y, const RowRegs<T, EPL>& g) {
+#pragma clang fp contract(off)
+  float x[EPL];
+#pragma unroll
+  for (int e = 0; e < EPL; ++e) x[e] = elem<T, EPL>(y, e) * sigmoid_rt<T>(elem<T, EPL>(g, e));
+  RowRegs<T, EPL> r;
+  pack_row<T, EPL>(r, x);
+  return r;
 }
 
 typedef float f32x4_t __attribute__((ext_vector_type(4)));

@@ -26,6 +26,10 @@ struct PrefillArgs {
   const void* freqs;
   int64_t fb, ft, fh;
   int qknorm;
+  // gate logits of output row (b, i, h) at gate + b*gb + i*gt + h*gh, or null:
+  // y * sigmoid(gate) is stored in y's place (16-byte aligned rows)
+  const void* gate;
+  int64_t gb, gt, gh;
 };
 
 constexpr int kPrefillWindow = 64;      // (b, h) pairs per scheduling window

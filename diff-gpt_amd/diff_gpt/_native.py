@@ -110,6 +110,14 @@ _SIGNATURES = {
         + [ctypes.c_void_p, ctypes.POINTER(Stride3)] * 3  # k, v, y
         + [ctypes.c_float, ctypes.c_void_p],
     ),
+    "dg_prefill_rope_gate": (
+        ctypes.c_int,
+        [ctypes.c_int] * 6
+        + [ctypes.c_void_p, ctypes.POINTER(Stride3)] * 2  # q, freqs
+        + [ctypes.c_int, ctypes.c_int]  # freqs dtype, flags
+        + [ctypes.c_void_p, ctypes.POINTER(Stride3)] * 3  # k, v, y
+        + [ctypes.c_float, ctypes.c_void_p, ctypes.POINTER(Stride3), ctypes.c_void_p],  # scale, gate
+    ),
     "dg_rope_qknorm_append_at": (
         ctypes.c_int,
         [ctypes.c_int] * 4
@@ -388,12 +396,13 @@ def attention_(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, y: torch.Tenso
 
 
 def prefill_rope_(q: torch.Tensor, freqs: torch.Tensor, k: torch.Tensor, v: torch.Tensor, y: torch.Tensor,
-                  scale: float, qknorm: bool, keys_normed: bool = False) -> bool:
+                  scale: float, qknorm: bool, keys_normed: bool = False, gate: torch.Tensor | None = None) -> bool:
     """dg_prefill_rope: attention over k, v (B,Tk,H,D) views of the query rows
     q (B,Tq,H,D) after RoPE (freqs (B|1,Tq,H|1,D/2,2)) and, with qknorm, the
     QK-norm -- applied as the kernel loads q -- into y.  keys_normed (with
     qknorm) declares every key row RMS-normalised, which bounds the scores and
-    lets the kernel drop the softmax's running maximum.  Returns False, having
+    lets the kernel drop the softmax's running maximum.  gate (B,Tq,H,D), when
+    given, is dg_prefill_rope_gate's: y * sigmoid(gate) is stored.  Returns False, having
     done nothing, when the fused kernel does not take the shape (the caller
     then makes the two calls); raises on any other error."""
     B, Tq, H, D = q.shape
@@ -402,6 +411,8 @@ def prefill_rope_(q: torch.Tensor, freqs: torch.Tensor, k: torch.Tensor, v: torc
         raise ValueError("prefill_rope: inconsistent q/k/v/y shapes")
     if not (q.dtype == k.dtype == v.dtype == y.dtype):
         raise TypeError("prefill_rope: q/k/v/y must share one dtype")
+    if gate is not None and (gate.shape != q.shape or gate.dtype != q.dtype):
+        raise ValueError("prefill_rope: the gate must have q's shape and dtype")
     if freqs.dim() != 5 or freqs.shape[-2:] != (D // 2, 2):
         raise ValueError(f"freqs must be (B,T,H,D/2,2)-broadcastable, got {tuple(freqs.shape)}")
     if freqs.stride(-1) != 1 or freqs.stride(-2) != 2:
@@ -410,11 +421,15 @@ def prefill_rope_(q: torch.Tensor, freqs: torch.Tensor, k: torch.Tensor, v: torc
         raise ValueError("freqs does not broadcast against (B,Tq,H)")
     f_st = Stride3(*(0 if freqs.size(i) == 1 else freqs.stride(i) for i in range(3)))
     st = lambda t: ctypes.pointer(_bthd_strides(t))  # noqa: E731
-    rc = lib().dg_prefill_rope(
+    args = (
         B, H, Tq, Tk, D, _dtype_code(q), _ptr(q), st(q), _ptr(freqs), ctypes.pointer(f_st), _dtype_code(freqs),
         (DG_QKNORM if qknorm else 0) | (DG_KEYS_NORMED if qknorm and keys_normed else 0),
-        _ptr(k), st(k), _ptr(v), st(v), _ptr(y), st(y), float(scale), _stream(q),
+        _ptr(k), st(k), _ptr(v), st(v), _ptr(y), st(y), float(scale),
     )
+    if gate is None:
+        rc = lib().dg_prefill_rope(*args, _stream(q))
+    else:
+        rc = lib().dg_prefill_rope_gate(*args, _ptr(gate), st(gate), _stream(q))
     if rc == DG_EUNSUPPORTED:
         return False
     _check(rc, "prefill_rope")

@@ -25,6 +25,8 @@ from diff_gpt.model.rms_norm import rms_norm
 # dg_attn_res_norm takes at most this many sources of at most this width
 ATTN_RES_MAX_SOURCES = 32
 ATTN_RES_MAX_WIDTH = 2048
+# the widths dg_block_out takes
+BLOCK_OUT_WIDTHS = (64, 128)
 
 def block_attn_res(
     blocks: tuple[torch.Tensor, ...],
@@ -112,13 +114,16 @@ class Block(nn.Module):
             blocks = (*blocks, partial_block)
         sa = self.sa
         qkvg = F.linear(xn, sa._projection_weight())
-        y = sa._attend(qkvg, freqs_cis, kv_cache)
+        # a large prefill's gate goes with the attention's stores, unless
+        # dg_block_out takes the ungated output below or only one row goes on
+        gated = not _last_only and xn.size(-1) not in BLOCK_OUT_WIDTHS and sa._gates_in_prefill(qkvg)
+        y = sa._attend(qkvg, freqs_cis, kv_cache, gated=True) if gated else sa._attend(qkvg, freqs_cis, kv_cache)
         g = sa._gate_logits(qkvg)
         if _last_only:
             y, g, partial_in = y[:, -1:], g[:, -1:], partial_in[:, -1:]
             blocks = tuple(b[:, -1:] for b in blocks)
         up, swiglu, down = self.ffwd.net
-        if len(blocks) + 1 <= ATTN_RES_MAX_SOURCES:
+        if not gated and len(blocks) + 1 <= ATTN_RES_MAX_SOURCES:
             # gate, c_proj, the partial sum, the MLP's mixture and norm, the FFN
             # and the residual in one launch (n_embd 64 or 128)
             out = torch.empty_like(partial_in)
@@ -126,7 +131,8 @@ class Block(nn.Module):
                                   self.mlp_res_proj.weight, up.weight, down.weight, swiglu.alpha, swiglu.limit,
                                   out, _xn_out):
                 return blocks, out
-        _native.ops().gate_(y, g)  # y * sigmoid(g), mha.py:84
+        if not gated:
+            _native.ops().gate_(y, g)  # y * sigmoid(g), mha.py:84
         attn_out = sa.c_proj(y)
         partial_block = attn_out if committed else partial_in + attn_out
         out = self._mlp(blocks, partial_block)

@@ -38,6 +38,16 @@ from torch import nn
 from diff_gpt import _native
 from diff_gpt.model.kv_cache import KVCache
 
+# A prefill whose attention output has at least this many bytes applies the
+# sigmoid gate as the attention kernel stores it (dg_prefill_rope_gate):
+# 32 MiB, the 8 XCDs' L2s together.  Above, a gate launch of its own reads and
+# writes y through memory once more (n_embd 512 in bf16: the sub-layer over
+# 256 x 1024 rows, y 256 MiB, 1417 us apart and 1324 fused, a layer over
+# 64 x 1024, y 64 MiB, 930 and 899); below, y is still in the L2s when that
+# launch reads it, and the ungated output stays available to the launches that
+# gate it themselves.
+_FUSED_GATE_BYTES = 32 << 20
+
 
 class MultiHeadAttention(nn.Module):
     def __init__(
@@ -130,19 +140,34 @@ class MultiHeadAttention(nn.Module):
         _native.require_device("MultiHeadAttention", x)
         _native.require_inference("MultiHeadAttention", x, self.c_q.weight)
         qkvg = F.linear(x, self._projection_weight())  # (B, T, 3*inner + C)
-        y = self._attend(qkvg, freqs_cis, kv_cache)
-        ops = _native.ops()
-        ops.gate_(y, self._gate_logits(qkvg))  # y * sigmoid(g)
+        if self._gates_in_prefill(qkvg):
+            y = self._attend(qkvg, freqs_cis, kv_cache, gated=True)
+        else:
+            y = self._attend(qkvg, freqs_cis, kv_cache)
+            _native.ops().gate_(y, self._gate_logits(qkvg))  # y * sigmoid(g)
         return self.c_proj(y)
+
+    def _takes_mfma_prefill(self, qkvg: torch.Tensor) -> bool:
+        """Whether the prefill over these projections is dg_prefill_rope's (up to
+        alignment): head_dim 64 or 128, at least 16 tokens, not fp64."""
+        return (qkvg.size(1) >= 16 and self.head_dim in (64, 128)
+                and qkvg.dtype in (torch.bfloat16, torch.float16, torch.float32))
+
+    def _gates_in_prefill(self, qkvg: torch.Tensor) -> bool:
+        """Whether the gate is best applied by the attention kernel (_FUSED_GATE_BYTES)."""
+        B, T, _ = qkvg.size()
+        return (self._takes_mfma_prefill(qkvg)
+                and B * T * self.n_embd * qkvg.element_size() >= _FUSED_GATE_BYTES)
 
     def _gate_logits(self, qkvg: torch.Tensor) -> torch.Tensor:
         return qkvg[..., 3 * self.n_head * self.head_dim :]
 
-    def _attend(self, qkvg: torch.Tensor, freqs_cis: torch.Tensor, kv_cache: KVCache | None) -> torch.Tensor:
+    def _attend(self, qkvg: torch.Tensor, freqs_cis: torch.Tensor, kv_cache: KVCache | None,
+                gated: bool = False) -> torch.Tensor:
         """mha.py:44-83 on the projections qkvg (B, T, 3*inner + C), whose
         column slices are q, k, v and the gate logits: RoPE, QK-norm, the
         cache append and the attention; returns y (B, T, inner) before the
-        gate."""
+        gate, or with gated after it (mha.py:84)."""
         B, T, _ = qkvg.size()
         H, D = self.n_head, self.head_dim
         ops = _native.ops()
@@ -152,11 +177,14 @@ class MultiHeadAttention(nn.Module):
         v = qkvg[..., 2 * inner : 3 * inner].view(B, T, H, D)
 
         if kv_cache is not None and T == 1:
-            return self._decode_step(q, k, v, freqs_cis, kv_cache)
+            y = self._decode_step(q, k, v, freqs_cis, kv_cache)
+            if gated:
+                ops.gate_(y, self._gate_logits(qkvg))
+            return y
         assert kv_cache is None or kv_cache.pos_dev is None, "a captured decode step takes one token per row"
         # Prefills the MFMA kernel takes rotate and normalise q as they load it
         # (dg_prefill_rope); the first launch then handles k and v only.
-        fuse_q = T >= 16 and D in (64, 128) and q.dtype in (torch.bfloat16, torch.float16, torch.float32)
+        fuse_q = self._takes_mfma_prefill(qkvg)
         q_rot = None if fuse_q else torch.empty((B, T, H, D), dtype=q.dtype, device=q.device)
         q_in = None if fuse_q else q
         if kv_cache is None:
@@ -191,6 +219,9 @@ class MultiHeadAttention(nn.Module):
         if fuse_q:
             y = torch.empty((B, T, H, D), dtype=q.dtype, device=q.device)
             # every key normalised (mha.py:48): the kernel's bounded softmax
+            if gated and _native.prefill_rope_(q, freqs_cis, keys, values, y, scale, True, keys_normed,
+                                               gate=self._gate_logits(qkvg).view(B, T, H, D)):
+                return y.view(B, T, H * D)
             if not _native.prefill_rope_(q, freqs_cis, keys, values, y, scale, True, keys_normed):
                 # a layout the fused kernel does not take (alignment): rotate q apart
                 q_rot = torch.empty_like(y)
@@ -198,7 +229,10 @@ class MultiHeadAttention(nn.Module):
                 y = None
         if y is None:
             y = ops.attention(q_rot, keys, values, scale, prefix_len, group)
-        return y.view(B, T, H * D)
+        y = y.view(B, T, H * D)
+        if gated:
+            ops.gate_(y, self._gate_logits(qkvg))
+        return y
 
     def _decode_step(self, q, k, v, freqs, kv_cache: KVCache) -> torch.Tensor:
         """One new token per row over the KV cache (mha.py:44-68 with T = 1):

@@ -178,6 +178,20 @@ DG_API int dg_prefill_rope(int B, int H, int Tq, int Tk, int D, int dtype,
                            void* y, const dg_stride3* y_st, float scale, void* stream);
 
 /*
+ * dg_prefill_rope with the output gate of mha.py:84 applied as y is stored:
+ * y = (dg_prefill_rope's y) * sigmoid(g), with dg_gate's roundings, so y has
+ * the bits of dg_prefill_rope followed by dg_gate.  gate: the gate logits as a
+ * (B,Tq,H,D) view, rows 16-byte aligned (else DG_EUNSUPPORTED, nothing done).
+ */
+DG_API int dg_prefill_rope_gate(int B, int H, int Tq, int Tk, int D, int dtype,
+                                const void* q, const dg_stride3* q_st,
+                                const void* freqs, const dg_stride3* f_st, int freqs_dtype, int flags,
+                                const void* k, const dg_stride3* k_st,
+                                const void* v, const dg_stride3* v_st,
+                                void* y, const dg_stride3* y_st, float scale,
+                                const void* gate, const dg_stride3* g_st, void* stream);
+
+/*
  * A prefix shared by groups of rows: KVCache.prefill's batch broadcast
  * (kv_cache.py:77-79) gives the `group` consecutive rows of each group the
  * same positions 0 .. len-1.  Row b belongs to group b / group.

@@ -87,3 +87,65 @@ def test_mixture_forms_agree(dev, dtype, C, n):
     _native.attn_res_norm_([s[:33] for s in aligned], w, few)
     assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
     assert torch.equal(outs[0][:33], few)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("B,Tq,past", [(2, 16, 0), (1, 129, 0), (3, 33, 47), (2, 300, 1)])
+def test_prefill_gate_equals_prefill_then_gate(dev, dtype, D, B, Tq, past):
+    """dg_prefill_rope_gate against dg_prefill_rope and dg_gate, bit for bit:
+    ragged query counts, chunks, both softmax forms, the gate a column slice of
+    the projections; a gate off its alignment is declined."""
+    from diff_gpt import _native
+
+    dt, H = TDT[dtype], 3
+    g = torch.Generator(device=dev).manual_seed(5)
+    wide = torch.randn(B, Tq, 2, H, D, generator=g, device=dev).to(dt)
+    q, gate = wide[:, :, 0], wide[:, :, 1]
+    k = torch.nn.functional.normalize(torch.randn(B, past + Tq, H, D, generator=g, device=dev), dim=-1)
+    k = (k * D**0.5).to(dt)
+    v = torch.randn(B, past + Tq, H, D, generator=g, device=dev).to(dt)
+    ang = torch.rand(Tq, D // 2, generator=g, device=dev) * 6.0
+    freqs = torch.stack((ang.cos(), ang.sin()), dim=-1).to(dt).view(1, Tq, 1, D // 2, 2)
+    for normed in (False, True):
+        ya, yb = torch.empty_like(v[:, :Tq]), torch.empty_like(v[:, :Tq])
+        assert _native.prefill_rope_(q, freqs, k, v, ya, D**-0.5, True, normed)
+        _native.gate_(ya.view(B, Tq, H * D), gate.reshape(B, Tq, H * D))
+        assert _native.prefill_rope_(q, freqs, k, v, yb, D**-0.5, True, normed, gate=gate)
+        assert torch.equal(ya, yb)
+    off = torch.zeros(B, Tq, H, D + 8, dtype=dt, device=dev)[..., 1 : D + 1]
+    assert not _native.prefill_rope_(q, freqs, k, v, yb, D**-0.5, True, True, gate=off)
+
+
+@pytest.mark.parametrize("n_embd,n_head", [(512, 8), (1024, 8)])
+def test_layers_gating_in_the_prefill_equal_the_gate_launch(dev, n_embd, n_head, monkeypatch):
+    """A Block and a MultiHeadAttention whose output passes the fused gate's size
+    give the bits of the same call with the gate launched apart."""
+    from diff_gpt.model import mha as mha_mod
+    from diff_gpt.model.block import Block
+    from diff_gpt.model.kv_cache import KVCache
+    from diff_gpt.model.rope import precompute_freqs_cis
+
+    torch.manual_seed(0)
+    block = Block(n_embd, n_head, 1.702, 7.0, layer_idx=0).eval().to(dev).to(torch.bfloat16)
+    B, T, D = 2, 100, n_embd // n_head
+    x = torch.randn(B, T, n_embd, device=dev).to(torch.bfloat16)
+    other = torch.randn(B, T, n_embd, device=dev).to(torch.bfloat16)
+    freqs = precompute_freqs_cis(D, T, 10000.0).to(dev).to(torch.bfloat16).view(1, T, 1, D // 2, 2)
+    calls = []
+    real = mha_mod._native.prefill_rope_
+
+    def spy(*a, **k):
+        calls.append("gate" in k)
+        return real(*a, **k)
+
+    monkeypatch.setattr(mha_mod._native, "prefill_rope_", spy)
+    results = []
+    for limit in (0, 1 << 40):
+        monkeypatch.setattr(mha_mod, "_FUSED_GATE_BYTES", limit)
+        cache = KVCache(batch_size=B, num_heads=n_head, seq_len=T, head_dim=D, num_layers=1)
+        with torch.no_grad():
+            results.append((block.sa(x, freqs, None), block((x,), other, freqs_cis=freqs, kv_cache=cache)[1]))
+    assert calls == [True, True, False, False]
+    for fused, apart in zip(*results):
+        assert torch.equal(fused, apart)
