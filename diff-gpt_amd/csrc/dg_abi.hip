@@ -85,6 +85,14 @@ int mfma_prefill_rope(int B, int H, int Tq, int Tk, int D, int dtype, const void
                       const dg_stride3* y_st, float scale, const void* gate, const dg_stride3* g_st,
                       hipStream_t s);
 
+// dg_attn_small.hip
+bool small_prefill_applicable(int B, int H, int Tq, int Tk, int D, int dtype, const void* q, const dg_stride3* q_st,
+                              const void* k, const dg_stride3* k_st, const void* v, const dg_stride3* v_st,
+                              const void* y, const dg_stride3* y_st, float scale);
+int small_prefill(int B, int H, int Tq, int Tk, int D, int dtype, const void* q, const dg_stride3* q_st,
+                  const void* k, const dg_stride3* k_st, const void* v, const dg_stride3* v_st, void* y,
+                  const dg_stride3* y_st, float scale, hipStream_t s);
+
 // ---------------------------------------------------------------------------
 // Strided 4-D copy (exact), element size 2, 4 or 8 bytes.
 // ---------------------------------------------------------------------------
@@ -205,6 +213,8 @@ extern "C" int dg_attention_grouped(int B, int H, int Tq, int Tk, int D, int dty
   if (rows_hold_all &&
       mfma_prefill_applicable(B, H, Tq, Tk, D, dtype, q, q_st, k, k_st, v, v_st, y, y_st, scale))
     return mfma_prefill(B, H, Tq, Tk, D, dtype, q, q_st, k, k_st, v, v_st, y, y_st, scale, s);
+  if (rows_hold_all && small_prefill_applicable(B, H, Tq, Tk, D, dtype, q, q_st, k, k_st, v, v_st, y, y_st, scale))
+    return small_prefill(B, H, Tq, Tk, D, dtype, q, q_st, k, k_st, v, v_st, y, y_st, scale, s);
   // Groups of at least 16 rows: the shared prefix as a matrix product (when the
   // vector kernel would not split the keys, so no workspace is involved).
   if (vec_attention_splits(B, H, Tq, Tk, D) == 1 &&

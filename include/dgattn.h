@@ -128,8 +128,9 @@ DG_API int dg_rope_qknorm_append(int B, int T, int H, int D, int dtype,
  * dg_dtype for its meaning with fp64 data).
  * Prefills (Tq >= 16) at D = 64 or 128 with 16-byte aligned rows run on the
  * matrix cores: bf16 / fp16 products with fp32 accumulation, fp32 inputs on
- * fp32 products and accumulation; other shapes on the vector kernel, which
- * takes every even D up to 1024 (alignment as for dg_rope_qknorm_append).
+ * fp32 products and accumulation; at D = 16 or 32, Tq >= 16 and a positive
+ * scale on matrix cores with fp32 probabilities in every dtype.  Other shapes
+ * run on the vector kernel, which takes every even D up to 1024 (alignment as for dg_rope_qknorm_append).
  *
  * workspace: split-KV partials; dg_attention_workspace_size() gives the bytes
  * needed for these sizes: 0 unless a single-token decode splits the keys of
