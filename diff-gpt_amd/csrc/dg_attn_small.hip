@@ -31,6 +31,16 @@ struct SmallCfg {
   static constexpr int NT = D == 16 ? 4 : 2;
 };
 
+// The wait states a matrix instruction's result needs before another unit
+// reads it (10 for these, of 8 passes at most), spelled out where a branch
+// follows: the compiler (ROCm 7.2) leaves them out on the branch's far side.
+template <int N>
+__device__ __forceinline__ void mfma_settle(f32x4_t (&s)[N]) {
+  static_assert(N == 2 || N == 4, "operands");
+  if constexpr (N == 2) asm volatile("s_nop 10" : "+v"(s[0]), "+v"(s[1]));
+  else asm volatile("s_nop 10" : "+v"(s[0]), "+v"(s[1]), "+v"(s[2]), "+v"(s[3]));
+}
+
 template <typename T, int D>
 __global__ __launch_bounds__(256) void prefill_small_kernel(const PrefillArgs a, const int units, const int nqt) {
   using C = SmallCfg<T, D>;
@@ -85,10 +95,14 @@ __global__ __launch_bounds__(256) void prefill_small_kernel(const PrefillArgs a,
     float mt = kNegInf;
 #pragma unroll
     for (int u = 0; u < NT; ++u) {
-      const int k0 = t0 + 16 * u;
       s[u] = f32x4_t{kNegInf, kNegInf, kNegInf, kNegInf};
+      if (t0 + 16 * u < kend) s[u] = qk_mfma<T, DQ>(ch.k[u], qop, f32x4_t{0.f, 0.f, 0.f, 0.f});
+    }
+    mfma_settle(s);
+#pragma unroll
+    for (int u = 0; u < NT; ++u) {
+      const int k0 = t0 + 16 * u;
       if (k0 >= kend) continue;
-      s[u] = qk_mfma<T, DQ>(ch.k[u], qop, f32x4_t{0.f, 0.f, 0.f, 0.f});
       if (k0 + 15 > q0 + qoff || k0 + 16 > a.Tk) {  // the tile crosses the diagonal or the end
         const int lim = min(q0 + c + qoff, a.Tk - 1) - k0 - 4 * g;
 #pragma unroll
