@@ -21,15 +21,11 @@
 // arithmetic inside, as ATen's opmath does), so bf16 results follow the same
 // rounding steps.  The RMSNorms of outputs use the lane mapping and
 // reduction tree of rms_norm_kernel, so they produce its bits for the same row.
-#include <float.h>
-
 #include <type_traits>
 
-#include "dg_common.h"
+#include "dg_rows.h"
 
 namespace dg {
-
-constexpr int kMaxResSources = 32;
 
 struct AttnResArgs {
   const void* src[kMaxResSources];
@@ -41,116 +37,12 @@ struct AttnResArgs {
   int dup;  // 1 when source 1 is source 0 (same rows): read once
 };
 
-// RMSNorm of one row slice with rms_norm_kernel's arithmetic (squares summed
-// by tree_sum inside the lane, then the butterfly over the G lanes of the row,
-// here in registers: group_sum_dpp pairs the lanes as group_sum does, so the
-// bits are the same)
-template <int CH, int G>
-__device__ __forceinline__ void row_rms(float (&x)[CH], int N) {
-#pragma clang fp contract(off)
-  float sq[CH];
-#pragma unroll
-  for (int i = 0; i < CH; ++i) sq[i] = x[i] * x[i];
-  float ss = tree_sum<CH>(sq);
-  ss = group_sum_dpp<G>(ss);
-  const float mean = ss / (float)N;
-  const float r = 1.0f / sqrtf(mean + FLT_EPSILON);
-#pragma unroll
-  for (int i = 0; i < CH; ++i) x[i] = x[i] * r;
-}
-
-template <typename T, int CH>
-__device__ __forceinline__ void load_slice(const T* p, int c0, int N, bool vec, float (&x)[CH]) {
-  if (vec && c0 + CH <= N) {
-    load_vec<T, CH>(p, x);
-  } else {
-#pragma unroll
-    for (int i = 0; i < CH; ++i) x[i] = (c0 + i < N) ? to_f32(p[i]) : 0.f;
-  }
-}
-
 // Sources a lane loads into registers together, up front, to serve both
 // passes of the mixture (one round trip to memory for them, instead of one
-// per source and pass): about 32 registers of slices inside dg_block_out,
-// whose GEMM stages need the rest, and about 64 in attn_res_norm_kernel.
-template <int CH>
-constexpr int res_held() {
-  return CH <= 4 ? 8 : CH <= 8 ? 4 : CH <= 16 ? 2 : 1;
-}
+// per source and pass): about 64 registers of slices.
 template <int CH>
 constexpr int res_held_norm() {
   return CH <= 4 ? 16 : CH <= 8 ? 8 : CH <= 16 ? 4 : CH <= 32 ? 2 : 1;
-}
-
-// The mixture's arithmetic on a lane's slices as they are stored, the same in
-// its three kernels (so they agree bit for bit), each intermediate rounded to
-// T where its torch tensor is.  16-bit types work on packed pairs: the squares
-// and the products with w by v_dot2_f32_{bf16,f16} (exact products, fp32
-// sums), each rounding by one conversion of a pair.
-
-// sum of the slice's squares
-template <typename T, int CH>
-__device__ __forceinline__ float slice_squares(const RowRegs<T, CH>& x) {
-  return slice_dot<T, CH>(x, x);
-}
-// sum of rt(x r) w over the slice: the normalised row against the pseudo-query
-template <typename T, int CH>
-__device__ __forceinline__ float slice_score(const RowRegs<T, CH>& x, float r, const RowRegs<T, CH>& w) {
-#pragma clang fp contract(off)
-  float v[CH];
-#pragma unroll
-  for (int i = 0; i < CH; ++i) v[i] = elem<T, CH>(x, i) * r;
-  RowRegs<T, CH> n;
-  pack_row<T, CH>(n, v);
-  return slice_dot<T, CH>(n, w);
-}
-// h += rt(p x)
-template <typename T, int CH>
-__device__ __forceinline__ void slice_add(float (&h)[CH], float p, const RowRegs<T, CH>& x) {
-#pragma clang fp contract(off)
-  float v[CH];
-#pragma unroll
-  for (int i = 0; i < CH; ++i) v[i] = p * elem<T, CH>(x, i);
-  RowRegs<T, CH> n;
-  pack_row<T, CH>(n, v);
-#pragma unroll
-  for (int i = 0; i < CH; ++i) h[i] = h[i] + elem<T, CH>(n, i);
-}
-// the slice at p (elements c0 .. of a row of N), zeros past N
-template <typename T, int CH>
-__device__ __forceinline__ void load_packed(RowRegs<T, CH>& r, const T* p, int c0, int N, bool vec) {
-  if (vec && c0 + CH <= N) {
-    load_row<T, CH>(r, p);
-  } else {
-    float v[CH];
-#pragma unroll
-    for (int i = 0; i < CH; ++i) v[i] = (c0 + i < N) ? to_f32(p[i]) : 0.f;
-    pack_row<T, CH>(r, v);
-  }
-}
-// Sum over the G lanes of a row.  G = 64: halves and 16-lane rows first, in
-// the order attn_res_norm_wave_kernel folds several sums at once.
-__device__ __forceinline__ float row16_sum(float v) {
-  v = v + dpp<kDppQuadXor1>(v);
-  v = v + dpp<kDppQuadXor2>(v);
-  v = v + dpp<kDppHalfMirror>(v);
-  return v + dpp<kDppMirror>(v);
-}
-template <int G>
-__device__ __forceinline__ float score_sum(float v) {
-  if constexpr (G == 64) {
-    float a, b;
-    pair32(v, a, b);
-    v = a + b;
-    pair16(v, a, b);
-    return row16_sum(a + b);
-  } else {
-    return group_sum_dpp<G>(v);
-  }
-}
-__device__ __forceinline__ float row_factor(float ss, int N) {
-#pragma clang fp contract(off)
-  return 1.0f / sqrtf(ss / (float)N + FLT_EPSILON);
 }
 
 // NS: the most sources of the instance (the launch's fit).
@@ -408,17 +300,6 @@ __global__ __launch_bounds__(256) void attn_res_norm_split_kernel(const AttnResA
     for (int i = 0; i < CH; ++i)
       if (c0 + i < a.N) os[i] = from_f32<T>(hn[i]);
   }
-}
-
-// One SwiGLU element with the torch sequence's roundings (swi_glu.py:15-19).
-// clamp(max=limit) / clamp(-limit, limit) select existing values: exact.
-template <typename T>
-__device__ __forceinline__ float swiglu_value(float gate, float lin, float alpha, float limit) {
-#pragma clang fp contract(off)
-  gate = fminf(gate, limit);
-  lin = fminf(fmaxf(lin, -limit), limit);
-  const float s = sigmoid_rt<T>(rt<T>(alpha * gate));
-  return rt<T>(gate * s) * rt<T>(lin + 1.0f);
 }
 
 struct RowsArgs {
@@ -722,317 +603,6 @@ int res_pick(int npad, const AttnResArgs& a, hipStream_t s) {
 }
 
 }  // namespace
-
-// ---------------------------------------------------------------------------
-// A layer's work after its attention, in one launch (mha.py:84-85,
-// block.py:98-106, feed_forward.py:10-14):
-//
-//   block_out_kernel  a = y * sigmoid(g); attn_out = a @ W_proj^T; the
-//                     partial sum (attn_out, or partial_in + attn_out inside
-//                     a block); the MLP's mixture over the committed blocks
-//                     and that partial, its norm; the FFN (C -> 4C, clamped
-//                     SwiGLU, 2C -> C); and the residual
-//
-// A workgroup of 4 waves takes 16 token rows.  The stages meet in LDS (rows
-// padded by 16 bytes, so the 16 rows of a matrix-core operand read fall on
-// different banks); every GEMM is a sequence of 16 x 16 output tiles on the
-// matrix cores (qk_mfma's lane mapping: lane (c, g) feeds weight row
-// 16t + c and token row c with the contiguous quarter g of the contraction,
-// and gets back token row c's outputs 16t + 4g .. 16t + 4g + 3), the tiles of a
-// stage dealt round-robin to the 4 waves, each wave's weight fragments
-// fetched a stage or a tile ahead.  Every intermediate is rounded to T where
-// the torch sequence rounds it -- the gate as gate_kernel, each GEMM's fp32
-// sum once, the mixture as attn_res_norm_kernel, the SwiGLU as swiglu_kernel,
-// the residual adds -- so bf16 follows the same rounding steps; only the
-// GEMMs' summation order differs from hipBLASLt's.  C is 64 or 128.
-// (The same fusion before the attention -- the mixture, its norm and the
-// q/k/v/g projection in one launch -- measured no faster than the two
-// launches at 6400 rows and slower beyond: the mixture's dependent chain at
-// the occupancy its registers allow costs what the saved launch gains.)
-// ---------------------------------------------------------------------------
-constexpr int kLayerRows = 16;
-
-struct BlockOutArgs {
-  const void* y;        // (M, C) attention output (before the gate)
-  const void* g;        // (M, C) gate logits
-  const void* w_proj;   // (C, C)
-  const void* pin;      // (M, C) partial sum entering the layer; null when the layer commits it
-  const void* blk[kMaxResSources];  // committed blocks (the MLP mixture's first sources)
-  int64_t blk_ld[kMaxResSources];
-  const void* w_mix;    // (C,)
-  const void* w_up;     // (4C, C)
-  const void* w_down;   // (C, 2C)
-  void* out;            // (M, C) partial sum leaving the layer
-  void* xn;             // (M, C) rms_norm(out) as stored, or null
-  int64_t y_ld, g_ld, wp_ld, pin_ld, wu_ld, wd_ld, out_ld, xn_ld, M;
-  int nblk;
-  float alpha, limit;
-};
-
-// LDS row stride (elements) of a K-wide operand matrix: 16 bytes of padding
-template <typename T, int K>
-constexpr int lds_ld() {
-  return K + 16 / (int)sizeof(T);
-}
-
-// A lane's weight fragment of one 16 x 16 output tile over a K-long
-// contraction: weight row 16t + c (c = lane & 15), the contiguous quarter
-// g = lane >> 4 of the contraction, in chunks of 16 elements.  Loaded apart
-// from the product so that a wave can fetch it before the stage that
-// produces the tile's other operand, or one tile ahead.
-template <typename T, int K>
-struct TileW {
-  static constexpr int CQ = K / 4;  // contraction elements of a lane's quarter
-  static constexpr int KCH = 16;
-  static_assert(CQ % KCH == 0, "contraction chunking");
-  RowRegs<T, KCH> r[CQ / KCH];
-};
-
-template <typename T, int K>
-__device__ __forceinline__ void load_tile_w(TileW<T, K>& f, const T* __restrict__ w, int64_t w_ld, int t, int lane) {
-  const int c = lane & 15, g = lane >> 4;
-  const T* wr = w + (int64_t)(16 * t + c) * w_ld + g * TileW<T, K>::CQ;
-#pragma unroll
-  for (int i = 0; i < TileW<T, K>::CQ / 16; ++i) load_row<T, 16>(f.r[i], wr + 16 * i);
-}
-
-// The tile's product against the token rows of the LDS matrix x.
-template <typename T, int K>
-__device__ __forceinline__ f32x4_t layer_tile(const TileW<T, K>& f, const T* x, int lane) {
-  constexpr int CQ = TileW<T, K>::CQ;
-  const int c = lane & 15, g = lane >> 4;
-  const T* xr = x + c * lds_ld<T, K>() + g * CQ;
-  f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int i = 0; i < CQ / 16; ++i) {
-    RowRegs<T, 16> xo;
-    load_row<T, 16>(xo, xr + 16 * i);
-    acc = qk_mfma<T, 16>(f.r[i], xo, acc);
-  }
-  return acc;
-}
-
-// rms_norm(block_attn_res(V, w)) of the 16 rows into LDS xn, with
-// attn_res_norm_kernel's arithmetic; 16 lanes per row (CH = C / 16 elements
-// each).  Sources 0 .. nmem-1 are rows of global tensors; with last != null
-// the last source is that LDS matrix.  The caller has loaded the first
-// res_held<CH>() global sources (held) and the lane's slice of the
-// pseudo-query (w) into registers at the start of the kernel; they serve both
-// passes, further global sources and the LDS one are read where used.
-template <typename T, int C>
-__device__ __forceinline__ void layer_mixture(const void* const* src, const int64_t* ld, int nmem, const T* last,
-                                              const float (&held)[res_held<C / 16>()][C / 16],
-                                              const float (&w)[C / 16], int64_t row0, int64_t M, T* xn) {
-#pragma clang fp contract(off)
-  constexpr int CH = C / 16;
-  constexpr int G = 16;
-  constexpr int HELD = res_held<CH>();
-  const int r = threadIdx.x / G, sub = threadIdx.x % G, c0 = sub * CH;
-  const int64_t row = min(row0 + r, M - 1);  // rows past M: a finite copy, never stored
-  const int nsrc = nmem + (last != nullptr ? 1 : 0);
-  auto get = [&](int n, float (&x)[CH]) __attribute__((always_inline)) {
-    if (n < HELD && n < nmem) {
-#pragma unroll
-      for (int i = 0; i < CH; ++i) x[i] = held[n][i];
-    } else if (n < nmem) {
-      load_vec<T, CH>(static_cast<const T*>(src[n]) + row * ld[n] + c0, x);
-    } else {
-      load_vec<T, CH>(last + r * lds_ld<T, C>() + c0, x);
-    }
-  };
-  float score[kMaxResSources];
-  float mx = -INFINITY;
-#pragma unroll
-  for (int n = 0; n < kMaxResSources; ++n) {
-    score[n] = -INFINITY;
-    if (n >= nsrc) continue;  // uniform
-    float x[CH];
-    get(n, x);
-    row_rms<CH, G>(x, C);
-    float prod[CH];
-#pragma unroll
-    for (int i = 0; i < CH; ++i) prod[i] = rt<T>(x[i]) * w[i];
-    float dot = tree_sum<CH>(prod);
-    dot = group_sum_dpp<G>(dot);
-    score[n] = rt<T>(dot);
-    mx = fmaxf(mx, score[n]);
-  }
-  float e[kMaxResSources];
-  float sum = 0.f;
-#pragma unroll
-  for (int n = 0; n < kMaxResSources; ++n) {
-    e[n] = 0.f;
-    if (n >= nsrc) continue;
-    e[n] = expf(score[n] - mx);
-    sum += e[n];
-  }
-  float h[CH];
-#pragma unroll
-  for (int i = 0; i < CH; ++i) h[i] = 0.f;
-#pragma unroll
-  for (int n = 0; n < kMaxResSources; ++n) {
-    if (n >= nsrc) continue;
-    const float p = rt<T>(e[n] / sum);
-    float x[CH];
-    get(n, x);
-#pragma unroll
-    for (int i = 0; i < CH; ++i) h[i] = h[i] + rt<T>(p * x[i]);
-  }
-#pragma unroll
-  for (int i = 0; i < CH; ++i) h[i] = rt<T>(h[i]);
-  row_rms<CH, G>(h, C);
-  store_vec<T, CH>(xn + r * lds_ld<T, C>() + c0, h);
-}
-
-// FFN weight fragments loaded at the start of block_out_kernel: at C = 64 in
-// 16-bit types all of a wave's up and down tiles (72 registers); otherwise
-// the first up tile, each later one fetched while the one before runs, and
-// the down tiles behind the last up tile (fp32 fragments are twice the
-// registers, and loading all of them up front measured slower).
-template <typename T, int C>
-constexpr int block_up_depth() {
-  return (C == 64 && sizeof(T) == 2) ? C / 16 : 1;
-}
-
-template <typename T, int C>
-__global__ __launch_bounds__(256) void block_out_kernel(const BlockOutArgs a) {
-#pragma clang fp contract(off)
-  constexpr int LDC = lds_ld<T, C>(), LDH = lds_ld<T, 2 * C>();
-  constexpr int CH = C / 16;
-  constexpr int NPJ = C / 64;  // c_proj tiles per wave (C / 16 tiles over 4 waves)
-  constexpr int NUP = C / 16;  // FFN-up tiles per wave (4C / 16 over 4 waves)
-  constexpr int NDN = C / 64;  // FFN-down tiles per wave
-  constexpr int UPD = block_up_depth<T, C>();
-  constexpr bool kDownAtStart = UPD == NUP;  // else the down fragments follow the up tiles
-  constexpr int NDP = kDownAtStart ? NDN : 1;
-  constexpr int HELD = res_held<CH>();
-  __shared__ __attribute__((aligned(16))) T ga[kLayerRows * LDC];  // gated attention output, then xn
-  __shared__ __attribute__((aligned(16))) T pm[kLayerRows * LDC];  // the partial sum after the attention
-  __shared__ __attribute__((aligned(16))) T hh[kLayerRows * LDH];  // SwiGLU output
-  const int lane = threadIdx.x & 63;
-  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int c = lane & 15, g = lane >> 4;
-  const int64_t row0 = (int64_t)blockIdx.x * kLayerRows;
-  const T* w_proj = static_cast<const T*>(a.w_proj);
-  const T* w_up = static_cast<const T*>(a.w_up);
-  const T* w_down = static_cast<const T*>(a.w_down);
-
-  // Every global operand of the wave goes out here, in the order the stages
-  // use them, so that the stages wait on LDS and the matrix cores instead of
-  // one memory round trip each: the gate's rows (16 lanes per row), the
-  // c_proj fragments and the partial sum entering the layer (matrix-core
-  // lane mapping), the mixture's committed blocks and pseudo-query (16 lanes
-  // per row), the FFN fragments.
-  const int gr = threadIdx.x / 16, gc0 = (threadIdx.x % 16) * CH;
-  const int64_t grow = min(row0 + gr, a.M - 1);  // rows past M: a finite copy, never stored
-  const int64_t crow = min(row0 + c, a.M - 1);
-  float y[CH], gl[CH];
-  load_vec<T, CH>(static_cast<const T*>(a.y) + grow * a.y_ld + gc0, y);
-  load_vec<T, CH>(static_cast<const T*>(a.g) + grow * a.g_ld + gc0, gl);
-  TileW<T, C> wp[NPJ];
-#pragma unroll
-  for (int j = 0; j < NPJ; ++j) load_tile_w<T, C>(wp[j], w_proj, a.wp_ld, wv + 4 * j, lane);
-  float pin[NPJ][4];
-  if (a.pin != nullptr) {  // uniform
-#pragma unroll
-    for (int j = 0; j < NPJ; ++j)
-      load_vec<T, 4>(static_cast<const T*>(a.pin) + crow * a.pin_ld + 16 * (wv + 4 * j) + 4 * g, pin[j]);
-  }
-  float held[HELD][CH];
-#pragma unroll
-  for (int n = 0; n < HELD; ++n)
-    if (n < a.nblk) load_vec<T, CH>(static_cast<const T*>(a.blk[n]) + grow * a.blk_ld[n] + gc0, held[n]);  // uniform
-  float wmix[CH];
-  load_vec<T, CH>(static_cast<const T*>(a.w_mix) + gc0, wmix);
-  TileW<T, C> wu[UPD];
-#pragma unroll
-  for (int j = 0; j < UPD; ++j) load_tile_w<T, C>(wu[j], w_up, a.wu_ld, wv + 4 * j, lane);
-  TileW<T, 2 * C> wd[NDP];
-  if constexpr (kDownAtStart) {
-#pragma unroll
-    for (int j = 0; j < NDN; ++j) load_tile_w<T, 2 * C>(wd[j], w_down, a.wd_ld, wv + 4 * j, lane);
-  }
-  // keep the scheduler from sinking the loads toward their uses
-  __builtin_amdgcn_sched_barrier(0);
-
-  // 1) gate (gate_kernel's arithmetic)
-#pragma unroll
-  for (int i = 0; i < CH; ++i) y[i] = y[i] * sigmoid_rt<T>(gl[i]);
-  store_vec<T, CH>(ga + gr * LDC + gc0, y);
-  __syncthreads();
-  // 2) c_proj, then the partial sum
-#pragma unroll
-  for (int j = 0; j < NPJ; ++j) {
-    const f32x4_t acc = layer_tile<T, C>(wp[j], ga, lane);
-    const int f = 16 * (wv + 4 * j) + 4 * g;
-    float p[4];
-    if (a.pin != nullptr) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) p[i] = pin[j][i] + rt<T>(acc[i]);
-    } else {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) p[i] = acc[i];
-    }
-    store_vec<T, 4>(pm + c * LDC + f, p);
-  }
-  __syncthreads();
-  // 3) the MLP's mixture over the committed blocks and the new partial; its
-  //    norm overwrites the gated rows (no longer read)
-  layer_mixture<T, C>(a.blk, a.blk_ld, a.nblk, pm, held, wmix, row0, a.M, ga);
-  __syncthreads();
-  // 4) FFN up + SwiGLU (swiglu_kernel's arithmetic on the interleaved
-  //    (gate, linear) pairs: features 2j, 2j + 1 -> hidden j)
-#pragma unroll
-  for (int i = 0; i < NUP; ++i) {
-    const int t = wv + 4 * i;
-    TileW<T, C> next;
-    if (i + UPD < NUP) load_tile_w<T, C>(next, w_up, a.wu_ld, t + 4 * UPD, lane);
-    if constexpr (!kDownAtStart) {
-      if (i + 1 == NUP) load_tile_w<T, 2 * C>(wd[0], w_down, a.wd_ld, wv, lane);
-    }
-    const f32x4_t acc = layer_tile<T, C>(wu[i % UPD], ga, lane);
-    if (i + UPD < NUP) wu[i % UPD] = next;
-    float hv[2];
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      hv[q] = swiglu_value<T>(rt<T>(acc[2 * q]), rt<T>(acc[2 * q + 1]), a.alpha, a.limit);
-    }
-    store_vec<T, 2>(hh + c * LDH + 8 * t + 2 * g, hv);
-  }
-  __syncthreads();
-  // 5) FFN down + residual
-  const bool store = row0 + c < a.M;
-  T* orow = static_cast<T*>(a.out) + (row0 + c) * a.out_ld;
-#pragma unroll
-  for (int j = 0; j < NDN; ++j) {
-    const int t = wv + 4 * j;
-    TileW<T, 2 * C> next;
-    if constexpr (!kDownAtStart) {
-      if (j + 1 < NDN) load_tile_w<T, 2 * C>(next, w_down, a.wd_ld, t + 4, lane);
-    }
-    const f32x4_t acc = layer_tile<T, 2 * C>(wd[kDownAtStart ? j : 0], hh, lane);
-    if constexpr (!kDownAtStart) {
-      if (j + 1 < NDN) wd[0] = next;
-    }
-    const int f = 16 * t + 4 * g;
-    float pmv[4], o[4];
-    load_vec<T, 4>(pm + c * LDC + f, pmv);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) o[i] = pmv[i] + rt<T>(acc[i]);
-    if (store) store_vec<T, 4>(orow + f, o);
-    // the same lane alone reads and writes this slice of pm
-    if (a.xn != nullptr) store_vec<T, 4>(pm + c * LDC + f, o);  // uniform
-  }
-  // 6) dg_block_out_norm: the RMSNorm of the stored output rows (the head's
-  //    input after the last layer), 16 lanes per row
-  if (a.xn != nullptr) {  // uniform
-    __syncthreads();
-    float x[CH];
-    load_vec<T, CH>(pm + gr * LDC + gc0, x);
-    row_rms<CH, 16>(x, C);
-    if (row0 + gr < a.M) store_vec<T, CH>(static_cast<T*>(a.xn) + (row0 + gr) * a.xn_ld + gc0, x);
-  }
-}
 
 // ---------------------------------------------------------------------------
 // lm_head + softcap + greedy argmax.  Block = 4 waves = 16 rows of x; wave w
@@ -1340,80 +910,6 @@ extern "C" int dg_lm_head(int64_t M, int C, int V, int dtype, const void* x, int
   if (dtype == DG_F32) return launch_lm_head<float>(a, s);
   if (dtype == DG_BF16) return launch_lm_head<bf16_t>(a, s);
   return launch_lm_head<f16_t>(a, s);
-}
-
-namespace {
-bool rows16(const void* p, int64_t ld, int64_t es) {
-  return (reinterpret_cast<uintptr_t>(p) & 15) == 0 && (ld * es) % 16 == 0;
-}
-}  // namespace
-
-static int block_out_impl(int64_t M, int C, int dtype, const void* y, int64_t y_ld, const void* g, int64_t g_ld,
-                          const void* w_proj, int64_t wp_ld, const void* partial_in, int64_t pin_ld, int nblk,
-                          const void* const* blocks, const int64_t* blocks_ld, const void* w_mix, const void* w_up,
-                          int64_t wu_ld, const void* w_down, int64_t wd_ld, float alpha, float limit, void* out,
-                          int64_t out_ld, void* xn, int64_t xn_ld, void* stream) {
-  DG_REQUIRE(M >= 0 && C >= 1, DG_EINVAL, "block_out: bad sizes M=%lld C=%d", (long long)M, C);
-  DG_REQUIRE(dtype_ok(dtype), DG_EUNSUPPORTED, "block_out: dtype %d unsupported", dtype);
-  DG_REQUIRE(C == 64 || C == 128, DG_EUNSUPPORTED, "block_out: n_embd %d unsupported (64 or 128)", C);
-  DG_REQUIRE(nblk >= 0 && nblk + 1 <= kMaxResSources, DG_EINVAL, "block_out: %d blocks (0..%d)", nblk,
-             kMaxResSources - 1);
-  if (M == 0) return DG_OK;
-  DG_REQUIRE(y && g && w_proj && w_mix && w_up && w_down && out && (nblk == 0 || (blocks && blocks_ld)), DG_EINVAL,
-             "block_out: NULL pointer");
-  DG_REQUIRE(M <= (int64_t)kLayerRows * 0x7fffffffLL, DG_EINVAL, "block_out: too many rows (%lld)", (long long)M);
-  const int64_t es = dtype == DG_F32 ? 4 : 2;
-  BlockOutArgs a{};
-  bool ok = rows16(y, y_ld, es) && rows16(g, g_ld, es) && rows16(w_proj, wp_ld, es) && rows16(w_mix, 0, es) &&
-            rows16(w_up, wu_ld, es) && rows16(w_down, wd_ld, es) && rows16(out, out_ld, es) &&
-            (partial_in == nullptr || rows16(partial_in, pin_ld, es)) && (xn == nullptr || rows16(xn, xn_ld, es));
-  DG_REQUIRE(y_ld >= C && g_ld >= C && wp_ld >= C && wu_ld >= C && wd_ld >= 2 * C && out_ld >= C &&
-                 (partial_in == nullptr || pin_ld >= C) && (xn == nullptr || xn_ld >= C),
-             DG_EINVAL, "block_out: a row stride is narrower than its row");
-  for (int n = 0; n < nblk; ++n) {
-    DG_REQUIRE(blocks[n] != nullptr && blocks_ld[n] >= C, DG_EINVAL, "block_out: block %d is NULL or narrower than C",
-               n);
-    ok = ok && rows16(blocks[n], blocks_ld[n], es);
-    a.blk[n] = blocks[n];
-    a.blk_ld[n] = blocks_ld[n];
-  }
-  DG_REQUIRE(ok, DG_EUNSUPPORTED, "block_out: rows must be 16-byte aligned");
-  a.y = y; a.g = g; a.w_proj = w_proj; a.pin = partial_in; a.w_mix = w_mix; a.w_up = w_up; a.w_down = w_down;
-  a.out = out; a.xn = xn;
-  a.y_ld = y_ld; a.g_ld = g_ld; a.wp_ld = wp_ld; a.pin_ld = pin_ld; a.wu_ld = wu_ld; a.wd_ld = wd_ld;
-  a.out_ld = out_ld; a.xn_ld = xn_ld; a.M = M; a.nblk = nblk; a.alpha = alpha; a.limit = limit;
-  const dim3 grid((unsigned)((M + kLayerRows - 1) / kLayerRows));
-  hipStream_t s = static_cast<hipStream_t>(stream);
-#define DG_BLOCK_OUT(T)                                                                             \
-  do {                                                                                            \
-    if (C == 64) hipLaunchKernelGGL((block_out_kernel<T, 64>), grid, dim3(256), 0, s, a);         \
-    else hipLaunchKernelGGL((block_out_kernel<T, 128>), grid, dim3(256), 0, s, a);                \
-  } while (0)
-  if (dtype == DG_F32) DG_BLOCK_OUT(float);
-  else if (dtype == DG_BF16) DG_BLOCK_OUT(bf16_t);
-  else DG_BLOCK_OUT(f16_t);
-#undef DG_BLOCK_OUT
-  return check_launch("block_out_kernel");
-}
-
-extern "C" int dg_block_out(int64_t M, int C, int dtype, const void* y, int64_t y_ld, const void* g, int64_t g_ld,
-                            const void* w_proj, int64_t wp_ld, const void* partial_in, int64_t pin_ld, int nblk,
-                            const void* const* blocks, const int64_t* blocks_ld, const void* w_mix,
-                            const void* w_up, int64_t wu_ld, const void* w_down, int64_t wd_ld, float alpha,
-                            float limit, void* out, int64_t out_ld, void* stream) {
-  return block_out_impl(M, C, dtype, y, y_ld, g, g_ld, w_proj, wp_ld, partial_in, pin_ld, nblk, blocks, blocks_ld,
-                        w_mix, w_up, wu_ld, w_down, wd_ld, alpha, limit, out, out_ld, nullptr, 0, stream);
-}
-
-extern "C" int dg_block_out_norm(int64_t M, int C, int dtype, const void* y, int64_t y_ld, const void* g,
-                                 int64_t g_ld, const void* w_proj, int64_t wp_ld, const void* partial_in,
-                                 int64_t pin_ld, int nblk, const void* const* blocks, const int64_t* blocks_ld,
-                                 const void* w_mix, const void* w_up, int64_t wu_ld, const void* w_down,
-                                 int64_t wd_ld, float alpha, float limit, void* out, int64_t out_ld, void* xn,
-                                 int64_t xn_ld, void* stream) {
-  DG_REQUIRE(M == 0 || xn != nullptr, DG_EINVAL, "block_out_norm: NULL pointer");
-  return block_out_impl(M, C, dtype, y, y_ld, g, g_ld, w_proj, wp_ld, partial_in, pin_ld, nblk, blocks, blocks_ld,
-                        w_mix, w_up, wu_ld, w_down, wd_ld, alpha, limit, out, out_ld, xn, xn_ld, stream);
 }
 
 // ---------------------------------------------------------------------------

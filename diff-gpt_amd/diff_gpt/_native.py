@@ -197,6 +197,12 @@ _SIGNATURES = {
          ctypes.c_int64, ctypes.c_void_p, ctypes.c_int64, ctypes.c_float, ctypes.c_float, ctypes.c_void_p,
          ctypes.c_int64, ctypes.c_void_p],
     ),
+    "dg_block_in": (
+        ctypes.c_int,
+        [ctypes.c_int64, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.POINTER(ctypes.c_void_p),
+         ctypes.POINTER(ctypes.c_int64), ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p,
+         ctypes.c_int64, ctypes.c_void_p],
+    ),
     "dg_draw_argmax": (
         ctypes.c_int,
         [ctypes.c_int64, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p,
@@ -707,6 +713,32 @@ def _row_list(tensors: list[torch.Tensor], what: str):
     ptrs = (ctypes.c_void_p * max(1, len(rows)))(*[t.data_ptr() for t in rows])
     lds = (ctypes.c_int64 * max(1, len(rows)))(*[t.stride(0) for t in rows])
     return rows, ptrs, lds
+
+
+def block_in_(sources: list[torch.Tensor], w_mix: torch.Tensor | None, w_qkvg: torch.Tensor,
+              out: torch.Tensor) -> bool:
+    """dg_block_in: out (..., 4C) = the q/k/v/g projections (w_qkvg (4C, C)) of
+    rms_norm(block_attn_res(sources)) with pseudo-query w_mix, or with w_mix
+    None of the one source as it is.  Returns False, having done nothing, for
+    shapes the fused kernel does not take."""
+    C = w_qkvg.size(1)
+    if C not in (64, 128) or out.dtype not in (torch.float32, torch.bfloat16, torch.float16):
+        return False
+    rows, ptrs, lds = _row_list(sources, "block_in")
+    o2 = out.view(-1, 4 * C)
+    if len(rows) > 32 or any(t.dtype != out.dtype or t.shape != (o2.size(0), C) for t in rows):
+        return False
+    if w_qkvg.dtype != out.dtype or w_qkvg.shape != (4 * C, C) or w_qkvg.stride(1) != 1:
+        return False
+    w1 = None if w_mix is None else w_mix.reshape(-1).contiguous()
+    rc = lib().dg_block_in(
+        o2.size(0), C, _dtype_code(o2), len(rows), ptrs, lds, _ptr(w1), _ptr(w_qkvg), w_qkvg.stride(0), _ptr(o2),
+        o2.stride(0), _stream(o2),
+    )
+    if rc == DG_EUNSUPPORTED:
+        return False
+    _check(rc, "block_in")
+    return True
 
 
 def block_out_(y: torch.Tensor, g: torch.Tensor, w_proj: torch.Tensor, partial_in: torch.Tensor | None,

@@ -6,9 +6,10 @@ pseudo-query; a block boundary every ``layers_per_block`` layers commits the
 partial sum.  In Block.forward the mixture and the RMSNorm after it are one
 dg_attn_res_norm launch, the clamped SwiGLU of the MLP one dg_swiglu launch,
 and the attention sub-layer is the HIP path of MultiHeadAttention.  At
-n_embd 64 or 128 everything after the attention -- gate, c_proj, the partial
-sum, the MLP's mixture and norm, the FFN and the residual -- is one
-dg_block_out launch instead of six.
+n_embd 64 or 128 everything before the attention -- the mixture, its norm and
+the four projections -- is one dg_block_in launch, and everything after it --
+gate, c_proj, the partial sum, the MLP's mixture and norm, the FFN and the
+residual -- one dg_block_out launch instead of six.
 ``block_attn_res`` keeps the reference's torch formulation for direct callers.
 """
 
@@ -25,8 +26,8 @@ from diff_gpt.model.rms_norm import rms_norm
 # dg_attn_res_norm takes at most this many sources of at most this width
 ATTN_RES_MAX_SOURCES = 32
 ATTN_RES_MAX_WIDTH = 2048
-# the widths dg_block_out takes
-BLOCK_OUT_WIDTHS = (64, 128)
+# the widths dg_block_in and dg_block_out take
+LAYER_WIDTHS = (64, 128)
 
 def block_attn_res(
     blocks: tuple[torch.Tensor, ...],
@@ -107,16 +108,15 @@ class Block(nn.Module):
         head's input after the last layer, from the same launch when
         dg_block_out takes the layer."""
         _native.require_device("Block", partial_block)
-        xn = attn_res_norm(blocks, partial_block, self.attn_res_proj) if _xn is None else _xn
+        sa = self.sa
+        qkvg = self._project(blocks, partial_block, _xn)
         committed = self._at_boundary()
         partial_in = partial_block
         if committed:
             blocks = (*blocks, partial_block)
-        sa = self.sa
-        qkvg = F.linear(xn, sa._projection_weight())
         # a large prefill's gate goes with the attention's stores, unless
         # dg_block_out takes the ungated output below or only one row goes on
-        gated = not _last_only and xn.size(-1) not in BLOCK_OUT_WIDTHS and sa._gates_in_prefill(qkvg)
+        gated = not _last_only and sa.n_embd not in LAYER_WIDTHS and sa._gates_in_prefill(qkvg)
         y = sa._attend(qkvg, freqs_cis, kv_cache, gated=True) if gated else sa._attend(qkvg, freqs_cis, kv_cache)
         g = sa._gate_logits(qkvg)
         if _last_only:
@@ -139,6 +139,27 @@ class Block(nn.Module):
         if _xn_out is not None:
             _native.rms_norm_(out, _xn_out)
         return blocks, out
+
+    def _project(self, blocks: tuple[torch.Tensor, ...], partial_block: torch.Tensor,
+                 xn: torch.Tensor | None) -> torch.Tensor:
+        """The q/k/v/g projections (..., 3*inner + C) of the attention's input
+        attn_res_norm(blocks, partial_block), or of xn when the caller computed
+        it: one dg_block_in launch at n_embd 64 or 128, else the mixture's
+        launch and a GEMM."""
+        w = self.sa._projection_weight()
+        if w.size(1) in LAYER_WIDTHS and w.size(0) == 4 * w.size(1):
+            if xn is None and len(blocks) == 1 and partial_block is blocks[0]:
+                xn = rms_norm(partial_block)
+            out = torch.empty((*partial_block.shape[:-1], w.size(0)), dtype=w.dtype, device=partial_block.device)
+            if xn is not None:
+                if _native.block_in_([xn], None, w, out):
+                    return out
+            elif len(blocks) + 1 <= ATTN_RES_MAX_SOURCES:
+                if _native.block_in_([*blocks, partial_block], self.attn_res_proj.weight, w, out):
+                    return out
+        if xn is None:
+            xn = attn_res_norm(blocks, partial_block, self.attn_res_proj)
+        return F.linear(xn, w)
 
     def _mlp(self, blocks: tuple[torch.Tensor, ...], partial_block: torch.Tensor) -> torch.Tensor:
         xn = attn_res_norm(blocks, partial_block, self.mlp_res_proj)

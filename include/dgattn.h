@@ -444,6 +444,22 @@ DG_API int dg_lm_head(int64_t M, int C, int V, int dtype, const void* x, int64_t
                       int64_t w_ld, float cap, void* logits, int64_t logits_ld, int64_t* ids, void* stream);
 
 /*
+ * A layer's work before its attention in one launch: the attention's mixture
+ * over the nsrc sources (committed blocks, then the partial sum) with its
+ * RMSNorm (block.py:95-97), and the q/k/v/g projections of the result
+ * (mha.py:34-43): out (M, 4C) = rms_norm(block_attn_res(src, w_mix)) @
+ * w_qkvg^T, w_qkvg (4C, C).  With w_mix NULL, src[0] alone is the normalised
+ * input and is projected as it is.  Roundings as dg_attn_res_norm's, each
+ * projection's fp32 sum rounded once; the products run on the matrix cores, so
+ * the result agrees with dg_attn_res_norm + F.linear within the north-star
+ * bars, not bit for bit.  Supported: C = 64 or 128, nsrc <= 32, 16-byte
+ * aligned rows; anything else returns DG_EUNSUPPORTED and does nothing.
+ */
+DG_API int dg_block_in(int64_t M, int C, int dtype, int nsrc, const void* const* src, const int64_t* src_ld,
+                       const void* w_mix, const void* w_qkvg, int64_t w_ld, void* out, int64_t out_ld,
+                       void* stream);
+
+/*
  * A layer's work after its attention in one launch: mha.py:84-85 (the gate
  * y * sigmoid(g) and c_proj), block.py:98-106 (the partial sum: the
  * attention output itself when the layer commits its input block, else
