@@ -59,6 +59,17 @@ int shared_decode_step(int B, int H, int D, int dtype, const void* q, const dg_s
                        int64_t fpos, int fdtype, int pos, const int* pos_dev, int max_pos, void* y,
                        const dg_stride3* y_st, float scale, const PrefixRef& pre, int qknorm,
                        hipStream_t s);
+// dg_attn_wide.hip
+bool wide_step_applicable(int B, int H, int D, int dtype, const PrefixRef& pre, int max_pos, const void* q,
+                          const dg_stride3* q_st, const void* k, const dg_stride3* k_st, const void* v,
+                          const dg_stride3* v_st, const void* kc, const dg_stride3* kc_st, const void* vc,
+                          const dg_stride3* vc_st, const void* freqs, int64_t fpos, int fdtype, const void* y,
+                          const dg_stride3* y_st, float scale);
+int wide_decode_step(int B, int H, int D, int dtype, const void* q, const dg_stride3* q_st, const void* k,
+                     const dg_stride3* k_st, const void* v, const dg_stride3* v_st, void* kc, const dg_stride3* kc_st,
+                     void* vc, const dg_stride3* vc_st, const void* freqs, int64_t fpos, int fdtype, int pos,
+                     const int* pos_dev, int max_pos, void* y, const dg_stride3* y_st, float scale,
+                     const PrefixRef& pre, int qknorm, hipStream_t s);
 // dg_rope.hip
 int rope_append_at(int B, int H, int D, int dtype, const void* q, const dg_stride3* q_st, void* q_out,
                    const dg_stride3* qo_st, const void* k, const dg_stride3* k_st, void* k_cache,
@@ -358,6 +369,11 @@ extern "C" int dg_decode_step(int B, int H, int D, int dtype, const void* q, con
     return shared_decode_step(B, H, D, dtype, q, q_st, k, k_st, v, v_st, kw, kc_st, vw, vc_st, freqs,
                               freqs_pos_stride, freqs_dtype, pos, pos_dev, max_pos, y, y_st, scale, pre, qknorm,
                               s);
+  // groups of at least 16 rows at head_dim 64 / 128 in 16-bit types
+  if (wide_step_applicable(B, H, D, dtype, pre, max_pos, q, q_st, k, k_st, v, v_st, kw, kc_st, vw, vc_st, freqs,
+                           freqs_pos_stride, freqs_dtype, y, y_st, scale))
+    return wide_decode_step(B, H, D, dtype, q, q_st, k, k_st, v, v_st, kw, kc_st, vw, vc_st, freqs, freqs_pos_stride,
+                            freqs_dtype, pos, pos_dev, max_pos, y, y_st, scale, pre, qknorm, s);
   // Where the attention runs on the vector kernel: one launch of its fused
   // form, with the two launches' bits (below), unless the projections or the
   // table are not aligned to its lane slices.

@@ -31,16 +31,6 @@ struct SmallCfg {
   static constexpr int NT = D == 16 ? 4 : 2;
 };
 
-// The wait states a matrix instruction's result needs before another unit
-// reads it (10 for these, of 8 passes at most), spelled out where a branch
-// follows: the compiler (ROCm 7.2) leaves them out on the branch's far side.
-template <int N>
-__device__ __forceinline__ void mfma_settle(f32x4_t (&s)[N]) {
-  static_assert(N == 2 || N == 4, "operands");
-  if constexpr (N == 2) asm volatile("s_nop 10" : "+v"(s[0]), "+v"(s[1]));
-  else asm volatile("s_nop 10" : "+v"(s[0]), "+v"(s[1]), "+v"(s[2]), "+v"(s[3]));
-}
-
 template <typename T, int D>
 __global__ __launch_bounds__(256) void prefill_small_kernel(const PrefillArgs a, const int units, const int nqt) {
   using C = SmallCfg<T, D>;

@@ -516,6 +516,16 @@ __device__ __forceinline__ f32x4_t qk_mfma(const RowRegs<T, DQ>& kop, const RowR
   return acc;
 }
 
+// The wait states a matrix instruction's result needs before another unit
+// reads it (10 for these, of 8 passes at most), spelled out where a branch
+// follows: the compiler (ROCm 7.2) leaves them out on the branch's far side.
+template <int N>
+__device__ __forceinline__ void mfma_settle(f32x4_t (&s)[N]) {
+  static_assert(N == 2 || N == 4, "operands");
+  if constexpr (N == 2) asm volatile("s_nop 10" : "+v"(s[0]), "+v"(s[1]));
+  else asm volatile("s_nop 10" : "+v"(s[0]), "+v"(s[1]), "+v"(s[2]), "+v"(s[3]));
+}
+
 // Third dword of a raw buffer resource on gfx9-family chips (gfx950 included):
 // 32-bit data format, no swizzle, no stride.
 constexpr int kBufferWord3 = 0x00020000;

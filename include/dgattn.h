@@ -296,10 +296,15 @@ DG_API int dg_decode_attention_at(int B, int H, int D, int dtype,
  * *pos_dev is outside [own_start, max_pos)), else p = pos, which must lie in
  * [own_start, max_pos) and at or past the prefix's length.
  *
- * With a shared prefix (group >= 16, D 16 or 32) this is one launch: the new
+ * With a shared prefix (group >= 16) and D 16 or 32 this is one launch: the new
  * key and value are appended and also used from registers.  The cache
  * contents are those of dg_rope_qknorm_append bit for bit; y equals the
  * two-call result within fp32 rounding (the new key is accumulated last).
+ * So it is in bf16 / fp16 at D 64 or 128 (group >= 16, 16-byte aligned rows)
+ * where the shared key reads B * H * P repay the matrix-core kernel's fixed
+ * chain: B * H >= 320, 2 P >= m and B * H * P >= 3300 m + 200000 with
+ * m = max_pos - P; the probabilities enter the products there as two values of
+ * the data type, so y agrees with the two calls within rounding.
  * Where the attention runs on the vector kernel (every other shape whose
  * rows, projections and table are aligned to its lane slices) it is one
  * launch too: each (row, head) wave rotates q and k itself, the wave whose
