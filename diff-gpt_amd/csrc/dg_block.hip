@@ -665,8 +665,7 @@ __global__ __launch_bounds__(256) void lm_head_kernel(const LmHeadArgs a) {
     float out[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      float v = rt<T>(acc[t][r]);
-      if (a.cap > 0.f) v = rt<T>(a.cap * rt<T>(tanhf(rt<T>(v / a.cap))));
+      const float v = softcap_value<T>(acc[t][r], a.cap);
       out[r] = v;
       const int e = vbase + 16 * t + 4 * g + r;  // increasing within the lane
       if (v > best) {
@@ -677,16 +676,7 @@ __global__ __launch_bounds__(256) void lm_head_kernel(const LmHeadArgs a) {
     if (row_ok) store_vec<T, 4>(lrow + 16 * t, out);
   }
   if (a.ids == nullptr) return;  // uniform over the grid
-  // the row's four lanes: larger value, or equal value and smaller entry
-#pragma unroll
-  for (int off = 16; off <= 32; off <<= 1) {
-    const float ov = __shfl_xor(best, off, 64);
-    const int oi = __shfl_xor(bidx, off, 64);
-    if (ov > best || (ov == best && oi < bidx)) {
-      best = ov;
-      bidx = oi;
-    }
-  }
+  first_max(best, bidx);
   if (g == 0) {
     red_v[w][c] = best;
     red_i[w][c] = bidx;

@@ -521,8 +521,9 @@ __device__ __forceinline__ f32x4_t qk_mfma(const RowRegs<T, DQ>& kop, const RowR
 // follows: the compiler (ROCm 7.2) leaves them out on the branch's far side.
 template <int N>
 __device__ __forceinline__ void mfma_settle(f32x4_t (&s)[N]) {
-  static_assert(N == 2 || N == 4, "operands");
-  if constexpr (N == 2) asm volatile("s_nop 10" : "+v"(s[0]), "+v"(s[1]));
+  static_assert(N == 1 || N == 2 || N == 4, "operands");
+  if constexpr (N == 1) asm volatile("s_nop 10" : "+v"(s[0]));
+  else if constexpr (N == 2) asm volatile("s_nop 10" : "+v"(s[0]), "+v"(s[1]));
   else asm volatile("s_nop 10" : "+v"(s[0]), "+v"(s[1]), "+v"(s[2]), "+v"(s[3]));
 }
 

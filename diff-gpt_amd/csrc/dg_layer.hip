@@ -241,12 +241,22 @@ struct BlockInArgs {
   void* out;          // (M, 4C)
   int64_t w_ld, out_ld, M;
   int nsrc, dup;      // dup: source 1 is source 0, read once
+  // the embedding's form: row r of src[0] is row ids[r] of the table of V rows
+  // (ids outside it give NaN rows); its norm goes to x (M, C), the norm of that
+  // as stored into the projection
+  const int64_t* ids;
+  int64_t V;
+  void* x;
+  int64_t x_ld;
 };
 
 // SPLIT: the output columns are dealt to SPLIT workgroups (blockIdx.y), each
 // with the mixture of its own, where a few groups would leave CUs idle.
-template <typename T, int C, int NS, int RT, int SPLIT>
+// EMBED: the embedding's form.
+template <typename T, int C, int NS, int RT, int SPLIT, bool EMBED>
 __global__ __launch_bounds__(kLayerThreads, C == 64 ? 4 : 2) void block_in_kernel(const BlockInArgs a) {
+#pragma clang fp contract(off)
+  static_assert(!EMBED || RT == 1, "a workgroup gathers one group of rows");
   constexpr int LDC = lds_ld<T, C>();
   constexpr int CH = C / kRowLanes;
   constexpr int NT = 4 * C / 16 / kLayerWaves / SPLIT;  // output tiles per wave
@@ -268,10 +278,19 @@ __global__ __launch_bounds__(kLayerThreads, C == 64 ? 4 : 2) void block_in_kerne
     load_held<T, CH, HELD>(held, a.src, a.ld, a.nsrc, a.dup != 0, row, gc0);
   };
   int group = blockIdx.x;
-  if (rows_here) load_rows(group);
+  bool bad_id = false;
+  if constexpr (EMBED) {
+    if (rows_here) {
+      const int64_t id = a.ids[min((int64_t)group * ROWS + gr, a.M - 1)];
+      bad_id = id < 0 || id >= a.V;
+      load_row<T, CH>(held[0], static_cast<const T*>(a.src[0]) + (bad_id ? 0 : id) * a.ld[0] + gc0);
+    }
+  } else {
+    if (rows_here) load_rows(group);
+  }
 #pragma unroll
   for (int i = 0; i < RowRegs<T, CH>::WORDS; ++i) wmix.w[i] = 0u;
-  if (a.w_mix != nullptr) load_row<T, CH>(wmix, static_cast<const T*>(a.w_mix) + gc0);
+  if (!EMBED && a.w_mix != nullptr) load_row<T, CH>(wmix, static_cast<const T*>(a.w_mix) + gc0);
   TileW<T, C> w[NT];
   const RowRegs<T, 16>* wf[NT];
 #pragma unroll
@@ -284,7 +303,20 @@ __global__ __launch_bounds__(kLayerThreads, C == 64 ? 4 : 2) void block_in_kerne
 
   for (int buf = 0;; buf ^= 1) {
     // every wave left the products of the group before last at the last barrier
-    if (rows_here) {
+    if (EMBED && rows_here) {
+      // rms_norm(table row), stored, and the norm of the stored row
+      float x[CH];
+#pragma unroll
+      for (int i = 0; i < CH; ++i) x[i] = bad_id ? __builtin_nanf("") : elem<T, CH>(held[0], i);
+      row_rms<CH, kRowLanes>(x, C);
+      const int64_t row = (int64_t)group * ROWS + gr;
+      if (row < a.M && (SPLIT == 1 || blockIdx.y == 0))
+        store_vec<T, CH>(static_cast<T*>(a.x) + row * a.x_ld + gc0, x);
+#pragma unroll
+      for (int i = 0; i < CH; ++i) x[i] = rt<T>(x[i]);
+      row_rms<CH, kRowLanes>(x, C);
+      store_vec<T, CH>(xn[buf] + gr * LDC + gc0, x);
+    } else if (rows_here) {
       if (a.w_mix != nullptr) {  // uniform
         float h[CH];
         const int64_t row = min((int64_t)group * ROWS + gr, a.M - 1);
@@ -331,12 +363,32 @@ struct BlockOutArgs {
   int64_t y_ld, g_ld, wp_ld, pin_ld, wu_ld, wd_ld, out_ld, xn_ld, M;
   int nblk, dup;        // dup: block 1 is block 0, read once
   float alpha, limit;
+  // what follows the layer (its tail)
+  const void* t_mix;    // (C,) the next layer's pseudo-query (kTailIn)
+  const void* t_w;      // (t_n, C): the next layer's projections, or the lm_head's table (kTailHead)
+  void* t_out;          // (M, t_n)
+  int64_t* t_ids;       // (M,) first maximum of each logits row, or null
+  int64_t t_wld, t_old;
+  int t_n;
+  float t_cap;          // logit soft cap, 0: none
+};
+
+// What a launch adds after the layer.  At few rows every launch is a chain of
+// latencies, and the next one's rows are the rows this workgroup holds: its
+// weights are fetched under the FFN-down products instead.  n_embd 64 in fp32,
+// 32 rows, us: the layer 7.5 and the next one's projections 4.1 in one launch
+// 9.7, the head (5.7) 10.0; the embedding (4.1) and layer 0's projections 3.6.
+enum LayerTail {
+  kTailNone,
+  kTailIn,    // block_in_kernel of the next layer, whose sources are the committed blocks and out
+  kTailHead,  // lm_head_kernel over rms_norm(out)
 };
 
 // NS: the most committed blocks of the instance.
-template <typename T, int C, int NS, int RT>
+template <typename T, int C, int NS, int RT, LayerTail TAIL>
 __global__ __launch_bounds__(kLayerThreads, C == 64 ? 4 : 2) void block_out_kernel(const BlockOutArgs a) {
 #pragma clang fp contract(off)
+  static_assert(TAIL == kTailNone || (RT == 1 && (C == 64 || sizeof(T) == 2)), "a tail follows one group of rows");
   constexpr int LDC = lds_ld<T, C>(), LDH = lds_ld<T, 2 * C>();
   constexpr int CH = C / kRowLanes;
   constexpr int ROWS = RT * kLayerRows;
@@ -487,6 +539,25 @@ __global__ __launch_bounds__(kLayerThreads, C == 64 ? 4 : 2) void block_out_kern
         }
       }
     }
+    // the tail's operands, into the registers that the products above leave: its
+    // tiles are dealt to the waves in runs of tail_n from tail_0 on
+    constexpr int TB = NUP;  // tiles held at a time
+    const T* t_w = static_cast<const T*>(a.t_w);
+    const int tail_n = TAIL == kTailNone ? 0 : (a.t_n / 16 + kLayerWaves - 1) / kLayerWaves;
+    const int tail_0 = tail_n * wv;
+    const int tail_end = min(tail_0 + tail_n, a.t_n / 16);
+    if constexpr (TAIL != kTailNone) {
+#pragma unroll
+      for (int b = 0; b < TB; ++b)
+        if (tail_0 + b < tail_end) load_tile_w<T, C>(wu[b].r, t_w, a.t_wld, tail_0 + b, lane);
+      if constexpr (TAIL == kTailIn) {
+        if (rows_here) {
+          const int64_t row = min((int64_t)group * ROWS + gr, a.M - 1);
+          load_held<T, CH, HELD>(held, a.blk, a.blk_ld, a.nblk, a.dup != 0, row, gc0);
+          load_row<T, CH>(wmix, static_cast<const T*>(a.t_mix) + gc0);
+        }
+      }
+    }
     __syncthreads();
     // 5) FFN down + residual
     if (has_d) {
@@ -504,19 +575,83 @@ __global__ __launch_bounds__(kLayerThreads, C == 64 ? 4 : 2) void block_out_kern
         for (int i = 0; i < 4; ++i) o[i] = pmv[i] + rt<T>(acc[0][i]);
         if (row < a.M) store_vec<T, 4>(static_cast<T*>(a.out) + row * a.out_ld + col, o);
         // the same lane alone reads and writes this slice of pm
-        if (a.xn != nullptr) store_vec<T, 4>(pr, o);  // uniform
+        if (TAIL != kTailNone || a.xn != nullptr) store_vec<T, 4>(pr, o);  // uniform
       }
     }
-    // 6) dg_block_out_norm: the RMSNorm of the stored output rows (the head's
-    //    input after the last layer)
-    if (a.xn != nullptr) {  // uniform
+    // 6) the row work after the layer: dg_block_out_norm's and the head's
+    //    RMSNorm of the stored output rows, or the next layer's mixture and norm
+    if (TAIL != kTailNone || a.xn != nullptr) {  // uniform
       __syncthreads();
       if (rows_here) {
         float x[CH];
-        load_vec<T, CH>(pm + gr * LDC + gc0, x);
-        row_rms<CH, kRowLanes>(x, C);
         const int64_t row = (int64_t)group * ROWS + gr;
-        if (row < a.M) store_vec<T, CH>(static_cast<T*>(a.xn) + row * a.xn_ld + gc0, x);
+        if constexpr (TAIL == kTailIn) {
+          RowRegs<T, CH> last;
+          load_row<T, CH>(last, pm + gr * LDC + gc0);
+          layer_mixture<T, CH, NS, true>(held, a.nblk, a.blk, a.blk_ld, min(row, a.M - 1), gc0, last, wmix, C, x);
+        } else {
+          load_vec<T, CH>(pm + gr * LDC + gc0, x);
+          row_rms<CH, kRowLanes>(x, C);
+          if (a.xn != nullptr && row < a.M)
+            store_vec<T, CH>(static_cast<T*>(a.xn) + row * a.xn_ld + gc0, x);
+        }
+        // the FFN-up products read ga last, before the barrier of stage 5
+        if constexpr (TAIL != kTailNone) store_vec<T, CH>(ga + gr * LDC + gc0, x);
+      }
+    }
+    // 7) the tail's products
+    if constexpr (TAIL != kTailNone) {
+      __syncthreads();
+      const int64_t row = (int64_t)group * ROWS + c;
+      T* t_out = static_cast<T*>(a.t_out) + min(row, a.M - 1) * a.t_old + 4 * g;
+      float best = kNegInf;
+      int best_i = 0x7fffffff;
+#pragma unroll 1
+      for (int t0 = tail_0; t0 < tail_end; t0 += TB) {
+#pragma unroll
+        for (int b = 0; b < TB; ++b) {
+          const int t = t0 + b;
+          if (t >= tail_end) continue;  // wave-uniform
+          f32x4_t acc[1];
+          const RowRegs<T, 16>* const f[1] = {wu[b].r};
+          layer_tiles<T, C, 1>(acc, f, ga, lane);
+          mfma_settle(acc);
+          if (t + TB < tail_end) load_tile_w<T, C>(wu[b].r, t_w, a.t_wld, t + TB, lane);
+          float v[4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) v[i] = acc[0][i];
+          if constexpr (TAIL == kTailHead) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              v[i] = softcap_value<T>(v[i], a.t_cap);
+              if (v[i] > best) {  // entries rise with t and i: the first maximum stays
+                best = v[i];
+                best_i = 16 * t + 4 * g + i;
+              }
+            }
+          }
+          if (row < a.M) store_vec<T, 4>(t_out + 16 * t, v);
+        }
+      }
+      if (TAIL == kTailHead && a.t_ids != nullptr) {  // uniform
+        // hh's last readers passed the barrier of stage 6
+        float* red_v = reinterpret_cast<float*>(hh);
+        int* red_i = reinterpret_cast<int*>(red_v + kLayerWaves * kLayerRows);
+        first_max(best, best_i);
+        if (g == 0) {
+          red_v[wv * kLayerRows + c] = best;
+          red_i[wv * kLayerRows + c] = best_i;
+        }
+        __syncthreads();
+        if (threadIdx.x < kLayerRows && row < a.M) {
+          for (int q = 1; q < kLayerWaves; ++q) {  // waves in entry order
+            if (red_v[q * kLayerRows + c] > best) {
+              best = red_v[q * kLayerRows + c];
+              best_i = red_i[q * kLayerRows + c];
+            }
+          }
+          a.t_ids[row] = (int64_t)(best_i == 0x7fffffff ? 0 : best_i);
+        }
       }
     }
     // the next group's stages write ga, pm and hh again: every wave has passed
@@ -559,10 +694,23 @@ void launch_block_in_ns(const BlockInArgs& a, hipStream_t s) {
   // n_embd 64: two workgroups per group up to 256 groups (100 rows in fp32: 4.2
   // us, 5.2 with one; 6400 rows, 400 groups: 9.1, 8.8 with one).  n_embd 128:
   // four (1850 rows in fp32: 8.9 us, 12.8 with one; bf16 6.1 and 7.1)
-  if (deep) hipLaunchKernelGGL((block_in_kernel<T, C, NS, 2, 1>), dim3(grid), dim3(kLayerThreads), 0, s, a);
+  if (deep) hipLaunchKernelGGL((block_in_kernel<T, C, NS, 2, 1, false>), dim3(grid), dim3(kLayerThreads), 0, s, a);
   else if (C == 64 && grid > 256)
-    hipLaunchKernelGGL((block_in_kernel<T, C, NS, 1, 1>), dim3(grid), dim3(kLayerThreads), 0, s, a);
-  else hipLaunchKernelGGL((block_in_kernel<T, C, NS, 1, SPLIT>), dim3(grid, SPLIT), dim3(kLayerThreads), 0, s, a);
+    hipLaunchKernelGGL((block_in_kernel<T, C, NS, 1, 1, false>), dim3(grid), dim3(kLayerThreads), 0, s, a);
+  else
+    hipLaunchKernelGGL((block_in_kernel<T, C, NS, 1, SPLIT, false>), dim3(grid, SPLIT), dim3(kLayerThreads), 0, s,
+                       a);
+}
+
+// The embedding's form: a workgroup per 16 rows at any size.
+template <typename T, int C>
+void launch_embed_in(const BlockInArgs& a, hipStream_t s) {
+  constexpr int SPLIT = 4 * C / 16 / kLayerWaves;
+  const unsigned grid = layer_grid(a.M, false, C);
+  if (C == 64 && grid > 256)
+    hipLaunchKernelGGL((block_in_kernel<T, C, 4, 1, 1, true>), dim3(grid), dim3(kLayerThreads), 0, s, a);
+  else
+    hipLaunchKernelGGL((block_in_kernel<T, C, 4, 1, SPLIT, true>), dim3(grid, SPLIT), dim3(kLayerThreads), 0, s, a);
 }
 
 template <typename T, int C>
@@ -582,11 +730,35 @@ void launch_block_out_ns(const BlockOutArgs& a, hipStream_t s) {
   const unsigned grid = layer_grid(a.M, deep, C);
   if constexpr (kDeep) {
     if (deep) {
-      hipLaunchKernelGGL((block_out_kernel<T, C, NS, 2>), dim3(grid), dim3(kLayerThreads), 0, s, a);
+      hipLaunchKernelGGL((block_out_kernel<T, C, NS, 2, kTailNone>), dim3(grid), dim3(kLayerThreads), 0, s, a);
       return;
     }
   }
-  hipLaunchKernelGGL((block_out_kernel<T, C, NS, 1>), dim3(grid), dim3(kLayerThreads), 0, s, a);
+  hipLaunchKernelGGL((block_out_kernel<T, C, NS, 1, kTailNone>), dim3(grid), dim3(kLayerThreads), 0, s, a);
+}
+
+// With a tail: a workgroup per 16 rows at any size.
+template <typename T, int C, int NS>
+void launch_block_tail_ns(const BlockOutArgs& a, hipStream_t s) {
+  const dim3 grid(layer_grid(a.M, false, C)), block(kLayerThreads);
+  if (a.t_mix != nullptr) hipLaunchKernelGGL((block_out_kernel<T, C, NS, 1, kTailIn>), grid, block, 0, s, a);
+  else hipLaunchKernelGGL((block_out_kernel<T, C, NS, 1, kTailHead>), grid, block, 0, s, a);
+}
+
+// fp32 at n_embd 128 has none: 256 KB of weights a workgroup, fetched as they
+// are used, take longer than the launch they save (3 layers, 100 rows: 100 us
+// one by one, 106 joined).
+template <typename T, int C>
+int launch_block_tail(const BlockOutArgs& a, hipStream_t s) {
+  if constexpr (C == 128 && sizeof(T) == 4) {
+    set_error("block_out: n_embd 128 in fp32 is unsupported with what follows the layer");
+    return DG_EUNSUPPORTED;
+  } else {
+    if (a.nblk <= 4) launch_block_tail_ns<T, C, 4>(a, s);
+    else if (a.nblk <= 8) launch_block_tail_ns<T, C, 8>(a, s);
+    else launch_block_tail_ns<T, C, kMaxResSources>(a, s);
+    return check_launch("block_out_kernel");
+  }
 }
 
 template <typename T, int C>
@@ -639,11 +811,46 @@ extern "C" int dg_block_in(int64_t M, int C, int dtype, int nsrc, const void* co
   return check_launch("block_in_kernel");
 }
 
+extern "C" int dg_embed_in(int64_t M, int C, int dtype, const int64_t* ids, int64_t V, const void* table,
+                           int64_t table_ld, void* x, int64_t x_ld, const void* w_qkvg, int64_t w_ld, void* out,
+                           int64_t out_ld, void* stream) {
+  DG_REQUIRE(M >= 0 && C >= 1 && V >= 1, DG_EINVAL, "embed_in: bad sizes M=%lld C=%d V=%lld", (long long)M, C,
+             (long long)V);
+  DG_REQUIRE(layer_dtype_ok(dtype), DG_EUNSUPPORTED, "embed_in: dtype %d unsupported", dtype);
+  DG_REQUIRE(C == 64 || C == 128, DG_EUNSUPPORTED, "embed_in: n_embd %d unsupported (64 or 128)", C);
+  if (M == 0) return DG_OK;
+  DG_REQUIRE(ids && table && x && w_qkvg && out, DG_EINVAL, "embed_in: NULL pointer");
+  DG_REQUIRE(M <= (int64_t)kLayerRows * 0x7fffffffLL, DG_EINVAL, "embed_in: too many rows (%lld)", (long long)M);
+  DG_REQUIRE(table_ld >= C && x_ld >= C && w_ld >= C && out_ld >= 4 * (int64_t)C, DG_EINVAL,
+             "embed_in: a row stride is narrower than its row");
+  const int64_t es = dtype_bytes(dtype);
+  DG_REQUIRE(rows16(table, table_ld, es) && rows16(x, x_ld, es) && rows16(w_qkvg, w_ld, es) && rows16(out, out_ld, es),
+             DG_EUNSUPPORTED, "embed_in: rows must be 16-byte aligned");
+  BlockInArgs a{};
+  a.src[0] = table; a.ld[0] = table_ld; a.nsrc = 1;
+  a.ids = ids; a.V = V; a.x = x; a.x_ld = x_ld;
+  a.w = w_qkvg; a.out = out;
+  a.w_ld = w_ld; a.out_ld = out_ld; a.M = M;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  DG_LAYER(launch_embed_in);
+  return check_launch("block_in_kernel");
+}
+
+struct LayerTailArgs {
+  const void* mix;  // the next layer's pseudo-query; null: the head
+  const void* w;
+  void* out;
+  int64_t* ids;
+  int64_t w_ld, out_ld;
+  int n;
+  float cap;
+};
+
 static int block_out_impl(int64_t M, int C, int dtype, const void* y, int64_t y_ld, const void* g, int64_t g_ld,
                           const void* w_proj, int64_t wp_ld, const void* partial_in, int64_t pin_ld, int nblk,
                           const void* const* blocks, const int64_t* blocks_ld, const void* w_mix, const void* w_up,
                           int64_t wu_ld, const void* w_down, int64_t wd_ld, float alpha, float limit, void* out,
-                          int64_t out_ld, void* xn, int64_t xn_ld, void* stream) {
+                          int64_t out_ld, void* xn, int64_t xn_ld, const LayerTailArgs* tail, void* stream) {
   DG_REQUIRE(M >= 0 && C >= 1, DG_EINVAL, "block_out: bad sizes M=%lld C=%d", (long long)M, C);
   DG_REQUIRE(layer_dtype_ok(dtype), DG_EUNSUPPORTED, "block_out: dtype %d unsupported", dtype);
   DG_REQUIRE(C == 64 || C == 128, DG_EUNSUPPORTED, "block_out: n_embd %d unsupported (64 or 128)", C);
@@ -669,12 +876,29 @@ static int block_out_impl(int64_t M, int C, int dtype, const void* y, int64_t y_
     a.blk_ld[n] = blocks_ld[n];
   }
   DG_REQUIRE(ok, DG_EUNSUPPORTED, "block_out: rows must be 16-byte aligned");
+  if (tail != nullptr) {
+    DG_REQUIRE(tail->w && tail->out, DG_EINVAL, "block_out: NULL pointer");
+    DG_REQUIRE(tail->w_ld >= C && tail->out_ld >= tail->n && tail->cap >= 0.f, DG_EINVAL,
+               "block_out: bad strides or cap of what follows the layer");
+    const int n = tail->n;
+    DG_REQUIRE(n == 64 || n == 128 || n == 256 || n == 512 || n == 1024, DG_EUNSUPPORTED,
+               "block_out: vocabulary %d unsupported (64, 128, 256, 512 or 1024)", n);
+    DG_REQUIRE(rows16(tail->mix, 0, es) && rows16(tail->w, tail->w_ld, es) && rows16(tail->out, tail->out_ld, es),
+               DG_EUNSUPPORTED, "block_out: rows must be 16-byte aligned");
+    a.t_mix = tail->mix; a.t_w = tail->w; a.t_out = tail->out; a.t_ids = tail->ids;
+    a.t_wld = tail->w_ld; a.t_old = tail->out_ld; a.t_n = tail->n; a.t_cap = tail->cap;
+  }
   a.y = y; a.g = g; a.w_proj = w_proj; a.pin = partial_in; a.w_mix = w_mix; a.w_up = w_up; a.w_down = w_down;
   a.out = out; a.xn = xn;
   a.y_ld = y_ld; a.g_ld = g_ld; a.wp_ld = wp_ld; a.pin_ld = pin_ld; a.wu_ld = wu_ld; a.wd_ld = wd_ld;
   a.out_ld = out_ld; a.xn_ld = xn_ld; a.M = M; a.nblk = nblk; a.alpha = alpha; a.limit = limit;
   a.dup = nblk > 1 && blocks[1] == blocks[0] && blocks_ld[1] == blocks_ld[0] ? 1 : 0;
   hipStream_t s = static_cast<hipStream_t>(stream);
+  if (tail != nullptr) {
+    if (dtype == DG_F32) return C == 64 ? launch_block_tail<float, 64>(a, s) : launch_block_tail<float, 128>(a, s);
+    if (dtype == DG_BF16) return C == 64 ? launch_block_tail<bf16_t, 64>(a, s) : launch_block_tail<bf16_t, 128>(a, s);
+    return C == 64 ? launch_block_tail<f16_t, 64>(a, s) : launch_block_tail<f16_t, 128>(a, s);
+  }
   DG_LAYER(launch_block_out);
   return check_launch("block_out_kernel");
 }
@@ -685,7 +909,7 @@ extern "C" int dg_block_out(int64_t M, int C, int dtype, const void* y, int64_t 
                             const void* w_up, int64_t wu_ld, const void* w_down, int64_t wd_ld, float alpha,
                             float limit, void* out, int64_t out_ld, void* stream) {
   return block_out_impl(M, C, dtype, y, y_ld, g, g_ld, w_proj, wp_ld, partial_in, pin_ld, nblk, blocks, blocks_ld,
-                        w_mix, w_up, wu_ld, w_down, wd_ld, alpha, limit, out, out_ld, nullptr, 0, stream);
+                        w_mix, w_up, wu_ld, w_down, wd_ld, alpha, limit, out, out_ld, nullptr, 0, nullptr, stream);
 }
 
 extern "C" int dg_block_out_norm(int64_t M, int C, int dtype, const void* y, int64_t y_ld, const void* g,
@@ -696,5 +920,29 @@ extern "C" int dg_block_out_norm(int64_t M, int C, int dtype, const void* y, int
                                  int64_t xn_ld, void* stream) {
   DG_REQUIRE(M == 0 || xn != nullptr, DG_EINVAL, "block_out_norm: NULL pointer");
   return block_out_impl(M, C, dtype, y, y_ld, g, g_ld, w_proj, wp_ld, partial_in, pin_ld, nblk, blocks, blocks_ld,
-                        w_mix, w_up, wu_ld, w_down, wd_ld, alpha, limit, out, out_ld, xn, xn_ld, stream);
+                        w_mix, w_up, wu_ld, w_down, wd_ld, alpha, limit, out, out_ld, xn, xn_ld, nullptr, stream);
+}
+
+extern "C" int dg_block_out_in(int64_t M, int C, int dtype, const void* y, int64_t y_ld, const void* g, int64_t g_ld,
+                               const void* w_proj, int64_t wp_ld, const void* partial_in, int64_t pin_ld, int nblk,
+                               const void* const* blocks, const int64_t* blocks_ld, const void* w_mix,
+                               const void* w_up, int64_t wu_ld, const void* w_down, int64_t wd_ld, float alpha,
+                               float limit, void* out, int64_t out_ld, const void* next_mix, const void* next_qkvg,
+                               int64_t nq_ld, void* qkvg, int64_t qkvg_ld, void* stream) {
+  DG_REQUIRE(M == 0 || next_mix != nullptr, DG_EINVAL, "block_out_in: NULL pointer");
+  const LayerTailArgs tail{next_mix, next_qkvg, qkvg, nullptr, nq_ld, qkvg_ld, 4 * C, 0.f};
+  return block_out_impl(M, C, dtype, y, y_ld, g, g_ld, w_proj, wp_ld, partial_in, pin_ld, nblk, blocks, blocks_ld,
+                        w_mix, w_up, wu_ld, w_down, wd_ld, alpha, limit, out, out_ld, nullptr, 0, &tail, stream);
+}
+
+extern "C" int dg_block_out_head(int64_t M, int C, int dtype, const void* y, int64_t y_ld, const void* g,
+                                 int64_t g_ld, const void* w_proj, int64_t wp_ld, const void* partial_in,
+                                 int64_t pin_ld, int nblk, const void* const* blocks, const int64_t* blocks_ld,
+                                 const void* w_mix, const void* w_up, int64_t wu_ld, const void* w_down,
+                                 int64_t wd_ld, float alpha, float limit, void* out, int64_t out_ld, void* xn,
+                                 int64_t xn_ld, int V, const void* table, int64_t table_ld, float cap, void* logits,
+                                 int64_t logits_ld, int64_t* ids, void* stream) {
+  const LayerTailArgs tail{nullptr, table, logits, ids, table_ld, logits_ld, V, cap};
+  return block_out_impl(M, C, dtype, y, y_ld, g, g_ld, w_proj, wp_ld, partial_in, pin_ld, nblk, blocks, blocks_ld,
+                        w_mix, w_up, wu_ld, w_down, wd_ld, alpha, limit, out, out_ld, xn, xn_ld, &tail, stream);
 }

@@ -120,4 +120,27 @@ __device__ __forceinline__ float swiglu_value(float gate, float lin, float alpha
   return rt<T>(gate * s) * rt<T>(lin + 1.0f);
 }
 
+// A logit from its fp32 sum: rounded to T (F.linear's output), then, with cap
+// > 0, softcap_kernel's arithmetic and rounding.
+template <typename T>
+__device__ __forceinline__ float softcap_value(float v, float cap) {
+#pragma clang fp contract(off)
+  v = rt<T>(v);
+  return cap > 0.f ? rt<T>(cap * rt<T>(tanhf(rt<T>(v / cap)))) : v;
+}
+
+// The first maximum over the four lanes (l & 15, g) of a row: larger value, or
+// equal value and smaller entry.
+__device__ __forceinline__ void first_max(float& best, int& entry) {
+#pragma unroll
+  for (int off = 16; off <= 32; off <<= 1) {
+    const float ov = __shfl_xor(best, off, 64);
+    const int oi = __shfl_xor(entry, off, 64);
+    if (ov > best || (ov == best && oi < entry)) {
+      best = ov;
+      entry = oi;
+    }
+  }
+}
+
 }  // namespace dg

@@ -208,6 +208,30 @@ _SIGNATURES = {
         [ctypes.c_int64, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p,
          ctypes.c_int64, ctypes.c_void_p, ctypes.c_void_p],
     ),
+    "dg_embed_in": (
+        ctypes.c_int,
+        [ctypes.c_int64, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p,
+         ctypes.c_int64, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p,
+         ctypes.c_int64, ctypes.c_void_p],
+    ),
+    "dg_block_out_in": (
+        ctypes.c_int,
+        [ctypes.c_int64, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p,
+         ctypes.c_int64, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p, ctypes.c_int64, ctypes.c_int,
+         ctypes.POINTER(ctypes.c_void_p), ctypes.POINTER(ctypes.c_int64), ctypes.c_void_p, ctypes.c_void_p,
+         ctypes.c_int64, ctypes.c_void_p, ctypes.c_int64, ctypes.c_float, ctypes.c_float, ctypes.c_void_p,
+         ctypes.c_int64, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p, ctypes.c_int64,
+         ctypes.c_void_p],
+    ),
+    "dg_block_out_head": (
+        ctypes.c_int,
+        [ctypes.c_int64, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p,
+         ctypes.c_int64, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p, ctypes.c_int64, ctypes.c_int,
+         ctypes.POINTER(ctypes.c_void_p), ctypes.POINTER(ctypes.c_int64), ctypes.c_void_p, ctypes.c_void_p,
+         ctypes.c_int64, ctypes.c_void_p, ctypes.c_int64, ctypes.c_float, ctypes.c_float, ctypes.c_void_p,
+         ctypes.c_int64, ctypes.c_void_p, ctypes.c_int64, ctypes.c_int, ctypes.c_void_p, ctypes.c_int64,
+         ctypes.c_float, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p, ctypes.c_void_p],
+    ),
     "dg_block_out_norm": (
         ctypes.c_int,
         [ctypes.c_int64, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p,
@@ -618,11 +642,15 @@ def rms_norm_(x: torch.Tensor, out: torch.Tensor) -> None:
 
 
 def embed_norm_(ids: torch.Tensor, table: torch.Tensor, x_out: torch.Tensor,
-                xn_out: torch.Tensor | None) -> bool:
+                xn_out: torch.Tensor | None, w_qkvg: torch.Tensor | None = None,
+                qkvg: torch.Tensor | None = None) -> bool:
     """x_out = rms_norm(table[ids]) and, when given, xn_out = rms_norm(x_out)
     in one dg_embed_norm launch (bits of the separate launches; ids outside
-    the table give NaN rows).  False, with nothing launched, for what it does
-    not take: fp64, C > 8192, a table or output without unit column stride."""
+    the table give NaN rows).  With w_qkvg (4C, C) the launch projects
+    rms_norm(x_out) into qkvg (..., 4C) instead of storing it (dg_embed_in).
+    False, with nothing launched, for what it does not take: fp64, C > 8192, a
+    table or output without unit column stride (with w_qkvg: what block_in_
+    does not take)."""
     V, C = table.shape
     if table.dtype not in (torch.float32, torch.bfloat16, torch.float16) or C > 8192:
         return False
@@ -638,6 +666,21 @@ def embed_norm_(ids: torch.Tensor, table: torch.Tensor, x_out: torch.Tensor,
     if not i1.is_contiguous():
         i1 = i1.contiguous()
     xn2 = o2[1] if xn_out is not None else None
+    if w_qkvg is not None:
+        if xn2 is not None:
+            raise ValueError("embed_norm: the norm is either stored or projected")
+        if w_qkvg.shape != (4 * C, C) or w_qkvg.dtype != table.dtype or w_qkvg.stride(1) != 1:
+            return False
+        if qkvg.dtype != table.dtype or not qkvg.is_contiguous() or qkvg.numel() != i1.numel() * 4 * C:
+            raise ValueError("embed_norm: the projections' rows must be contiguous (..., 4C)")
+        rc = lib().dg_embed_in(
+            i1.numel(), C, _dtype_code(table), _ptr(i1), V, _ptr(table), table.stride(0), _ptr(o2[0]), C,
+            _ptr(w_qkvg), w_qkvg.stride(0), _ptr(qkvg), 4 * C, _stream(table),
+        )
+        if rc == DG_EUNSUPPORTED:
+            return False
+        _check(rc, "embed_in")
+        return True
     rc = lib().dg_embed_norm(
         i1.numel(), C, _dtype_code(table), _ptr(i1), V, _ptr(table), table.stride(0),
         _ptr(o2[0]), C, _ptr(xn2), C, _stream(table),
@@ -741,15 +784,32 @@ def block_in_(sources: list[torch.Tensor], w_mix: torch.Tensor | None, w_qkvg: t
     return True
 
 
+class Tail:
+    """What follows a layer over the same rows and can go with its launch: the
+    next layer's projections (w_mix its pseudo-query, w (4C, C), out (..., 4C))
+    or, with w_mix None, the head (w (V, C) the embedding table, out (..., V)
+    the logits, cap, ids the int64 argmax of each row or None).  done: a
+    launch has written out (and ids)."""
+
+    __slots__ = ("w_mix", "w", "out", "cap", "ids", "done")
+
+    def __init__(self, w_mix: torch.Tensor | None, w: torch.Tensor, out: torch.Tensor, cap: float = 0.0,
+                 ids: torch.Tensor | None = None) -> None:
+        self.w_mix, self.w, self.out, self.cap, self.ids, self.done = w_mix, w, out, cap, ids, False
+
+
 def block_out_(y: torch.Tensor, g: torch.Tensor, w_proj: torch.Tensor, partial_in: torch.Tensor | None,
                blocks: list[torch.Tensor], w_mix: torch.Tensor, w_up: torch.Tensor, w_down: torch.Tensor,
-               alpha: float, limit: float, out: torch.Tensor, xn_out: torch.Tensor | None = None) -> bool:
+               alpha: float, limit: float, out: torch.Tensor, xn_out: torch.Tensor | None = None,
+               tail: Tail | None = None) -> bool:
     """dg_block_out: from the attention output y (..., C) and the gate logits
     g, the layer's new partial sum into out: c_proj(y * sigmoid(g)), added to
     partial_in unless that is None (the layer commits its input), then plus
     the FFN of the MLP mixture over blocks and that partial.  With xn_out
-    (dg_block_out_norm) also rms_norm(out) into it.  Returns False, having
-    done nothing, for shapes the fused kernel does not take."""
+    (dg_block_out_norm) also rms_norm(out) into it.  A tail goes with the same
+    launch (dg_block_out_in, dg_block_out_head) where it can, and is left
+    undone otherwise.  Returns False, having done nothing, for shapes the fused
+    kernel does not take."""
     C = out.size(-1)
     y2, g2, o2 = _rows(y, "block_out"), _rows(g, "block_out"), out.view(-1, C)
     p2 = None if partial_in is None else _rows(partial_in, "block_out")
@@ -768,6 +828,26 @@ def block_out_(y: torch.Tensor, g: torch.Tensor, w_proj: torch.Tensor, partial_i
         _ptr(w_mix.reshape(-1).contiguous()), _ptr(w_up), w_up.stride(0), _ptr(w_down), w_down.stride(0),
         float(alpha), float(limit), _ptr(o2), o2.stride(0),
     ]
+    if tail is not None and tail.w.dtype == out.dtype and tail.w.stride(1) == 1 and tail.w.size(1) == C:
+        n = tail.w.size(0)
+        t2 = tail.out.view(-1, n)
+        if t2.size(0) != o2.size(0) or t2.dtype != out.dtype or (tail.w_mix is not None and n != 4 * C):
+            raise ValueError("block_out: inconsistent shapes after the layer")
+        if tail.ids is not None and (tail.ids.dtype != torch.int64 or tail.ids.numel() != o2.size(0)
+                                     or not tail.ids.is_contiguous()):
+            raise ValueError("block_out: ids must be a contiguous int64 tensor of the rows")
+        if tail.w_mix is None:
+            rc = lib().dg_block_out_head(*args, _ptr(x2), C, n, _ptr(tail.w), tail.w.stride(0), float(tail.cap),
+                                         _ptr(t2), n, _ptr(tail.ids), _stream(o2))
+        elif x2 is None:
+            rc = lib().dg_block_out_in(*args, _ptr(tail.w_mix.reshape(-1).contiguous()), _ptr(tail.w),
+                                       tail.w.stride(0), _ptr(t2), n, _stream(o2))
+        else:
+            rc = DG_EUNSUPPORTED  # the next layer's projections and the norm are not written together
+        if rc != DG_EUNSUPPORTED:
+            _check(rc, "block_out")
+            tail.done = True
+            return True
     if x2 is None:
         rc = lib().dg_block_out(*args, _stream(o2))
     else:

@@ -96,6 +96,8 @@ class Block(nn.Module):
         _last_only: bool = False,
         _xn: torch.Tensor | None = None,
         _xn_out: torch.Tensor | None = None,
+        _qkvg: torch.Tensor | None = None,
+        _tail: _native.Tail | None = None,
     ) -> tuple[tuple[torch.Tensor, ...], torch.Tensor]:
         """block.py:87-107.  With _last_only the attention still runs over
         every position (its keys and values go to the cache), and the rest of
@@ -106,10 +108,12 @@ class Block(nn.Module):
         caller (layer 0's, from the embedding launch).  _xn_out, when given
         (shaped as the returned partial sum), receives rms_norm of it: the
         head's input after the last layer, from the same launch when
-        dg_block_out takes the layer."""
+        dg_block_out takes the layer.  _qkvg, when given, is this layer's
+        q/k/v/g projections, computed by an earlier launch; _tail what follows
+        this layer (its ``done`` says whether the launch took it)."""
         _native.require_device("Block", partial_block)
         sa = self.sa
-        qkvg = self._project(blocks, partial_block, _xn)
+        qkvg = self._project(blocks, partial_block, _xn) if _qkvg is None else _qkvg
         committed = self._at_boundary()
         partial_in = partial_block
         if committed:
@@ -129,7 +133,7 @@ class Block(nn.Module):
             out = torch.empty_like(partial_in)
             if _native.block_out_(y, g, sa.c_proj.weight, None if committed else partial_in, list(blocks),
                                   self.mlp_res_proj.weight, up.weight, down.weight, swiglu.alpha, swiglu.limit,
-                                  out, _xn_out):
+                                  out, _xn_out, tail=_tail):
                 return blocks, out
         if not gated:
             _native.ops().gate_(y, g)  # y * sigmoid(g), mha.py:84

@@ -20,6 +20,15 @@ from diff_gpt.model.rope import precompute_freqs_cis
 from diff_gpt.sampler.sampler import Sampler
 from diff_gpt.sampler.temperature import TemperatureSampler, draw_one
 
+# n_embd -> the most rows whose launches are joined (GPT._joins).  Three layers
+# over rows of one token, us one by one -> joined: n_embd 64 in bf16, 100 rows
+# 51.7 -> 43.9, 8192 120 -> 111, 16384 193 -> 194 (32-row groups need the
+# launches of their own); in fp32, which has no 32-row form, 100 rows 59.7 ->
+# 51.4, 35328 480 -> 473, so any number.  n_embd 128 in bf16: 4096 rows 110 ->
+# 100, 8192 166 -> 178; in fp32 the embedding's launch alone joins: 100 rows
+# 99.9 -> 98.1, 16384 427 -> 430.
+JOINED_ROWS = {64: 8192, 128: 4096}
+
 
 def _ordinal_target_table(V: int, sigma: float, dtype: torch.dtype, device) -> torch.Tensor:
     """(V, V) table whose row t is the soft target for token t: a discretised
@@ -169,20 +178,47 @@ class GPT(BaseGPT):
             argmax_out.copy_(torch.argmax(logits, dim=-1))
         return logits
 
-    def _embed(self, idx: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor | None]:
-        """x = rms_norm(token_embedding_table(idx)) (gpt.py:154-155) and, when there
-        is a layer 0, rms_norm(x): one dg_embed_norm launch.  An id outside the
-        vocabulary gives a NaN row (nn.Embedding raises).  fp64 tables take
-        nn.Embedding and the RMSNorm kernel."""
+    def _embed(self, idx: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor | None, torch.Tensor | None]:
+        """x = rms_norm(token_embedding_table(idx)) (gpt.py:154-155) and, when
+        there is a layer 0, what it begins with: its q/k/v/g projections of
+        rms_norm(x) at few rows (one dg_embed_in launch), else rms_norm(x) (one
+        dg_embed_norm launch).  An id outside the vocabulary gives a NaN row
+        (nn.Embedding raises).  fp64 tables take nn.Embedding and the RMSNorm
+        kernel."""
         table = self.token_embedding_table.weight
         _native.require_device("GPT", idx, table)
         _native.require_inference("GPT", table)
         C = table.size(1)
         x = torch.empty((*idx.shape, C), dtype=table.dtype, device=table.device)
+        if self.blocks and self._joins(idx.numel()):
+            w = self.blocks[0].sa._projection_weight()
+            qkvg = torch.empty((*idx.shape, w.size(0)), dtype=table.dtype, device=table.device)
+            if _native.embed_norm_(idx, table, x, None, w, qkvg):
+                return x, None, qkvg
         xn0 = torch.empty_like(x) if self.blocks else None
         if _native.embed_norm_(idx, table, x, xn0):
-            return x, xn0
-        return rms_norm(self.token_embedding_table(idx)), None
+            return x, xn0, None
+        return rms_norm(self.token_embedding_table(idx)), None, None
+
+    def _joins(self, rows: int) -> bool:
+        """Whether, over ``rows`` rows, the embedding, the layers' projections and
+        the head go with the launch before them (not past hooks, which may read
+        or replace what lies between)."""
+        w = self.token_embedding_table.weight
+        if rows > JOINED_ROWS.get(w.size(1), 0) and not (w.size(1) == 64 and w.dtype == torch.float32):
+            return False
+        return not any(b._forward_hooks or b._forward_pre_hooks for b in self.blocks)
+
+    def _tail(self, i: int, partial: torch.Tensor, rows: tuple[int, int], ids: torch.Tensor | None) -> _native.Tail:
+        """What follows layer i over its (B, T) rows: layer i + 1's projections
+        or the head."""
+        alloc = lambda n: torch.empty((*rows, n), dtype=partial.dtype, device=partial.device)  # noqa: E731
+        if i + 1 < len(self.blocks):
+            block = self.blocks[i + 1]
+            w = block.sa._projection_weight()
+            return _native.Tail(block.attn_res_proj.weight, w, alloc(w.size(0)))
+        w = self.lm_head.weight
+        return _native.Tail(None, w, alloc(w.size(0)), float(self.logit_softcap), ids)
 
     def forward(
         self,
@@ -214,7 +250,7 @@ class GPT(BaseGPT):
 
         # the normalised embedding and, when layer 0 reads it, layer 0's
         # attention input rms_norm(x) (its one-block mixture) in one launch
-        x, xn0 = self._embed(idx)
+        x, xn0, qkvg = self._embed(idx)
         # Block-AttnRes state: the normalised embedding is block 0 and also the
         # first partial sum
         blocks: tuple[torch.Tensor, ...] = (x,)
@@ -224,14 +260,18 @@ class GPT(BaseGPT):
         xn_head = None
         if self.blocks:
             xn_head = torch.empty((B, 1 if _last_only else T, x.size(-1)), dtype=x.dtype, device=x.device)
+        tail = None
         for i, block in enumerate(self.blocks):
+            rows = (B, 1 if _last_only and i == last else T)
+            tail = self._tail(i, x, rows, _argmax_out) if self._joins(rows[0] * rows[1]) else None
             blocks, partial = block(blocks, partial, freqs_cis=freqs_cis, kv_cache=kv_cache,
                                     _last_only=_last_only and i == last, _xn=xn0 if i == 0 else None,
-                                    _xn_out=xn_head if i == last else None)
+                                    _xn_out=xn_head if i == last else None, _qkvg=qkvg, _tail=tail)
+            qkvg = tail.out if tail is not None and tail.done else None
         if _last_only and not self.blocks:
             partial = partial[:, -1:]
 
-        logits = self._head(partial, _argmax_out, xn_head)
+        logits = tail.out if tail is not None and tail.done else self._head(partial, _argmax_out, xn_head)
 
         loss = None
         if targets is not None:

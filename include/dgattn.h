@@ -502,6 +502,42 @@ DG_API int dg_block_out_norm(int64_t M, int C, int dtype, const void* y, int64_t
                              int64_t xn_ld, void* stream);
 
 /*
+ * dg_block_out and what follows it over the same rows, in one launch, at any
+ * number of rows (it pays where launches are latency-bound: a few thousand).
+ * dg_block_out_in: dg_block_in of the next layer over the sources blocks[0 ..
+ * nblk-1], out, with its pseudo-query next_mix and projections next_qkvg (4C,
+ * C), into qkvg (M, 4C).  dg_block_out_head (after the last layer): dg_lm_head
+ * of rms_norm(out) against table (V, C) with cap, into logits (M, V) and, when
+ * ids != NULL, the first maximum of each row; xn, when not NULL, receives
+ * rms_norm(out).  Bits of the separate calls.  Support as dg_block_out and
+ * dg_block_in, V as dg_lm_head, without fp32 at C = 128.
+ */
+DG_API int dg_block_out_in(int64_t M, int C, int dtype, const void* y, int64_t y_ld, const void* g, int64_t g_ld,
+                           const void* w_proj, int64_t wp_ld, const void* partial_in, int64_t pin_ld, int nblk,
+                           const void* const* blocks, const int64_t* blocks_ld, const void* w_mix,
+                           const void* w_up, int64_t wu_ld, const void* w_down, int64_t wd_ld, float alpha,
+                           float limit, void* out, int64_t out_ld, const void* next_mix, const void* next_qkvg,
+                           int64_t nq_ld, void* qkvg, int64_t qkvg_ld, void* stream);
+
+DG_API int dg_block_out_head(int64_t M, int C, int dtype, const void* y, int64_t y_ld, const void* g,
+                             int64_t g_ld, const void* w_proj, int64_t wp_ld, const void* partial_in,
+                             int64_t pin_ld, int nblk, const void* const* blocks, const int64_t* blocks_ld,
+                             const void* w_mix, const void* w_up, int64_t wu_ld, const void* w_down,
+                             int64_t wd_ld, float alpha, float limit, void* out, int64_t out_ld, void* xn,
+                             int64_t xn_ld, int V, const void* table, int64_t table_ld, float cap, void* logits,
+                             int64_t logits_ld, int64_t* ids, void* stream);
+
+/*
+ * dg_embed_norm and dg_block_in of layer 0 in one launch (gpt.py:154-155,
+ * mha.py:34-43): x (M, C) = rms_norm(table[ids]) and out (M, 4C) =
+ * rms_norm(x) @ w_qkvg^T.  Bits of the separate calls; an id outside [0, V)
+ * gives NaN rows.  Support as dg_block_in.
+ */
+DG_API int dg_embed_in(int64_t M, int C, int dtype, const int64_t* ids, int64_t V, const void* table,
+                       int64_t table_ld, void* x, int64_t x_ld, const void* w_qkvg, int64_t w_ld, void* out,
+                       int64_t out_ld, void* stream);
+
+/*
  * The sampler's draw (temperature.py:24-25, torch.multinomial with one
  * sample, by its Exp(1) method): ids[r] = the first index of the maximum of
  * probs[r, j] / q[r, j] over j < V, q the caller's Exp(1) variates (torch's
