@@ -371,6 +371,7 @@ struct BlockOutArgs {
   int64_t t_wld, t_old;
   int t_n;
   float t_cap;          // logit soft cap, 0: none
+  int* t_advance;       // device position to move on by one after the step, or null (kTailHead)
 };
 
 // What a launch adds after the layer.  At few rows every launch is a chain of
@@ -602,6 +603,8 @@ __global__ __launch_bounds__(kLayerThreads, C == 64 ? 4 : 2) void block_out_kern
     // 7) the tail's products
     if constexpr (TAIL != kTailNone) {
       __syncthreads();
+      // the step's readers of the position are launches before this one
+      if (TAIL == kTailHead && a.t_advance != nullptr && blockIdx.x == 0 && threadIdx.x == 0) *a.t_advance += 1;
       const int64_t row = (int64_t)group * ROWS + c;
       T* t_out = static_cast<T*>(a.t_out) + min(row, a.M - 1) * a.t_old + 4 * g;
       float best = kNegInf;
@@ -844,6 +847,7 @@ struct LayerTailArgs {
   int64_t w_ld, out_ld;
   int n;
   float cap;
+  int* advance;
 };
 
 static int block_out_impl(int64_t M, int C, int dtype, const void* y, int64_t y_ld, const void* g, int64_t g_ld,
@@ -887,6 +891,7 @@ static int block_out_impl(int64_t M, int C, int dtype, const void* y, int64_t y_
                DG_EUNSUPPORTED, "block_out: rows must be 16-byte aligned");
     a.t_mix = tail->mix; a.t_w = tail->w; a.t_out = tail->out; a.t_ids = tail->ids;
     a.t_wld = tail->w_ld; a.t_old = tail->out_ld; a.t_n = tail->n; a.t_cap = tail->cap;
+    a.t_advance = tail->advance;
   }
   a.y = y; a.g = g; a.w_proj = w_proj; a.pin = partial_in; a.w_mix = w_mix; a.w_up = w_up; a.w_down = w_down;
   a.out = out; a.xn = xn;
@@ -930,7 +935,7 @@ extern "C" int dg_block_out_in(int64_t M, int C, int dtype, const void* y, int64
                                float limit, void* out, int64_t out_ld, const void* next_mix, const void* next_qkvg,
                                int64_t nq_ld, void* qkvg, int64_t qkvg_ld, void* stream) {
   DG_REQUIRE(M == 0 || next_mix != nullptr, DG_EINVAL, "block_out_in: NULL pointer");
-  const LayerTailArgs tail{next_mix, next_qkvg, qkvg, nullptr, nq_ld, qkvg_ld, 4 * C, 0.f};
+  const LayerTailArgs tail{next_mix, next_qkvg, qkvg, nullptr, nq_ld, qkvg_ld, 4 * C, 0.f, nullptr};
   return block_out_impl(M, C, dtype, y, y_ld, g, g_ld, w_proj, wp_ld, partial_in, pin_ld, nblk, blocks, blocks_ld,
                         w_mix, w_up, wu_ld, w_down, wd_ld, alpha, limit, out, out_ld, nullptr, 0, &tail, stream);
 }
@@ -941,8 +946,8 @@ extern "C" int dg_block_out_head(int64_t M, int C, int dtype, const void* y, int
                                  const void* w_mix, const void* w_up, int64_t wu_ld, const void* w_down,
                                  int64_t wd_ld, float alpha, float limit, void* out, int64_t out_ld, void* xn,
                                  int64_t xn_ld, int V, const void* table, int64_t table_ld, float cap, void* logits,
-                                 int64_t logits_ld, int64_t* ids, void* stream) {
-  const LayerTailArgs tail{nullptr, table, logits, ids, table_ld, logits_ld, V, cap};
+                                 int64_t logits_ld, int64_t* ids, int32_t* advance, void* stream) {
+  const LayerTailArgs tail{nullptr, table, logits, ids, table_ld, logits_ld, V, cap, advance};
   return block_out_impl(M, C, dtype, y, y_ld, g, g_ld, w_proj, wp_ld, partial_in, pin_ld, nblk, blocks, blocks_ld,
                         w_mix, w_up, wu_ld, w_down, wd_ld, alpha, limit, out, out_ld, xn, xn_ld, &tail, stream);
 }

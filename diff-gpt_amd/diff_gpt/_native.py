@@ -230,7 +230,7 @@ _SIGNATURES = {
          ctypes.POINTER(ctypes.c_void_p), ctypes.POINTER(ctypes.c_int64), ctypes.c_void_p, ctypes.c_void_p,
          ctypes.c_int64, ctypes.c_void_p, ctypes.c_int64, ctypes.c_float, ctypes.c_float, ctypes.c_void_p,
          ctypes.c_int64, ctypes.c_void_p, ctypes.c_int64, ctypes.c_int, ctypes.c_void_p, ctypes.c_int64,
-         ctypes.c_float, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p, ctypes.c_void_p],
+         ctypes.c_float, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p],
     ),
     "dg_block_out_norm": (
         ctypes.c_int,
@@ -788,14 +788,16 @@ class Tail:
     """What follows a layer over the same rows and can go with its launch: the
     next layer's projections (w_mix its pseudo-query, w (4C, C), out (..., 4C))
     or, with w_mix None, the head (w (V, C) the embedding table, out (..., V)
-    the logits, cap, ids the int64 argmax of each row or None).  done: a
-    launch has written out (and ids)."""
+    the logits, cap, ids the int64 argmax of each row or None, advance an int32
+    device position to move on by one or None).  done: a launch has written out
+    (and ids, and advance)."""
 
-    __slots__ = ("w_mix", "w", "out", "cap", "ids", "done")
+    __slots__ = ("w_mix", "w", "out", "cap", "ids", "advance", "done")
 
     def __init__(self, w_mix: torch.Tensor | None, w: torch.Tensor, out: torch.Tensor, cap: float = 0.0,
-                 ids: torch.Tensor | None = None) -> None:
-        self.w_mix, self.w, self.out, self.cap, self.ids, self.done = w_mix, w, out, cap, ids, False
+                 ids: torch.Tensor | None = None, advance: torch.Tensor | None = None) -> None:
+        self.w_mix, self.w, self.out, self.cap, self.ids, self.advance = w_mix, w, out, cap, ids, advance
+        self.done = False
 
 
 def block_out_(y: torch.Tensor, g: torch.Tensor, w_proj: torch.Tensor, partial_in: torch.Tensor | None,
@@ -838,7 +840,7 @@ def block_out_(y: torch.Tensor, g: torch.Tensor, w_proj: torch.Tensor, partial_i
             raise ValueError("block_out: ids must be a contiguous int64 tensor of the rows")
         if tail.w_mix is None:
             rc = lib().dg_block_out_head(*args, _ptr(x2), C, n, _ptr(tail.w), tail.w.stride(0), float(tail.cap),
-                                         _ptr(t2), n, _ptr(tail.ids), _stream(o2))
+                                         _ptr(t2), n, _ptr(tail.ids), _ptr(tail.advance), _stream(o2))
         elif x2 is None:
             rc = lib().dg_block_out_in(*args, _ptr(tail.w_mix.reshape(-1).contiguous()), _ptr(tail.w),
                                        tail.w.stride(0), _ptr(t2), n, _stream(o2))

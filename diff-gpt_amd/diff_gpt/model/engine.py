@@ -72,9 +72,12 @@ class _DecodeGraph:
             cache.pos = pos0
             self.graph = torch.cuda.CUDAGraph()
             with torch.cuda.graph(self.graph):
-                logits, _ = model.forward(self.ids, kv_cache=cache)
+                if type(model) is GPT:  # the last launch may advance the position
+                    logits, _ = model.forward(self.ids, kv_cache=cache, _advance=True)
+                else:
+                    logits, _ = model.forward(self.ids, kv_cache=cache)
+                    cache.pos_dev.add_(1)
                 self.logits = logits[:, -1, :]
-                cache.pos_dev.add_(1)
             cache.pos = pos0
         except BaseException:
             cache.pos = pos0

@@ -209,7 +209,8 @@ class GPT(BaseGPT):
             return False
         return not any(b._forward_hooks or b._forward_pre_hooks for b in self.blocks)
 
-    def _tail(self, i: int, partial: torch.Tensor, rows: tuple[int, int], ids: torch.Tensor | None) -> _native.Tail:
+    def _tail(self, i: int, partial: torch.Tensor, rows: tuple[int, int], ids: torch.Tensor | None,
+              advance: torch.Tensor | None) -> _native.Tail:
         """What follows layer i over its (B, T) rows: layer i + 1's projections
         or the head."""
         alloc = lambda n: torch.empty((*rows, n), dtype=partial.dtype, device=partial.device)  # noqa: E731
@@ -218,7 +219,7 @@ class GPT(BaseGPT):
             w = block.sa._projection_weight()
             return _native.Tail(block.attn_res_proj.weight, w, alloc(w.size(0)))
         w = self.lm_head.weight
-        return _native.Tail(None, w, alloc(w.size(0)), float(self.logit_softcap), ids)
+        return _native.Tail(None, w, alloc(w.size(0)), float(self.logit_softcap), ids, advance)
 
     def forward(
         self,
@@ -228,6 +229,7 @@ class GPT(BaseGPT):
         *,
         _argmax_out: torch.Tensor | None = None,
         _last_only: bool = False,
+        _advance: bool = False,
     ) -> tuple[torch.Tensor, torch.Tensor | None]:
         """gpt.py:140-200.  _argmax_out (B, T) int64, when given, receives the
         first maximum of every logits row (greedy sampling without a separate
@@ -260,10 +262,11 @@ class GPT(BaseGPT):
         xn_head = None
         if self.blocks:
             xn_head = torch.empty((B, 1 if _last_only else T, x.size(-1)), dtype=x.dtype, device=x.device)
+        advance = kv_cache.pos_dev if _advance else None
         tail = None
         for i, block in enumerate(self.blocks):
             rows = (B, 1 if _last_only and i == last else T)
-            tail = self._tail(i, x, rows, _argmax_out) if self._joins(rows[0] * rows[1]) else None
+            tail = (self._tail(i, x, rows, _argmax_out, advance) if self._joins(rows[0] * rows[1]) else None)
             blocks, partial = block(blocks, partial, freqs_cis=freqs_cis, kv_cache=kv_cache,
                                     _last_only=_last_only and i == last, _xn=xn0 if i == 0 else None,
                                     _xn_out=xn_head if i == last else None, _qkvg=qkvg, _tail=tail)
@@ -271,7 +274,12 @@ class GPT(BaseGPT):
         if _last_only and not self.blocks:
             partial = partial[:, -1:]
 
-        logits = tail.out if tail is not None and tail.done else self._head(partial, _argmax_out, xn_head)
+        if tail is not None and tail.done:
+            logits = tail.out
+        else:
+            logits = self._head(partial, _argmax_out, xn_head)
+            if advance is not None:
+                advance.add_(1)
 
         loss = None
         if targets is not None:

@@ -509,7 +509,9 @@ DG_API int dg_block_out_norm(int64_t M, int C, int dtype, const void* y, int64_t
  * C), into qkvg (M, 4C).  dg_block_out_head (after the last layer): dg_lm_head
  * of rms_norm(out) against table (V, C) with cap, into logits (M, V) and, when
  * ids != NULL, the first maximum of each row; xn, when not NULL, receives
- * rms_norm(out).  Bits of the separate calls.  Support as dg_block_out and
+ * rms_norm(out); advance, when not NULL, is a device position that moves on by
+ * one (a decode step's last launch).  Bits of the separate calls.  Support as
+ * dg_block_out and
  * dg_block_in, V as dg_lm_head, without fp32 at C = 128.
  */
 DG_API int dg_block_out_in(int64_t M, int C, int dtype, const void* y, int64_t y_ld, const void* g, int64_t g_ld,
@@ -525,7 +527,7 @@ DG_API int dg_block_out_head(int64_t M, int C, int dtype, const void* y, int64_t
                              const void* w_mix, const void* w_up, int64_t wu_ld, const void* w_down,
                              int64_t wd_ld, float alpha, float limit, void* out, int64_t out_ld, void* xn,
                              int64_t xn_ld, int V, const void* table, int64_t table_ld, float cap, void* logits,
-                             int64_t logits_ld, int64_t* ids, void* stream);
+                             int64_t logits_ld, int64_t* ids, int32_t* advance, void* stream);
 
 /*
  * dg_embed_norm and dg_block_in of layer 0 in one launch (gpt.py:154-155,

@@ -133,3 +133,36 @@ def test_gpt_with_joined_launches(dev, dtype, embd, layers_per_block, monkeypatc
     assert all(torch.equal(a, b) for a, b in zip(joined, apart))
     assert all(torch.equal(a, b) for a, b in zip(hooked, hooked_apart))
     assert not torch.equal(hooked[0], joined[0])
+
+
+def test_head_advances_the_position(dev):
+    """A device position moves on by one with the head's launch, at one
+    workgroup and at many; the layer without a joined head adds it itself."""
+    from diff_gpt import _native
+
+    for M in (1, 100, 5000):
+        y, g, _, blocks, w = _layer(M, 64, 2, torch.float32, dev)
+        out, pos = torch.empty(M, 64, device=dev), torch.tensor([41, 7], dtype=torch.int32, device=dev)
+        table = _rand(1, dev, torch.float32, 256, 64)
+        tail = _native.Tail(None, table, torch.empty(M, 256, device=dev), 15.0, advance=pos)
+        assert _native.block_out_(y, g, w["proj"], None, blocks, w["mix"], w["up"], w["down"], 1.702, 7.0, out, tail=tail)
+        assert pos.tolist() == [42, 7]
+
+
+@pytest.mark.parametrize("vocab", [128, 192])  # 192: no joined head
+def test_step_advances_the_cache(dev, vocab):
+    from diff_gpt.model import gpt
+    from diff_gpt.model.kv_cache import KVCache
+
+    torch.manual_seed(0)
+    model = gpt.GPT(vocab_size=vocab, n_embd=64, block_size=32, n_head=4, n_layer=2, use_checkpoint=False).eval().to(dev)
+    kv = KVCache(batch_size=3, num_heads=4, seq_len=20, head_dim=16, num_layers=2)
+    ids = torch.randint(0, vocab, (3, 9), generator=torch.Generator().manual_seed(4)).to(dev)
+    with torch.inference_mode():
+        model(ids, kv_cache=kv)
+        kv.pos_dev = torch.tensor([9], dtype=torch.int32, device=dev)
+        model(ids[:, :1], kv_cache=kv, _advance=True)
+        assert kv.pos_dev.item() == 10
+        kv.pos = 10
+        model(ids[:, :1], kv_cache=kv)
+        assert kv.pos_dev.item() == 10
