@@ -27,7 +27,7 @@ LIB = PKG / "lib" / "libdgattn.so"
 TIMELINE_LIB = PKG / "lib" / "libdgattn_timeline.so"
 SOURCES = ["dg_abi.hip", "dg_rope.hip", "dg_attn_vec.hip", "dg_attn_mfma.hip", "dg_attn_mfma_f32.hip",
            "dg_attn_small.hip", "dg_attn_shared.hip", "dg_attn_wide.hip", "dg_block.hip", "dg_layer.hip",
-           "dg_noalloc.hip"]
+           "dg_linear.hip", "dg_noalloc.hip"]
 HEADERS = ["dg_common.h", "dg_rope_math.h", "dg_prefill.h", "dg_rows.h", str(REPO / "include" / "dgattn.h")]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")

@@ -208,6 +208,12 @@ _SIGNATURES = {
         [ctypes.c_int64, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p,
          ctypes.c_int64, ctypes.c_void_p, ctypes.c_void_p],
     ),
+    "dg_linear_rows": (
+        ctypes.c_int,
+        [ctypes.c_int64, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_int64,
+         ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p, ctypes.c_int64,
+         ctypes.c_int, ctypes.c_float, ctypes.c_float, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p],
+    ),
     "dg_embed_in": (
         ctypes.c_int,
         [ctypes.c_int64, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p,
@@ -857,6 +863,34 @@ def block_out_(y: torch.Tensor, g: torch.Tensor, w_proj: torch.Tensor, partial_i
     if rc == DG_EUNSUPPORTED:
         return False
     _check(rc, "block_out")
+    return True
+
+
+def linear_rows_(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, gate: torch.Tensor | None = None,
+                 residual: torch.Tensor | None = None, swiglu: tuple[float, float] | None = None) -> bool:
+    """dg_linear_rows: out (..., N) = (x [* sigmoid(gate)]) @ w^T [+ residual], or
+    with swiglu (alpha, limit) out (..., N/2) = the SwiGLU of x @ w^T.  Returns
+    False, having done nothing, for what it does not take."""
+    N, K = w.shape
+    o2, x2 = out.view(-1, out.size(-1)), _rows(x, "linear_rows")
+    g2 = None if gate is None else _rows(gate, "linear_rows")
+    r2 = None if residual is None else _rows(residual, "linear_rows")
+    M = o2.size(0)
+    if x2.shape != (M, K) or o2.size(1) != (N if swiglu is None else N // 2):
+        raise ValueError("linear_rows: inconsistent x/w/out shapes")
+    if (g2 is not None and g2.shape != (M, K)) or (r2 is not None and r2.shape != (M, N)):
+        raise ValueError("linear_rows: inconsistent gate/residual shapes")
+    if any(t is not None and t.dtype != out.dtype for t in (x2, w, g2, r2)) or w.stride(1) != 1 or o2.stride(1) != 1:
+        return False
+    ld = lambda t: 0 if t is None else t.stride(0)  # noqa: E731
+    alpha, limit = swiglu if swiglu is not None else (0.0, 0.0)
+    rc = lib().dg_linear_rows(
+        M, N, K, _dtype_code(out), _ptr(x2), ld(x2), _ptr(g2), ld(g2), _ptr(w), ld(w), _ptr(r2), ld(r2),
+        0 if swiglu is None else 1, float(alpha), float(limit), _ptr(o2), ld(o2), _stream(o2),
+    )
+    if rc == DG_EUNSUPPORTED:
+        return False
+    _check(rc, "linear_rows")
     return True
 
 

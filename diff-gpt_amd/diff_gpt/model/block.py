@@ -29,6 +29,26 @@ ATTN_RES_MAX_WIDTH = 2048
 # the widths dg_block_in and dg_block_out take
 LAYER_WIDTHS = (64, 128)
 
+
+
+def _few_rows(x: torch.Tensor, w: torch.Tensor, tile: int) -> bool:
+    """Whether F.linear(x, w) and the elementwise work around it go to
+    dg_linear_rows: 16-bit products whose workgroups, of 32 rows and ``tile``
+    features, times K stay within 256 x 1024, K at most 1024 (512 for the FFN's
+    first product).  Beyond, its tiles read the operands too often.  us, the
+    separate launches -> one, bf16:
+      gate, c_proj, sum    n_embd  512: 64 rows 9.5 -> 6.2, 512 9.0 -> 6.4, 2048 10.9 -> 16.1
+                           n_embd 1024: 64 rows 10.8 -> 8.9, 256 10.7 -> 9.3, 400 11.6 -> 15.9
+      FFN up, SwiGLU       n_embd  512: 64 rows 7.9 -> 5.5, 512 9.2 -> 8.2, 768 11.0 -> 11.4
+                           n_embd 1024: 16 rows 6.6 -> 7.5, 200 10.8 -> 13.7
+      FFN down, residual   n_embd  512: 64 rows 8.7 -> 6.1, 512 7.8 -> 6.3, 768 8.7 -> 9.7
+                           n_embd 1024: 16 rows 7.2 -> 8.3, 256 9.1 -> 9.9"""
+    N, K = w.shape
+    if x.dtype not in (torch.bfloat16, torch.float16) or K > 1024 or K % 512:
+        return False
+    return (x.numel() // K + 31) // 32 * (N // tile) * K <= 256 * 1024
+
+
 def block_attn_res(
     blocks: tuple[torch.Tensor, ...],
     partial_block: torch.Tensor,
@@ -135,10 +155,21 @@ class Block(nn.Module):
                                   self.mlp_res_proj.weight, up.weight, down.weight, swiglu.alpha, swiglu.limit,
                                   out, _xn_out, tail=_tail):
                 return blocks, out
-        if not gated:
-            _native.ops().gate_(y, g)  # y * sigmoid(g), mha.py:84
-        attn_out = sa.c_proj(y)
-        partial_block = attn_out if committed else partial_in + attn_out
+        joined = None
+        if not gated and _few_rows(y, sa.c_proj.weight, 32) and not (sa.c_proj._forward_hooks
+                                                                   or sa.c_proj._forward_pre_hooks):
+            # the gate, c_proj and the partial sum in one launch
+            joined = torch.empty_like(partial_in)
+            if not _native.linear_rows_(y, sa.c_proj.weight, joined, gate=g,
+                                        residual=None if committed else partial_in):
+                joined = None
+        if joined is not None:
+            partial_block = joined
+        else:
+            if not gated:
+                _native.ops().gate_(y, g)  # y * sigmoid(g), mha.py:84
+            attn_out = sa.c_proj(y)
+            partial_block = attn_out if committed else partial_in + attn_out
         out = self._mlp(blocks, partial_block)
         if _xn_out is not None:
             _native.rms_norm_(out, _xn_out)
@@ -168,5 +199,15 @@ class Block(nn.Module):
     def _mlp(self, blocks: tuple[torch.Tensor, ...], partial_block: torch.Tensor) -> torch.Tensor:
         xn = attn_res_norm(blocks, partial_block, self.mlp_res_proj)
         up, swiglu, down = self.ffwd.net
-        hidden = _native.ops().swiglu(F.linear(xn, up.weight), swiglu.alpha, swiglu.limit)
+        hidden = None
+        if up.weight.size(1) <= 512 and _few_rows(xn, up.weight, 64):
+            hidden = torch.empty((*xn.shape[:-1], up.weight.size(0) // 2), dtype=xn.dtype, device=xn.device)
+            if not _native.linear_rows_(xn, up.weight, hidden, swiglu=(swiglu.alpha, swiglu.limit)):
+                hidden = None
+        if hidden is None:
+            hidden = _native.ops().swiglu(F.linear(xn, up.weight), swiglu.alpha, swiglu.limit)
+        if _few_rows(hidden, down.weight, 32):
+            out = torch.empty_like(partial_block)
+            if _native.linear_rows_(hidden, down.weight, out, residual=partial_block):
+                return out
         return partial_block + F.linear(hidden, down.weight)

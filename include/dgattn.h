@@ -540,6 +540,22 @@ DG_API int dg_embed_in(int64_t M, int C, int dtype, const int64_t* ids, int64_t 
                        int64_t out_ld, void* stream);
 
 /*
+ * A linear layer over few rows with the elementwise work around it:
+ * out (M, N) = (x [* sigmoid(g)]) @ w^T [+ residual], or with swiglu out (M,
+ * N/2) = the clamped SwiGLU (alpha, limit) of x @ w^T's interleaved pairs
+ * (mha.py:84-85, feed_forward.py:10-14; g and residual are then NULL).
+ * Roundings as dg_gate, F.linear (the fp32 sum once), dg_swiglu and the
+ * residual add in turn; the sums' order is not hipBLASLt's, so the result
+ * agrees with the separate launches within rounding, not bit for bit.
+ * Supported: bf16 / fp16, K a multiple of 512, N of 32 (64 with swiglu),
+ * 16-byte aligned rows; anything else returns DG_EUNSUPPORTED and does
+ * nothing.  Any M, for a few hundred rows.
+ */
+DG_API int dg_linear_rows(int64_t M, int N, int K, int dtype, const void* x, int64_t x_ld, const void* g,
+                          int64_t g_ld, const void* w, int64_t w_ld, const void* residual, int64_t res_ld,
+                          int swiglu, float alpha, float limit, void* out, int64_t out_ld, void* stream);
+
+/*
  * The sampler's draw (temperature.py:24-25, torch.multinomial with one
  * sample, by its Exp(1) method): ids[r] = the first index of the maximum of
  * probs[r, j] / q[r, j] over j < V, q the caller's Exp(1) variates (torch's

@@ -128,7 +128,7 @@ def test_layers_gating_in_the_prefill_equal_the_gate_launch(dev, n_embd, n_head,
 
     torch.manual_seed(0)
     block = Block(n_embd, n_head, 1.702, 7.0, layer_idx=0).eval().to(dev).to(torch.bfloat16)
-    B, T, D = 2, 100, n_embd // n_head
+    B, T, D = 2, 700, n_embd // n_head  # more rows than dg_linear_rows takes, whose sums are ordered differently
     x = torch.randn(B, T, n_embd, device=dev).to(torch.bfloat16)
     other = torch.randn(B, T, n_embd, device=dev).to(torch.bfloat16)
     freqs = precompute_freqs_cis(D, T, 10000.0).to(dev).to(torch.bfloat16).view(1, T, 1, D // 2, 2)
