@@ -30,7 +30,6 @@ ATTN_RES_MAX_WIDTH = 2048
 LAYER_WIDTHS = (64, 128)
 
 
-
 def _few_rows(x: torch.Tensor, w: torch.Tensor, tile: int) -> bool:
     """Whether F.linear(x, w) and the elementwise work around it go to
     dg_linear_rows: 16-bit products whose workgroups, of 32 rows and ``tile``
@@ -43,10 +42,20 @@ def _few_rows(x: torch.Tensor, w: torch.Tensor, tile: int) -> bool:
                            n_embd 1024: 16 rows 6.6 -> 7.5, 200 10.8 -> 13.7
       FFN down, residual   n_embd  512: 64 rows 8.7 -> 6.1, 512 7.8 -> 6.3, 768 8.7 -> 9.7
                            n_embd 1024: 16 rows 7.2 -> 8.3, 256 9.1 -> 9.9"""
-    N, K = w.shape
-    if x.dtype not in (torch.bfloat16, torch.float16) or K > 1024 or K % 512:
+    if x.dtype not in (torch.bfloat16, torch.float16):
         return False
+    N, K = w.shape
+    if K > 1024 or K % 512:
+        return False
+    if torch.is_grad_enabled() and w.requires_grad:
+        return False  # F.linear records its product
     return (x.numel() // K + 31) // 32 * (N // tile) * K <= 256 * 1024
+
+
+def _plain_linear(m: nn.Module) -> bool:
+    """A Linear that nothing watches or replaces, whose product may be taken
+    from its weight."""
+    return type(m) is nn.Linear and m.bias is None and not m._forward_hooks and not m._forward_pre_hooks
 
 
 def block_attn_res(
@@ -147,7 +156,7 @@ class Block(nn.Module):
             y, g, partial_in = y[:, -1:], g[:, -1:], partial_in[:, -1:]
             blocks = tuple(b[:, -1:] for b in blocks)
         up, swiglu, down = self.ffwd.net
-        if not gated and len(blocks) + 1 <= ATTN_RES_MAX_SOURCES:
+        if not gated and sa.n_embd in LAYER_WIDTHS and len(blocks) + 1 <= ATTN_RES_MAX_SOURCES:
             # gate, c_proj, the partial sum, the MLP's mixture and norm, the FFN
             # and the residual in one launch (n_embd 64 or 128)
             out = torch.empty_like(partial_in)
@@ -156,8 +165,7 @@ class Block(nn.Module):
                                   out, _xn_out, tail=_tail):
                 return blocks, out
         joined = None
-        if not gated and _few_rows(y, sa.c_proj.weight, 32) and not (sa.c_proj._forward_hooks
-                                                                   or sa.c_proj._forward_pre_hooks):
+        if not gated and _few_rows(y, sa.c_proj.weight, 32) and _plain_linear(sa.c_proj):
             # the gate, c_proj and the partial sum in one launch
             joined = torch.empty_like(partial_in)
             if not _native.linear_rows_(y, sa.c_proj.weight, joined, gate=g,
@@ -200,7 +208,7 @@ class Block(nn.Module):
         xn = attn_res_norm(blocks, partial_block, self.mlp_res_proj)
         up, swiglu, down = self.ffwd.net
         hidden = None
-        if up.weight.size(1) <= 512 and _few_rows(xn, up.weight, 64):
+        if _few_rows(xn, up.weight, 64) and xn.size(-1) <= 512:
             hidden = torch.empty((*xn.shape[:-1], up.weight.size(0) // 2), dtype=xn.dtype, device=xn.device)
             if not _native.linear_rows_(xn, up.weight, hidden, swiglu=(swiglu.alpha, swiglu.limit)):
                 hidden = None

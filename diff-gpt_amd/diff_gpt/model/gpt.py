@@ -263,10 +263,13 @@ class GPT(BaseGPT):
         if self.blocks:
             xn_head = torch.empty((B, 1 if _last_only else T, x.size(-1)), dtype=x.dtype, device=x.device)
         advance = kv_cache.pos_dev if _advance else None
+        joins = self._joins(B * T)
+        joins_last = self._joins(B) if _last_only else joins
         tail = None
         for i, block in enumerate(self.blocks):
-            rows = (B, 1 if _last_only and i == last else T)
-            tail = (self._tail(i, x, rows, _argmax_out, advance) if self._joins(rows[0] * rows[1]) else None)
+            one = _last_only and i == last
+            rows = (B, 1 if one else T)
+            tail = self._tail(i, x, rows, _argmax_out, advance) if (joins_last if one else joins) else None
             blocks, partial = block(blocks, partial, freqs_cis=freqs_cis, kv_cache=kv_cache,
                                     _last_only=_last_only and i == last, _xn=xn0 if i == 0 else None,
                                     _xn_out=xn_head if i == last else None, _qkvg=qkvg, _tail=tail)
