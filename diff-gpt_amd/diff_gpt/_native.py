@@ -327,7 +327,12 @@ def require_inference(what: str, *tensors: torch.Tensor | None) -> None:
 
 
 def _stream(t: torch.Tensor) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+    # the handle alone: torch.cuda.current_stream builds a Stream object around
+    # it, several microseconds of every launch's host time
+    device = t.get_device()
+    if device < 0:
+        raise ValueError(f"expected a tensor on a ROCm device, got {t.device}")
+    return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(device))
 
 
 def _bthd_strides(t: torch.Tensor) -> Stride3:
