@@ -12,11 +12,14 @@
 //     D = 128).  S^T (16 keys x 16 rows) = K Q^T on v_mfma_f32_16x16x32, lane
 //     (c, g) = (l & 15, l >> 4) getting row c's scores of keys 4g .. 4g + 3; then
 //     O^T (16 dims x 16 rows) += V^T P^T, the lane's scores of two key tiles
-//     being its operand as they stand.  P enters as hi + lo, both rounded to
-//     the data type (lo the rounding error of hi), so the products carry twice
-//     the type's mantissa of each probability; sums are fp32.  V goes to LDS by
-//     direct copies (16-byte pieces XOR-swizzled by row, 8 KB per wave, no
-//     barrier) and comes back transposed (ds_read_b64_tr_b16).
+//     being its operand as they stand.  P enters as three terms of the data
+//     type, each the rounding error of those before it: all 24 bits of the fp32
+//     probability (of fp16's, what lies above 2^-41), with exact products and
+//     fp32 sums.  The second and third terms have an accumulator of their own,
+//     added at the end where the first one's is finite, so an infinite V gives
+//     the infinity that an fp32 probability would.  V goes to LDS by direct
+//     copies (16-byte pieces XOR-swizzled by row, 8 KB per wave, no barrier) and
+//     comes back transposed (ds_read_b64_tr_b16).
 //   * each wave first takes the own keys of two of the 16 rows, half a wave per
 //     row, as the vector kernel does (D / 8 lanes of 16 bytes per key), appends
 //     their new key and value, and adds the new key from registers at the end.
@@ -24,10 +27,14 @@
 //     merge the 8 prefix parts and the row's own part.
 //
 // All row tiles of one (group, head) run on one XCD, so its L2 holds their
-// prefix once.  Those 400 rows with 40 own keys: 15 us.  What bounds it then is
-// the latency of two chains in a workgroup, 64-key chunks of the prefix and 16-key
-// trips over the own keys (48 own keys after a 3000-token prefix: 21 us for 100
-// rows, 25 for 400); from some 6000 rows of 8 heads the rows' own K/V from HBM.
+// prefix once.  Those 400 rows with 40 own keys: 56 us in the vector kernel, 15.6
+// here (15.0 with two terms of P, 19.2 with fp32 P and V on
+// v_mfma_f32_16x16x4_f32).  What bounds it then is the latency of two chains in a
+// workgroup, 64-key chunks of the prefix and 16-key trips over the own keys (48
+// own keys after a 3000-token prefix: 21 us for 100 rows, 26 for 400); from some
+// 6000 rows of 8 heads the rows' own K/V from HBM.  The error against float64 is
+// the vector kernel's (400 rows, 1024 + 40 keys: 1.646443e-3 of the norm in bf16,
+// 2.064455e-4 in fp16, either kernel).
 #include "dg_prefill.h"
 #include "dg_rope_math.h"
 
@@ -95,6 +102,9 @@ __global__ __launch_bounds__(64 * kWideWaves, 4) void attn_wide_kernel(const Wid
   constexpr int KPH = 32 / LPK;    // keys per half-wave and slot
   constexpr int U = 4;             // slots per trip
   constexpr int PPR = D / 8;       // 16-byte pieces of a V row
+  // scale of a probability's second and third terms: fp16's exponents end at
+  // 2^-24, and a first term's rounding error is at most 2^-12 of 2^kLazyLog2
+  constexpr float kRest = __is_same(T, f16_t) ? 65536.0f : 1.0f;
   using Row = RowRegs<T, 8>;
   __shared__ __attribute__((aligned(16))) uint16_t stage[kWideWaves][4096];  // V, then the part's acc
   __shared__ __attribute__((aligned(16))) float own_acc[kWideRows][D];
@@ -267,9 +277,9 @@ __global__ __launch_bounds__(64 * kWideWaves, 4) void attn_wide_kernel(const Wid
   const int t16 = lane & 15;
 
   float m = kNegInf, l = 0.f;
-  f32x4_t o[NB];
+  f32x4_t o[NB], rest[NB];
 #pragma unroll
-  for (int nb = 0; nb < NB; ++nb) o[nb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  for (int nb = 0; nb < NB; ++nb) o[nb] = rest[nb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   for (int k0 = wv * KC; k0 < plen; k0 += kWideWaves * KC) {
     // every lane is done reading the chunk before (its products waited for
     // the reads) when the copies of this one go out
@@ -314,10 +324,13 @@ __global__ __launch_bounds__(64 * kWideWaves, 4) void attn_wide_kernel(const Wid
 #pragma unroll
       for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) o[nb][r] *= alpha;
+        for (int r = 0; r < 4; ++r) {
+          o[nb][r] *= alpha;
+          rest[nb][r] *= alpha;
+        }
     }
     const float moff = m * cl;
-    u32x4_t hi[NT / 2], lo[NT / 2];
+    u32x4_t p[NT / 2][3];  // P^T operands of 32 keys: the three terms
 #pragma unroll
     for (int u = 0; u < NT; ++u)
 #pragma unroll
@@ -326,10 +339,13 @@ __global__ __launch_bounds__(64 * kWideWaves, 4) void attn_wide_kernel(const Wid
         const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[u][2 * w + 1], cl, -moff));
         l += p0;
         l += p1;
-        RowRegs<T, 2> h;
-        h.w[0] = pack_pair<T>(p0, p1);
-        hi[u / 2][2 * (u & 1) + w] = h.w[0];
-        lo[u / 2][2 * (u & 1) + w] = pack_pair<T>(p0 - elem<T, 2>(h, 0), p1 - elem<T, 2>(h, 1));
+        RowRegs<T, 2> term[3];
+        term[0].w[0] = pack_pair<T>(p0, p1);
+        const float r0 = (p0 - elem<T, 2>(term[0], 0)) * kRest, r1 = (p1 - elem<T, 2>(term[0], 1)) * kRest;
+        term[1].w[0] = pack_pair<T>(r0, r1);
+        term[2].w[0] = pack_pair<T>(r0 - elem<T, 2>(term[1], 0), r1 - elem<T, 2>(term[1], 1));
+#pragma unroll
+        for (int k = 0; k < 3; ++k) p[u / 2][k][2 * (u & 1) + w] = term[k].w[0];
       }
     // this wave's V copies are in LDS
     __builtin_amdgcn_s_waitcnt(0);
@@ -347,8 +363,9 @@ __global__ __launch_bounds__(64 * kWideWaves, 4) void attn_wide_kernel(const Wid
           vv[u] = lds_read_tr16(st + row * D + 8 * wide_slot<D>(col >> 3, row) + (col & 7));
         }
         const u32x4_t vf = {vv[0].x, vv[0].y, vv[1].x, vv[1].y};
-        o[nb] = wide_mma<T>(vf, hi[t], o[nb]);
-        o[nb] = wide_mma<T>(vf, lo[t], o[nb]);
+        o[nb] = wide_mma<T>(vf, p[t][0], o[nb]);
+        rest[nb] = wide_mma<T>(vf, p[t][1], rest[nb]);
+        rest[nb] = wide_mma<T>(vf, p[t][2], rest[nb]);
       }
   }
   float x, y;
@@ -364,7 +381,14 @@ __global__ __launch_bounds__(64 * kWideWaves, 4) void attn_wide_kernel(const Wid
   float* part = reinterpret_cast<float*>(st);
 #pragma unroll
   for (int nb = 0; nb < NB; ++nb) {
-    const float w[4] = {o[nb][0], o[nb][1], o[nb][2], o[nb][3]};
+    float w[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      // a value that is not finite has made the first terms' sum so, and the
+      // others' (whose terms are zero or negative for some keys) a NaN
+      const bool finite = __builtin_fabsf(o[nb][r]) < __builtin_huge_valf();
+      w[r] = finite ? __builtin_fmaf(rest[nb][r], 1.0f / kRest, o[nb][r]) : o[nb][r];
+    }
     store_vec<float, 4>(part + c * D + 4 * ((4 * nb + g) ^ (c & (UPR - 1))), w);
   }
   if (g == 0) {
@@ -411,14 +435,15 @@ bool w16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 // saved, (rows * heads * P) key reads, can repay.  Both sides of the line, 8 heads
 // of 64, us with the vector kernel -> here (D = 128 alike, both about twice):
 //   rows * heads * P >= 3300 * own_max + 200000 (own_max: the own pages' room)
-//     1 x 100 rows, P  200, own  48 of   96:  10.0 ->   9.2 below the line
-//     1 x 100 rows, P 1024, own 250 of  256:  30.2 ->  24.9 just below
-//     1 x  20 rows, P 1024, own 250 of  256:  11.8 ->  22.2 below
-//    32 x  32 rows, P   64, own  48 of   96:  25.2 ->  22.4 just above
-//    32 x  32 rows, P 1024, own 1000 of 1024: 438 ->  391   above
-//     4 x 100 rows, P 3000, own   8 of   96:   146 ->  21.2 above
-//   rows * heads >= 320: 20 rows x 8, P 3000, own 48 of 96: 20.0 -> 21.0
-//   2 P >= own_max: 64 x 100 rows, P 64, own 250 of 256: 559 -> 582
+//     1 x 100 rows, P  200, own  48 of   96:   9.5 ->   9.1 below the line
+//     1 x 100 rows, P 1024, own 250 of  256:  30.6 ->  24.4 just below
+//     1 x  20 rows, P 1024, own 250 of  256:  11.4 ->  22.1 below
+//    32 x  32 rows, P   64, own  48 of   96:  24.7 ->  21.8 just above
+//     2 x  32 rows, P 1100, own  48 of   96:  14.8 ->  12.9 just above
+//    32 x  32 rows, P 1024, own 1000 of 1024: 452 ->  389   above
+//     4 x 100 rows, P 3000, own   8 of   96:   142 ->  21.7 above
+//   rows * heads >= 320: 20 rows x 8, P 3000, own 48 of 96: 18.7 -> 20.9
+//   2 P >= own_max: 64 x 100 rows, P 64, own 250 of 256: 564 -> 590
 bool wide_step_applicable(int B, int H, int D, int dtype, const PrefixRef& pre, int max_pos, const void* q,
                           const dg_stride3* q_st, const void* k, const dg_stride3* k_st, const void* v,
                           const dg_stride3* v_st, const void* kc, const dg_stride3* kc_st, const void* vc,
