@@ -81,18 +81,23 @@ __device__ __forceinline__ float rt(float x) {
   return to_f32(from_f32<T>(x));
 }
 
-// sigmoid rounded to T.  fp32: as ATen evaluates it, 1 / (1 + exp(-x)).  16-bit
-// types: the hardware exp2 and reciprocal (a few units of 2^-22, far below the
-// rounding to T that follows) in place of expf and a correctly rounded divide,
-// which at about 40 VALU instructions per element bounded the gate over a
-// prefill's rows (gate_vec_kernel).
+// sigmoid(x) rounded to T, of an x that is a value of T.  fp32: as ATen evaluates
+// it, 1 / (1 + exp(-x)).  16-bit types: the hardware exp2 and reciprocal in place
+// of expf and a correctly rounded divide, which at about 40 VALU instructions per
+// element bounded the gate over a prefill's rows (gate_vec_kernel).  The fp32
+// value is then off by about (2 + |x|) 2^-23 of itself (the rounded product with
+// log2(e) is an error of the exponent), and the rounding to T takes it to the
+// value ATen's sequence rounds to for every one of T's 65536 arguments (the tests
+// go through all).  The reciprocal is taken of a quarter of the sum, since it
+// flushes a result below 2^-126, which sigmoid reaches at -87.3, to zero.
 template <typename T>
 __device__ __forceinline__ float sigmoid_rt(float x) {
 #pragma clang fp contract(off)
   if constexpr (sizeof(T) == 4) {
     return 1.0f / (1.0f + expf(-x));
   } else {
-    return rt<T>(__builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x * -1.44269504f)));
+    const float e = __builtin_amdgcn_exp2f(x * -1.44269504f);
+    return rt<T>(__builtin_amdgcn_rcpf(__builtin_fmaf(0.25f, e, 0.25f)) * 0.25f);
   }
 }
 

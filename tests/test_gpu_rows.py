@@ -62,6 +62,38 @@ def test_gate_limits(dev, dtype):
     assert bool((d <= tol * ref.double().abs().nan_to_num(0.0) + torch.finfo(TDT[dtype]).tiny).all())
 
 
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+def test_sigmoid_of_every_argument(dev, dtype):
+    """The gate and the SwiGLU of all 65536 arguments of a 16-bit type, in their
+    vector and general forms, are torch's own sequence on the device bit for bit:
+    subnormal results (arguments from -87.5 to -88.5 in bf16) included.  NaN
+    arguments go to the gate alone (swi_glu.py's clamp passes them on, the
+    kernel's minimum does not)."""
+    from diff_gpt import _native
+
+    dt = TDT[dtype]
+    bits = lambda t: t.contiguous().view(torch.int16)  # noqa: E731
+    x = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(dt).to(dev).view(256, 256)
+    nan = x.isnan()
+    for y in (1.0, 1.25):
+        ref = torch.full_like(x, y) * torch.sigmoid(x)
+        for off in (0, 1):
+            g, got = (torch.zeros(256, 264, dtype=dt, device=dev)[:, off : off + 256] for _ in range(2))
+            g.copy_(x)
+            got.fill_(y)
+            _native.gate_(got, g)
+            assert torch.equal(got.isnan(), nan) and torch.equal(bits(got)[~nan], bits(ref)[~nan])
+    gate = x.clamp(max=7.0)
+    ref = gate * torch.sigmoid(1.702 * gate) * (torch.zeros_like(x) + 1)
+    for off in (0, 1):
+        pairs = torch.zeros(256, 520, dtype=dt, device=dev)[:, off : off + 512]
+        pairs[:, ::2] = x
+        out = torch.empty(256, 256, dtype=dt, device=dev)
+        _native.swiglu_(pairs, out, 1.702, 7.0)
+        assert torch.equal(bits(out)[~nan & ~ref.isnan()], bits(ref)[~nan & ~ref.isnan()])
+        assert bool(out[~nan & ref.isnan()].isnan().all())
+
+
 @pytest.mark.parametrize("dtype", ["f32", "bf16", "f16"])
 @pytest.mark.parametrize("C", [64, 256, 512, 1024, 2048])
 @pytest.mark.parametrize("n", [1, 2, 4, 5, 7, 8, 12, 13])
