@@ -16,6 +16,7 @@ residual -- one dg_block_out launch instead of six.
 import torch
 import torch.nn.functional as F
 from torch import nn
+from torch.nn.modules import module as _modules
 
 from diff_gpt import _native
 from diff_gpt.model.feed_forward import FeedForward
@@ -50,6 +51,16 @@ def _few_rows(x: torch.Tensor, w: torch.Tensor, tile: int) -> bool:
     if torch.is_grad_enabled() and w.requires_grad:
         return False  # F.linear records its product
     return (x.numel() // K + 31) // 32 * (N // tile) * K <= 256 * 1024
+
+
+def as_written(m: nn.Module, cls: type, forward) -> bool:
+    """Whether calling m runs cls's own ``forward`` and nothing else: not a
+    subclass's, not one put into the instance or the class since, no hooks on the
+    module or on all modules, not compiled."""
+    return (type(m) is cls and cls.forward is forward and "forward" not in m.__dict__
+            and not m._forward_hooks and not m._forward_pre_hooks
+            and not _modules._global_forward_hooks and not _modules._global_forward_pre_hooks
+            and m._compiled_call_impl is None)
 
 
 def _plain_linear(m: nn.Module) -> bool:
@@ -219,3 +230,12 @@ class Block(nn.Module):
             if _native.linear_rows_(hidden, down.weight, out, residual=partial_block):
                 return out
         return partial_block + F.linear(hidden, down.weight)
+
+
+_BLOCK_FORWARD = Block.forward
+
+
+def plain_block(m: nn.Module) -> bool:
+    """Whether m's output is what Block.forward returned, so that the launch inside
+    may go on with what reads it."""
+    return as_written(m, Block, _BLOCK_FORWARD)

@@ -21,7 +21,7 @@ from typing import Generator, Sequence
 import numpy as np
 import torch
 
-from diff_gpt.model.gpt import GPT, BaseGPT
+from diff_gpt.model.gpt import GPT, BaseGPT, plain_gpt
 from diff_gpt.model.kv_cache import KVCache
 from diff_gpt.sampler.sampler import Sampler
 from diff_gpt.sampler.temperature import draw_one
@@ -72,7 +72,7 @@ class _DecodeGraph:
             cache.pos = pos0
             self.graph = torch.cuda.CUDAGraph()
             with torch.cuda.graph(self.graph):
-                if type(model) is GPT:  # the last launch may advance the position
+                if plain_gpt(model):  # the last launch may advance the position
                     logits, _ = model.forward(self.ids, kv_cache=cache, _advance=True)
                 else:
                     logits, _ = model.forward(self.ids, kv_cache=cache)

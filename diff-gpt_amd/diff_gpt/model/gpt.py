@@ -13,7 +13,7 @@ import torch.nn as nn
 from torch.nn import functional as F
 
 from diff_gpt import _native
-from diff_gpt.model.block import Block
+from diff_gpt.model.block import Block, plain_block
 from diff_gpt.model.kv_cache import KVCache
 from diff_gpt.model.rms_norm import rms_norm
 from diff_gpt.model.rope import precompute_freqs_cis
@@ -202,22 +202,25 @@ class GPT(BaseGPT):
 
     def _joins(self, rows: int) -> bool:
         """Whether, over ``rows`` rows, the embedding, the layers' projections and
-        the head go with the launch before them (not past hooks, which may read
-        or replace what lies between)."""
+        the head go with the launch before them: only where every layer is a Block
+        as written, since an overridden forward or a hook may read or replace what
+        lies between."""
         w = self.token_embedding_table.weight
         if rows > JOINED_ROWS.get(w.size(1), 0) and not (w.size(1) == 64 and w.dtype == torch.float32):
             return False
-        return not any(b._forward_hooks or b._forward_pre_hooks for b in self.blocks)
+        return all(plain_block(b) for b in self.blocks)
 
     def _tail(self, i: int, partial: torch.Tensor, rows: tuple[int, int], ids: torch.Tensor | None,
-              advance: torch.Tensor | None) -> _native.Tail:
+              advance: torch.Tensor | None) -> _native.Tail | None:
         """What follows layer i over its (B, T) rows: layer i + 1's projections
-        or the head."""
+        or the head (not an overridden one)."""
         alloc = lambda n: torch.empty((*rows, n), dtype=partial.dtype, device=partial.device)  # noqa: E731
         if i + 1 < len(self.blocks):
             block = self.blocks[i + 1]
             w = block.sa._projection_weight()
             return _native.Tail(block.attn_res_proj.weight, w, alloc(w.size(0)))
+        if type(self)._head is not _GPT_HEAD or "_head" in self.__dict__:
+            return None
         w = self.lm_head.weight
         return _native.Tail(None, w, alloc(w.size(0)), float(self.logit_softcap), ids, advance)
 
@@ -270,9 +273,11 @@ class GPT(BaseGPT):
             one = _last_only and i == last
             rows = (B, 1 if one else T)
             tail = self._tail(i, x, rows, _argmax_out, advance) if (joins_last if one else joins) else None
+            # a Block with a forward of its own is not handed what joined launches pass on
+            joined = {} if qkvg is None and tail is None else {"_qkvg": qkvg, "_tail": tail}
             blocks, partial = block(blocks, partial, freqs_cis=freqs_cis, kv_cache=kv_cache,
                                     _last_only=_last_only and i == last, _xn=xn0 if i == 0 else None,
-                                    _xn_out=xn_head if i == last else None, _qkvg=qkvg, _tail=tail)
+                                    _xn_out=xn_head if i == last else None, **joined)
             qkvg = tail.out if tail is not None and tail.done else None
         if _last_only and not self.blocks:
             partial = partial[:, -1:]
@@ -336,3 +341,13 @@ class GPT(BaseGPT):
     @property
     def device_type(self) -> str:
         return str(self.freqs_cis.device.type)
+
+
+_GPT_HEAD = GPT._head
+_GPT_FORWARD = GPT.forward
+
+
+def plain_gpt(model: nn.Module) -> bool:
+    """Whether model.forward is GPT.forward as written, which takes the private
+    arguments of a captured step."""
+    return type(model) is GPT and GPT.forward is _GPT_FORWARD and "forward" not in model.__dict__

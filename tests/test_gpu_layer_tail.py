@@ -5,6 +5,9 @@ with and without them."""
 import pytest
 import torch
 
+from diff_gpt.model.block import Block
+from diff_gpt.model.rms_norm import rms_norm
+
 pytestmark = pytest.mark.gpu
 
 TDT = {"f32": torch.float32, "bf16": torch.bfloat16, "f16": torch.float16}
@@ -133,6 +136,124 @@ def test_gpt_with_joined_launches(dev, dtype, embd, layers_per_block, monkeypatc
     assert all(torch.equal(a, b) for a, b in zip(joined, apart))
     assert all(torch.equal(a, b) for a, b in zip(hooked, hooked_apart))
     assert not torch.equal(hooked[0], joined[0])
+
+
+class _Doubled(Block):
+    """A layer with a forward of its own, of the arguments a Block took before
+    launches were joined."""
+
+    def forward(self, blocks, partial_block, freqs_cis, kv_cache, *, _last_only=False, _xn=None, _xn_out=None):
+        blocks, out = super().forward(blocks, partial_block, freqs_cis, kv_cache, _last_only=_last_only, _xn=_xn)
+        out = out * 2
+        if _xn_out is not None:
+            _xn_out.copy_(rms_norm(out))
+        return blocks, out
+
+
+@pytest.mark.parametrize("embd", [64, 128])
+@pytest.mark.parametrize("layer", [0, 1, 2])
+def test_an_overridden_layer_is_heard(dev, embd, layer, monkeypatch):
+    """A layer's output replaced by a subclass, by a forward put into the instance
+    or the class, or by a hook on all modules is what the next layer and the head
+    read, as it is with a hook on the layer (whose head reads the last layer's
+    norm by way of _xn_out, so only the next layer's input shows there)."""
+    from torch.nn.modules.module import register_module_forward_hook
+
+    from diff_gpt.model import gpt
+
+    def build():
+        torch.manual_seed(0)
+        return gpt.GPT(vocab_size=128, n_embd=embd, block_size=32, n_head=4, n_layer=3,
+                       use_checkpoint=False).eval().to(dev).to(torch.bfloat16)
+
+    idx = torch.randint(0, 128, (3, 17), generator=torch.Generator().manual_seed(4)).to(dev)
+
+    @torch.inference_mode()
+    def logits(model):
+        return model(idx)[0]
+
+    plain = logits(build())
+    model = build()
+    model.blocks[layer].__class__ = _Doubled
+    doubled = logits(model)
+    assert not torch.equal(doubled, plain) or layer == 2  # 2 x keeps the head's norm but for its epsilon
+    model = build()
+    with monkeypatch.context() as m:
+        m.setattr(gpt.GPT, "_joins", lambda self, rows: False)
+        model.blocks[layer].__class__ = _Doubled
+        assert torch.equal(logits(model), doubled)
+    # the same by an instance's forward
+    model = build()
+    block = model.blocks[layer]
+    inner = Block.forward
+
+    def doubling(blocks, partial_block, freqs_cis, kv_cache, *, _last_only=False, _xn=None, _xn_out=None):
+        blocks, out = inner(block, blocks, partial_block, freqs_cis, kv_cache, _last_only=_last_only, _xn=_xn)
+        out = out * 2
+        if _xn_out is not None:
+            _xn_out.copy_(rms_norm(out))
+        return blocks, out
+
+    block.forward = doubling
+    assert torch.equal(logits(model), doubled)
+    del block.forward
+    assert torch.equal(logits(model), plain)
+    # by the class's, and by a hook on all modules
+    if layer < 2:
+        hook = block.register_forward_hook(lambda mod, i, o: (o[0], o[1] * 2))
+        hooked = logits(model)
+        hook.remove()
+        assert torch.equal(hooked, doubled)
+        with monkeypatch.context() as m:
+            m.setattr(Block, "forward",
+                      lambda self, *a, **k: (lambda o: (o[0], o[1] * 2) if self is block else o)(inner(self, *a, **k)))
+            assert torch.equal(logits(model), doubled)
+        hook = register_module_forward_hook(lambda mod, i, o: (o[0], o[1] * 2) if mod is block else None)
+        try:
+            assert torch.equal(logits(model), doubled)
+        finally:
+            hook.remove()
+    assert torch.equal(logits(model), plain)
+
+
+def test_an_overridden_head_is_heard(dev):
+    from diff_gpt.model import gpt
+
+    class Halved(gpt.GPT):
+        def _head(self, partial, argmax_out, xn=None):
+            return super()._head(partial, argmax_out, xn) * 0.5
+
+    torch.manual_seed(0)
+    model = gpt.GPT(vocab_size=128, n_embd=64, block_size=32, n_head=4, n_layer=2).eval().to(dev)
+    idx = torch.randint(0, 128, (3, 17), generator=torch.Generator().manual_seed(4)).to(dev)
+    with torch.inference_mode():
+        full = model(idx)[0]
+        model.__class__ = Halved
+        assert torch.equal(model(idx)[0], full * 0.5)
+
+
+def test_a_captured_step_of_an_overridden_model(dev):
+    """A forward put into the model's instance, of the arguments GPT.forward took
+    before the head's launch could advance the position, is captured as it is."""
+    from diff_gpt.model import gpt
+    from diff_gpt.model.engine import Engine
+    from diff_gpt.sampler.temperature import TemperatureSampler
+
+    torch.manual_seed(0)
+    model = gpt.GPT(vocab_size=128, n_embd=64, block_size=32, n_head=4, n_layer=2).eval().to(dev)
+    inner = model.forward
+
+    def forward(idx, targets=None, kv_cache=None, *, _argmax_out=None, _last_only=False):
+        logits, loss = inner(idx, targets, kv_cache, _argmax_out=_argmax_out, _last_only=_last_only)
+        return -logits, loss
+
+    def tokens(use_graph):
+        return Engine(model, use_graph=use_graph).generate_batch([1, 2, 3], num_samples=4, max_tokens=6,
+                                                                 sampler=TemperatureSampler(0.0))
+
+    plain = tokens(True)
+    model.forward = forward
+    assert tokens(True) == tokens(False) != plain
 
 
 def test_head_advances_the_position(dev):
