@@ -29,6 +29,7 @@ ATTN_RES_MAX_SOURCES = 32
 ATTN_RES_MAX_WIDTH = 2048
 # the widths dg_block_in and dg_block_out take
 LAYER_WIDTHS = (64, 128)
+_LINEAR_FORWARD = nn.Linear.forward
 
 
 def _few_rows(x: torch.Tensor, w: torch.Tensor, tile: int) -> bool:
@@ -66,7 +67,7 @@ def as_written(m: nn.Module, cls: type, forward) -> bool:
 def _plain_linear(m: nn.Module) -> bool:
     """A Linear that nothing watches or replaces, whose product may be taken
     from its weight."""
-    return type(m) is nn.Linear and m.bias is None and not m._forward_hooks and not m._forward_pre_hooks
+    return as_written(m, nn.Linear, _LINEAR_FORWARD) and m.bias is None
 
 
 def block_attn_res(

@@ -81,3 +81,41 @@ def test_block_with_and_without(dev, layer_idx, monkeypatch):
     assert torch.equal(one.isfinite(), apart.isfinite())
     ok = apart.isfinite()
     assert (one[ok].double() - apart[ok].double()).abs().max() <= 2e-2 * apart[ok].double().abs().max()
+
+
+def test_a_replaced_output_projection_is_heard(dev, monkeypatch):
+    """c_proj with a forward of its own, in the instance or the class, or watched
+    by a hook on all modules, is called as it is with a hook of its own."""
+    from torch import nn
+    from torch.nn.modules.module import register_module_forward_hook
+
+    from diff_gpt.model.block import Block
+    from diff_gpt.model.rope import precompute_freqs_cis
+
+    torch.manual_seed(3)
+    blk = Block(512, 8, 1.702, 7.0, 0).eval().to(dev).to(torch.bfloat16)
+    x = torch.randn(33, 1, 512, device=dev).to(torch.bfloat16)
+    freqs = precompute_freqs_cis(64, 4, 10000.0).to(dev)[:1].view(1, 1, 1, 32, 2)
+    proj, inner = blk.sa.c_proj, nn.Linear.forward
+
+    @torch.inference_mode()
+    def out():
+        return blk((x,), x * 2, freqs, None)[1]
+
+    plain = out()
+    hook = proj.register_forward_hook(lambda m, i, o: o * 2)
+    ref = out()
+    hook.remove()
+    assert not torch.equal(ref, plain)
+    proj.forward = lambda y: inner(proj, y) * 2
+    assert torch.equal(out(), ref)
+    del proj.forward
+    with monkeypatch.context() as m:
+        m.setattr(nn.Linear, "forward", lambda self, y: inner(self, y) * (2 if self is proj else 1))
+        assert torch.equal(out(), ref)
+    hook = register_module_forward_hook(lambda m, i, o: o * 2 if m is proj else None)
+    try:
+        assert torch.equal(out(), ref)
+    finally:
+        hook.remove()
+    assert torch.equal(out(), plain)
