@@ -30,11 +30,14 @@ ATTN_RES_MAX_WIDTH = 2048
 # the widths dg_block_in and dg_block_out take
 LAYER_WIDTHS = (64, 128)
 _LINEAR_FORWARD = nn.Linear.forward
+_PLAIN_TENSORS = (torch.Tensor, nn.Parameter)
 
 
-def _few_rows(x: torch.Tensor, w: torch.Tensor, tile: int) -> bool:
-    """Whether F.linear(x, w) and the elementwise work around it go to
-    dg_linear_rows: 16-bit products whose workgroups, of 32 rows and ``tile``
+def _few_rows(x: torch.Tensor, w: torch.Tensor, tile: int, *others: torch.Tensor | None) -> bool:
+    """Whether F.linear(x, w) and the elementwise work around it, with the tensors
+    ``others``, go to dg_linear_rows: where F.linear would be the plain product --
+    autograd records nothing, autocast changes no type, the weight has no class of
+    its own that would answer for it -- and for 16-bit products whose workgroups, of 32 rows and ``tile``
     features, times K stay within 256 x 1024, K at most 1024 (512 for the FFN's
     first product).  Beyond, its tiles read the operands too often.  us, the
     separate launches -> one, bf16:
@@ -49,8 +52,10 @@ def _few_rows(x: torch.Tensor, w: torch.Tensor, tile: int) -> bool:
     N, K = w.shape
     if K > 1024 or K % 512:
         return False
-    if torch.is_grad_enabled() and w.requires_grad:
-        return False  # F.linear records its product
+    if type(w) not in _PLAIN_TENSORS or torch.is_autocast_enabled("cuda"):
+        return False
+    if torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in (x, w, *others)):
+        return False
     return (x.numel() // K + 31) // 32 * (N // tile) * K <= 256 * 1024
 
 
@@ -177,7 +182,7 @@ class Block(nn.Module):
                                   out, _xn_out, tail=_tail):
                 return blocks, out
         joined = None
-        if not gated and _few_rows(y, sa.c_proj.weight, 32) and _plain_linear(sa.c_proj):
+        if not gated and _few_rows(y, sa.c_proj.weight, 32, g, partial_in) and _plain_linear(sa.c_proj):
             # the gate, c_proj and the partial sum in one launch
             joined = torch.empty_like(partial_in)
             if not _native.linear_rows_(y, sa.c_proj.weight, joined, gate=g,
@@ -226,7 +231,7 @@ class Block(nn.Module):
                 hidden = None
         if hidden is None:
             hidden = _native.ops().swiglu(F.linear(xn, up.weight), swiglu.alpha, swiglu.limit)
-        if _few_rows(hidden, down.weight, 32):
+        if _few_rows(hidden, down.weight, 32, partial_block):
             out = torch.empty_like(partial_block)
             if _native.linear_rows_(hidden, down.weight, out, residual=partial_block):
                 return out

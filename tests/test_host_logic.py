@@ -239,3 +239,31 @@ def test_ordinal_soft_ce_against_float64_loop():
     plain = torch.nn.functional.cross_entropy(logits[keep], targets[keep]).item()
     assert abs(_ordinal_soft_ce(logits, targets, 1e-3).item() - plain) <= 1e-9
     assert _ordinal_soft_ce(logits, torch.full((40,), -100), 1.0).item() == 0.0
+
+
+def test_few_rows_leaves_what_f_linear_would_treat():
+    """A product goes to dg_linear_rows only where F.linear would neither record
+    it, nor change its type, nor hand it to a tensor class of the weight's own."""
+    from diff_gpt.model.block import _few_rows
+
+    class Weight(torch.Tensor):
+        pass
+
+    r = lambda *s: torch.zeros(*s, dtype=torch.bfloat16)  # noqa: E731
+    x, w, res = r(33, 1, 512), r(512, 512), r(33, 1, 512)
+    assert _few_rows(x, w, 32) and _few_rows(x, torch.nn.Parameter(w, requires_grad=False), 32, None, res)
+    assert not _few_rows(x, w.as_subclass(Weight), 32)
+    for i in range(3):
+        ts = [x, w, res]
+        ts[i] = ts[i].clone().requires_grad_()
+        assert not _few_rows(ts[0], ts[1], 32, ts[2])
+        with torch.no_grad():
+            assert _few_rows(ts[0], ts[1], 32, ts[2])
+    torch.set_autocast_enabled("cuda", True)  # torch.autocast itself asks for a device
+    try:
+        assert not _few_rows(x, w, 32)
+    finally:
+        torch.set_autocast_enabled("cuda", False)
+    # the type, the contraction and the number of rows
+    assert not _few_rows(x.float(), w.float(), 32) and not _few_rows(r(4, 768), r(512, 768), 32)
+    assert _few_rows(r(512, 512), w, 32) and not _few_rows(r(1056, 512), w, 32)
