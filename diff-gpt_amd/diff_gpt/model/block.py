@@ -33,6 +33,12 @@ _LINEAR_FORWARD = nn.Linear.forward
 _PLAIN_TENSORS = (torch.Tensor, nn.Parameter)
 
 
+def _empty_rows(x: torch.Tensor) -> torch.Tensor:
+    """An output shaped as x whose rows follow each other; empty_like would keep
+    the order of a permuted x's dimensions."""
+    return torch.empty(x.shape, dtype=x.dtype, device=x.device)
+
+
 def _few_rows(x: torch.Tensor, w: torch.Tensor, tile: int, *others: torch.Tensor | None) -> bool:
     """Whether F.linear(x, w) and the elementwise work around it, with the tensors
     ``others``, go to dg_linear_rows: where F.linear would be the plain product --
@@ -176,7 +182,7 @@ class Block(nn.Module):
         if not gated and sa.n_embd in LAYER_WIDTHS and len(blocks) + 1 <= ATTN_RES_MAX_SOURCES:
             # gate, c_proj, the partial sum, the MLP's mixture and norm, the FFN
             # and the residual in one launch (n_embd 64 or 128)
-            out = torch.empty_like(partial_in)
+            out = _empty_rows(partial_in)
             if _native.block_out_(y, g, sa.c_proj.weight, None if committed else partial_in, list(blocks),
                                   self.mlp_res_proj.weight, up.weight, down.weight, swiglu.alpha, swiglu.limit,
                                   out, _xn_out, tail=_tail):
@@ -184,7 +190,7 @@ class Block(nn.Module):
         joined = None
         if not gated and _few_rows(y, sa.c_proj.weight, 32, g, partial_in) and _plain_linear(sa.c_proj):
             # the gate, c_proj and the partial sum in one launch
-            joined = torch.empty_like(partial_in)
+            joined = _empty_rows(partial_in)
             if not _native.linear_rows_(y, sa.c_proj.weight, joined, gate=g,
                                         residual=None if committed else partial_in):
                 joined = None
@@ -232,7 +238,7 @@ class Block(nn.Module):
         if hidden is None:
             hidden = _native.ops().swiglu(F.linear(xn, up.weight), swiglu.alpha, swiglu.limit)
         if _few_rows(hidden, down.weight, 32, partial_block):
-            out = torch.empty_like(partial_block)
+            out = _empty_rows(partial_block)
             if _native.linear_rows_(hidden, down.weight, out, residual=partial_block):
                 return out
         return partial_block + F.linear(hidden, down.weight)

@@ -119,3 +119,24 @@ def test_a_replaced_output_projection_is_heard(dev, monkeypatch):
     finally:
         hook.remove()
     assert torch.equal(out(), plain)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("n_embd,n_head", [(64, 4), (128, 4), (512, 8), (1024, 8)])
+@pytest.mark.parametrize("layer_idx", [0, 1])
+def test_block_takes_permuted_inputs(dev, dtype, n_embd, n_head, layer_idx):
+    """Committed blocks and a partial sum whose dimensions lie in another order
+    than (B, T, C), at few rows and at many: the contiguous copies' result."""
+    from diff_gpt.model.block import Block
+    from diff_gpt.model.rope import precompute_freqs_cis
+
+    torch.manual_seed(3)
+    dt = {"f32": torch.float32, **TDT}[dtype]
+    blk = Block(n_embd, n_head, 1.702, 7.0, layer_idx, layers_per_block=2).eval().to(dev).to(dt)
+    for B, T in ((3, 5), (16, 100)):
+        freqs = precompute_freqs_cis(n_embd // n_head, T, 10000.0).to(dev).view(1, T, 1, -1, 2)
+        first, partial = (torch.randn(T, B, n_embd, device=dev).to(dt).transpose(0, 1) for _ in range(2))
+        with torch.inference_mode():
+            got = blk((first,), partial, freqs, None)[1]
+            ref = blk((first.contiguous(),), partial.contiguous(), freqs, None)[1]
+        assert torch.equal(got, ref)
