@@ -795,17 +795,28 @@ def block_in_(sources: list[torch.Tensor], w_mix: torch.Tensor | None, w_qkvg: t
     return True
 
 
+# vocabularies of the head behind a layer (dg_block_out_head)
+TAIL_VOCABS = (64, 128, 256, 512, 1024)
+
+
+def takes_tail(dtype: torch.dtype, C: int) -> bool:
+    """Whether dg_block_out goes on with what follows the layer at this type and
+    width (fp32 at n_embd 128 never does)."""
+    return dtype in (torch.bfloat16, torch.float16) and C in (64, 128) or dtype == torch.float32 and C == 64
+
+
 class Tail:
     """What follows a layer over the same rows and can go with its launch: the
     next layer's projections (w_mix its pseudo-query, w (4C, C), out (..., 4C))
     or, with w_mix None, the head (w (V, C) the embedding table, out (..., V)
     the logits, cap, ids the int64 argmax of each row or None, advance an int32
-    device position to move on by one or None).  done: a launch has written out
-    (and ids, and advance)."""
+    device position to move on by one or None).  out None: allocated for the
+    launch, and None again if it does not take the tail.  done: a launch has
+    written out (and ids, and advance)."""
 
     __slots__ = ("w_mix", "w", "out", "cap", "ids", "advance", "done")
 
-    def __init__(self, w_mix: torch.Tensor | None, w: torch.Tensor, out: torch.Tensor, cap: float = 0.0,
+    def __init__(self, w_mix: torch.Tensor | None, w: torch.Tensor, out: torch.Tensor | None = None, cap: float = 0.0,
                  ids: torch.Tensor | None = None, advance: torch.Tensor | None = None) -> None:
         self.w_mix, self.w, self.out, self.cap, self.ids, self.advance = w_mix, w, out, cap, ids, advance
         self.done = False
@@ -843,7 +854,10 @@ def block_out_(y: torch.Tensor, g: torch.Tensor, w_proj: torch.Tensor, partial_i
     ]
     if tail is not None and tail.w.dtype == out.dtype and tail.w.stride(1) == 1 and tail.w.size(1) == C:
         n = tail.w.size(0)
-        t2 = tail.out.view(-1, n)
+        t_out = tail.out
+        if t_out is None:
+            t_out = torch.empty((*out.shape[:-1], n), dtype=out.dtype, device=out.device)
+        t2 = t_out.view(-1, n)
         if t2.size(0) != o2.size(0) or t2.dtype != out.dtype or (tail.w_mix is not None and n != 4 * C):
             raise ValueError("block_out: inconsistent shapes after the layer")
         if tail.ids is not None and (tail.ids.dtype != torch.int64 or tail.ids.numel() != o2.size(0)
@@ -859,8 +873,9 @@ def block_out_(y: torch.Tensor, g: torch.Tensor, w_proj: torch.Tensor, partial_i
             rc = DG_EUNSUPPORTED  # the next layer's projections and the norm are not written together
         if rc != DG_EUNSUPPORTED:
             _check(rc, "block_out")
-            tail.done = True
+            tail.out, tail.done = t_out, True
             return True
+        del t_out, t2
     if x2 is None:
         rc = lib().dg_block_out(*args, _stream(o2))
     else:

@@ -210,19 +210,18 @@ class GPT(BaseGPT):
             return False
         return all(plain_block(b) for b in self.blocks)
 
-    def _tail(self, i: int, partial: torch.Tensor, rows: tuple[int, int], ids: torch.Tensor | None,
-              advance: torch.Tensor | None) -> _native.Tail | None:
-        """What follows layer i over its (B, T) rows: layer i + 1's projections
-        or the head (not an overridden one)."""
-        alloc = lambda n: torch.empty((*rows, n), dtype=partial.dtype, device=partial.device)  # noqa: E731
+    def _tail(self, i: int, ids: torch.Tensor | None, advance: torch.Tensor | None) -> _native.Tail | None:
+        """What follows layer i: layer i + 1's projections or the head (not an
+        overridden one).  None where no launch would take it."""
+        w = self.lm_head.weight
+        if not _native.takes_tail(w.dtype, w.size(1)):
+            return None
         if i + 1 < len(self.blocks):
             block = self.blocks[i + 1]
-            w = block.sa._projection_weight()
-            return _native.Tail(block.attn_res_proj.weight, w, alloc(w.size(0)))
-        if type(self)._head is not _GPT_HEAD or "_head" in self.__dict__:
+            return _native.Tail(block.attn_res_proj.weight, block.sa._projection_weight())
+        if w.size(0) not in _native.TAIL_VOCABS or type(self)._head is not _GPT_HEAD or "_head" in self.__dict__:
             return None
-        w = self.lm_head.weight
-        return _native.Tail(None, w, alloc(w.size(0)), float(self.logit_softcap), ids, advance)
+        return _native.Tail(None, w, None, float(self.logit_softcap), ids, advance)
 
     def forward(
         self,
@@ -271,8 +270,7 @@ class GPT(BaseGPT):
         tail = None
         for i, block in enumerate(self.blocks):
             one = _last_only and i == last
-            rows = (B, 1 if one else T)
-            tail = self._tail(i, x, rows, _argmax_out, advance) if (joins_last if one else joins) else None
+            tail = self._tail(i, _argmax_out, advance) if (joins_last if one else joins) else None
             # a Block with a forward of its own is not handed what joined launches pass on
             joined = {} if qkvg is None and tail is None else {"_qkvg": qkvg, "_tail": tail}
             blocks, partial = block(blocks, partial, freqs_cis=freqs_cis, kv_cache=kv_cache,

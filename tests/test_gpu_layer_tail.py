@@ -216,6 +216,32 @@ def test_an_overridden_layer_is_heard(dev, embd, layer, monkeypatch):
     assert torch.equal(logits(model), plain)
 
 
+@pytest.mark.parametrize("vocab", [1536, 1024])
+def test_logits_are_allocated_once(dev, vocab, monkeypatch):
+    """Peak memory of a forward with joined launches: no second (B, T, V) beside
+    the logits, whether the layer's launch takes the head or not."""
+    from diff_gpt.model import gpt
+
+    torch.manual_seed(0)
+    model = gpt.GPT(vocab_size=vocab, n_embd=64, block_size=64, n_head=4, n_layer=2).eval().to(dev)
+    idx = torch.randint(0, vocab, (256, 64), generator=torch.Generator().manual_seed(4)).to(dev)
+    logits_bytes = idx.numel() * vocab * 4
+
+    @torch.inference_mode()
+    def peak():
+        model(idx)
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        model(idx)
+        torch.cuda.synchronize()
+        return torch.cuda.max_memory_allocated() - before
+
+    joined = peak()
+    monkeypatch.setattr(gpt.GPT, "_joins", lambda self, rows: False)
+    assert joined < peak() + logits_bytes // 2
+
+
 def test_an_overridden_head_is_heard(dev):
     from diff_gpt.model import gpt
 

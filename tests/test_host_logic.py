@@ -267,3 +267,17 @@ def test_few_rows_leaves_what_f_linear_would_treat():
     # the type, the contraction and the number of rows
     assert not _few_rows(x.float(), w.float(), 32) and not _few_rows(r(4, 768), r(512, 768), 32)
     assert _few_rows(r(512, 512), w, 32) and not _few_rows(r(1056, 512), w, 32)
+
+
+@pytest.mark.parametrize("dtype,n_embd,vocab,layer,head", [
+    (torch.float32, 64, 256, True, True), (torch.float32, 64, 192, True, False), (torch.float32, 128, 256, False, False),
+    (torch.bfloat16, 128, 1024, True, True), (torch.float16, 128, 2048, True, False),
+    (torch.float64, 64, 256, False, False),
+])
+def test_tails_are_built_where_a_launch_takes_them(dtype, n_embd, vocab, layer, head):
+    """Nothing is prepared, and no buffer allocated, for what no launch takes: fp32
+    at n_embd 128, vocabularies that the head behind a layer does not have."""
+    m = GPT(vocab_size=vocab, n_embd=n_embd, block_size=16, n_head=4, n_layer=2).eval().to(dtype)
+    first, last = (m._tail(i, None, None) for i in range(2))
+    assert (first is not None) == layer and (last is not None) == head
+    assert all(t is None or t.out is None for t in (first, last))
