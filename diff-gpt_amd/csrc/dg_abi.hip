@@ -8,6 +8,7 @@
 namespace dg {
 
 static thread_local char g_err[512] = "";
+static thread_local const char* g_kernel = "";
 
 void set_error(const char* fmt, ...) {
   va_list ap;
@@ -22,6 +23,7 @@ int check_launch(const char* what) {
     set_error("%s: launch failed: %s", what, hipGetErrorString(e));
     return DG_ELAUNCH;
   }
+  g_kernel = what;
   return DG_OK;
 }
 
@@ -193,6 +195,8 @@ using namespace dg;
 extern "C" int dg_abi_version(void) { return DG_ABI_VERSION; }
 
 extern "C" const char* dg_last_error(void) { return g_err; }
+
+extern "C" const char* dg_last_kernel(void) { return g_kernel; }
 
 extern "C" size_t dg_attention_workspace_size(int B, int H, int Tq, int Tk, int D, int dtype) {
   // float64 runs on a kernel without key splits

@@ -77,6 +77,7 @@ _lib: ctypes.CDLL | None = None
 _SIGNATURES = {
     "dg_abi_version": (ctypes.c_int, []),
     "dg_last_error": (ctypes.c_char_p, []),
+    "dg_last_kernel": (ctypes.c_char_p, []),
     "dg_rope_qknorm_append": (
         ctypes.c_int,
         [ctypes.c_int] * 5
@@ -285,6 +286,11 @@ def _check(rc: int, what: str) -> None:
     if rc != 0:
         msg = lib().dg_last_error().decode(errors="replace")
         raise RuntimeError(f"dgattn.{what} failed (status {rc}): {msg}")
+
+
+def last_kernel() -> str:
+    """The kernel that this thread's last launch through the library ran."""
+    return lib().dg_last_kernel().decode()
 
 
 def _dtype_code(t: torch.Tensor) -> int:

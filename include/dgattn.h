@@ -86,6 +86,10 @@ DG_API int dg_abi_version(void);
 /* Message of the last failed call on this thread ("" if none). */
 DG_API const char* dg_last_error(void);
 
+/* Name of the kernel that this thread's last successful launch ran ("" before
+ * the first): which side of a dispatch rule a call took. */
+DG_API const char* dg_last_kernel(void);
+
 /*
  * Fused RoPE + QK-norm + KV append.  Replaces mha.py:44-56: apply_rotary_emb on
  * q and k (rope.py:4-27), rms_norm on both (rms_norm.py:5-7, eps = FLT_EPSILON,

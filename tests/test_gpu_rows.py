@@ -13,11 +13,11 @@ TDT = {"f32": torch.float32, "bf16": torch.bfloat16, "f16": torch.float16}
 
 
 def _rows(M, C, dtype, dev, seed, offset, scale=3.0):
-    """(M, C) values that depend on the seed alone, rows ``offset`` elements off a
-    16-byte boundary (the row stride is a multiple of 16 bytes)."""
+    """(M, C) values that depend on the seed alone, rows ``offset`` elements off
+    their alignment (32 elements more a row keep a wide row's lanes aligned too)."""
     g = torch.Generator(device=dev).manual_seed(seed)
     x = (torch.randn(M, C, generator=g, device=dev) * scale).to(dtype)
-    wide = torch.zeros(M, C + 8, dtype=dtype, device=dev)
+    wide = torch.zeros(M, C + 32, dtype=dtype, device=dev)
     wide[:, offset : offset + C] = x
     return wide[:, offset : offset + C]
 
@@ -34,12 +34,16 @@ def test_gate_and_swiglu_vector_rows_equal_the_general_form(dev, dtype, M, C):
     got, ref = (_rows(M, C, dt, dev, 1, off) for off in (0, 1))
     ga, gb = (_rows(M, C, dt, dev, 2, off) for off in (0, 1))
     _native.gate_(got, ga)
+    assert _native.last_kernel() == "gate_vec_kernel"
     _native.gate_(ref, gb)
+    assert _native.last_kernel() == "gate_kernel"
     assert torch.equal(got, ref)
     xa, xb = (_rows(M, C, dt, dev, 3, off) for off in (0, 1))
     oa, ob = (torch.empty(M, C // 2, dtype=dt, device=dev) for _ in range(2))
     _native.swiglu_(xa, oa, 1.702, 7.0)
+    assert _native.last_kernel() == "swiglu_vec_kernel"
     _native.swiglu_(xb, ob, 1.702, 7.0)
+    assert _native.last_kernel() == "swiglu_kernel"
     assert torch.equal(oa, ob)
 
 
@@ -110,13 +114,18 @@ def test_mixture_forms_agree(dev, dtype, C, n):
         aligned[1], shifted[1] = aligned[0], shifted[0]
     copied = [s.clone() for s in aligned]  # no two are the same rows
     w = torch.randn(1, C, generator=torch.Generator(device=dev).manual_seed(9), device=dev).to(dt)
+    # rows that fill a wave (64 lanes of 16 bytes or more), at most 96 registers of sources
+    full = C * dt.itemsize >= 1024
+    wave = full and any(n <= s and C // 64 * dt.itemsize // 4 * s <= 96 for s in (4, 6, 8, 12))
     outs = []
-    for srcs in (aligned, shifted, copied):
+    for srcs, held in ((aligned, wave), (shifted, False), (copied, wave)):
         out = torch.empty(M, C, dtype=dt, device=dev)
         _native.attn_res_norm_(srcs, w, out)
+        assert _native.last_kernel() == ("attn_res_norm_wave_kernel" if held else "attn_res_norm_kernel")
         outs.append(out)
     few = torch.empty(33, C, dtype=dt, device=dev)
     _native.attn_res_norm_([s[:33] for s in aligned], w, few)
+    assert _native.last_kernel() == ("attn_res_norm_split_kernel" if full else "attn_res_norm_kernel")
     assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
     assert torch.equal(outs[0][:33], few)
 

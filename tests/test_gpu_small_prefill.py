@@ -39,6 +39,7 @@ def test_small_prefill_matches_float64(dev, dtype, D, B, H, Tq, Tk):
     q, k, v = _case(dev, B, H, Tq, Tk, D, TDT[dtype], seed=Tq + D)
     y = torch.empty(B, Tq, H, D, dtype=TDT[dtype], device=dev)
     _native.attention_(q, k, v, y, D**-0.5)
+    assert _native.last_kernel() == "prefill_small_kernel"
     ref = _attend64(q, k, v)
     assert bool(((y.double() - ref).abs() <= HALF[dtype] * ref.abs() + 2e-6 * ref.abs().max()).all())
 
@@ -54,6 +55,7 @@ def test_small_prefill_large_scores_rescale(dev, D):
     k = k * torch.linspace(0.2, 3.0, 200, device=dev).view(1, 200, 1, 1)
     y = torch.empty(1, 200, 2, D, device=dev)
     _native.attention_(q, k, v, y, D**-0.5)
+    assert _native.last_kernel() == "prefill_small_kernel"
     ref = _attend64(q, k, v)
     assert bool(((y.double() - ref).abs() <= 2 * 6e-4 * ref.abs().max()).all())
 
@@ -76,6 +78,7 @@ def test_small_prefill_keeps_hidden_rows_out(dev, dtype, D, bad):
     v2 = v.clone()
     v2[:, j, :, 3] = bad
     _native.attention_(q, k, v2, y1, D**-0.5)
+    assert _native.last_kernel() == "prefill_small_kernel"
 
     def close(a, b):
         a, b = a.double(), b.double()

@@ -20,9 +20,10 @@ CASES = [  # (rows, group, H, prefix, cached own keys, spare capacity)
     (160, 16, 8, 513, 100, 30),
     (66, 33, 5, 1031, 7, 5),
     (20, 32, 16, 1100, 40, 2),  # fewer rows than a group
-    (20, 32, 16, 1068, 40, 2),  # the first prefix below the line: the two launches
+    (20, 32, 16, 1068, 40, 2),  # the first prefix below the line: the vector kernel
     (17, 17, 1, 63, 1, 3),
 ]
+VECTOR_CASES = CASES[-2:]
 
 
 def _case(dev, dtype, D, case, seed=0):
@@ -71,6 +72,7 @@ def test_wide_step(dev, dtype, D, case, f32_table):
         table = table.to(TDT[dtype])
     before = rows.clone()
     y = _step(pages, rows, qkv, table, pos, case)
+    assert (_native.last_kernel() == "attn_wide_kernel") == (case not in VECTOR_CASES)
     q_rot, k_rot = (torch.empty(B, 1, H, D, dtype=TDT[dtype], device=dev) for _ in range(2))
     _native.rope_qknorm_append_(qkv[0], qkv[1], None, table[pos].view(1, 1, 1, D // 2, 2), q_rot, k_rot, None, True)
     assert torch.equal(rows[0, :, :, own], k_rot[:, 0]) and torch.equal(rows[1, :, :, own], qkv[2][:, 0])
@@ -85,6 +87,7 @@ def test_wide_step(dev, dtype, D, case, f32_table):
 
     rows2 = before.clone()
     assert torch.equal(_step(pages, rows2, qkv, table, pos, case, device_pos=True), y)
+    assert (_native.last_kernel() == "attn_wide_kernel") == (case not in VECTOR_CASES)
     assert torch.equal(rows2.nan_to_num(5.0), rows.nan_to_num(5.0))
     # the prefix in every row instead of pages of its own
     dense = torch.cat((pages[:, group], before), dim=3)
@@ -118,6 +121,7 @@ def test_wide_step_values_not_finite(dev, dtype, D):
                             (0, 5, 0, 0, inf), (0, 5, 64, 0, inf)]:
         pages[1, grp, h, t, d] = x
     y = _step(pages, rows, qkv, table, pos, case)
+    assert _native.last_kernel() == "attn_wide_kernel"
     q_rot, k_rot = (torch.empty(B, 1, H, D, dtype=TDT[dtype], device=dev) for _ in range(2))
     _native.rope_qknorm_append_(qkv[0], qkv[1], None, table[pos].view(1, 1, 1, D // 2, 2), q_rot, k_rot, None, True)
     group = torch.arange(B, device=dev) // G
@@ -145,6 +149,7 @@ def test_wide_step_large_scores(dev):
     pre = _native.Prefix(700, 40, pages[0].transpose(1, 2), pages[1].transpose(1, 2), 700)
     _native.decode_step_(*qkv, table[pos], rows[0].transpose(1, 2), rows[1].transpose(1, 2), y, D**-0.5, pos,
                          qknorm=False, prefix=pre)
+    assert _native.last_kernel() == "attn_wide_kernel"
     q_rot = torch.empty_like(y)
     _native.rope_qknorm_append_(qkv[0], None, None, table[pos].view(1, 1, 1, D // 2, 2), q_rot, None, None, False)
     keys, vals = (torch.cat((pages[i].expand(40, -1, -1, -1), rows[i][:, :, :21]), dim=2).double() for i in (0, 1))
