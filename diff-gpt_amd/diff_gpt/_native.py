@@ -843,7 +843,9 @@ def block_out_(y: torch.Tensor, g: torch.Tensor, w_proj: torch.Tensor, partial_i
     C = out.size(-1)
     y2, g2, o2 = _rows(y, "block_out"), _rows(g, "block_out"), out.view(-1, C)
     p2 = None if partial_in is None else _rows(partial_in, "block_out")
-    _, ptrs, lds = _row_list(blocks, "block_out")
+    rows, ptrs, lds = _row_list(blocks, "block_out")
+    # copies made here live until the launch is on the stream
+    mix = w_mix.reshape(-1).contiguous()
     ws = (w_proj, w_up, w_down)
     if any(t.stride(1) != 1 or t.dtype != out.dtype for t in ws) or o2.stride(1) != 1:
         return False
@@ -855,7 +857,7 @@ def block_out_(y: torch.Tensor, g: torch.Tensor, w_proj: torch.Tensor, partial_i
     args = [
         o2.size(0), C, _dtype_code(o2), _ptr(y2), y2.stride(0), _ptr(g2), g2.stride(0), _ptr(w_proj),
         w_proj.stride(0), _ptr(p2), 0 if p2 is None else p2.stride(0), len(blocks), ptrs, lds,
-        _ptr(w_mix.reshape(-1).contiguous()), _ptr(w_up), w_up.stride(0), _ptr(w_down), w_down.stride(0),
+        _ptr(mix), _ptr(w_up), w_up.stride(0), _ptr(w_down), w_down.stride(0),
         float(alpha), float(limit), _ptr(o2), o2.stride(0),
     ]
     if tail is not None and tail.w.dtype == out.dtype and tail.w.stride(1) == 1 and tail.w.size(1) == C:
@@ -873,8 +875,8 @@ def block_out_(y: torch.Tensor, g: torch.Tensor, w_proj: torch.Tensor, partial_i
             rc = lib().dg_block_out_head(*args, _ptr(x2), C, n, _ptr(tail.w), tail.w.stride(0), float(tail.cap),
                                          _ptr(t2), n, _ptr(tail.ids), _ptr(tail.advance), _stream(o2))
         elif x2 is None:
-            rc = lib().dg_block_out_in(*args, _ptr(tail.w_mix.reshape(-1).contiguous()), _ptr(tail.w),
-                                       tail.w.stride(0), _ptr(t2), n, _stream(o2))
+            t_mix = tail.w_mix.reshape(-1).contiguous()
+            rc = lib().dg_block_out_in(*args, _ptr(t_mix), _ptr(tail.w), tail.w.stride(0), _ptr(t2), n, _stream(o2))
         else:
             rc = DG_EUNSUPPORTED  # the next layer's projections and the norm are not written together
         if rc != DG_EUNSUPPORTED:

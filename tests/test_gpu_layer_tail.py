@@ -66,6 +66,26 @@ def test_block_out_with_what_follows(dev, dtype, C, M, nblk, pin):
         assert torch.equal(plain.out, logits)
 
 
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_pseudo_queries_with_a_stride(dev, dtype):
+    """Pseudo-queries that are columns of another tensor are copied for the launch,
+    each into memory of its own."""
+    from diff_gpt import _native
+
+    C, dt = 64, TDT[dtype]
+    y, g, _, blocks, w = _layer(20, C, 3, dt, dev)
+    mixes = [_rand(i, dev, dt, 1, C, scale=4 * C**-0.5) for i in (11, 12)]
+    wq = _rand(9, dev, dt, 4 * C, C, scale=C**-0.5)
+    results = []
+    for strided in (False, True):
+        mix, t_mix = (_rand(1, dev, dt, C, 3).copy_(m.view(C, 1).expand(C, 3))[:, 1:2].T if strided else m for m in mixes)
+        assert mix.is_contiguous() != strided
+        out, tail = torch.empty(20, C, dtype=dt, device=dev), _native.Tail(t_mix, wq)
+        assert _native.block_out_(y, g, w["proj"], None, blocks, mix, w["up"], w["down"], 1.702, 7.0, out, tail=tail)
+        results.append((out, tail.out))
+    assert all(torch.equal(a, b) for a, b in zip(*results))
+
+
 def test_block_out_leaves_other_tails_undone(dev):
     """A vocabulary that the head does not take, a table without unit stride,
     fp32 at n_embd 128: the layer alone."""
