@@ -760,6 +760,8 @@ def attn_res_norm_(sources: list[torch.Tensor], w: torch.Tensor, out: torch.Tens
             raise ValueError("attn_res_norm: sources must share shape and dtype with the output")
     o2 = out.view(-1, C)
     w1 = w.reshape(-1).contiguous()
+    if w1.dtype != out.dtype or w1.numel() != C:
+        raise ValueError("attn_res_norm: the pseudo-query must have C elements of the output's dtype")
     ptrs = (ctypes.c_void_p * n)(*[t.data_ptr() for t in srcs])
     lds = (ctypes.c_int64 * n)(*[t.stride(0) for t in srcs])
     rc = lib().dg_attn_res_norm(
@@ -791,6 +793,8 @@ def block_in_(sources: list[torch.Tensor], w_mix: torch.Tensor | None, w_qkvg: t
     if w_qkvg.dtype != out.dtype or w_qkvg.shape != (4 * C, C) or w_qkvg.stride(1) != 1:
         return False
     w1 = None if w_mix is None else w_mix.reshape(-1).contiguous()
+    if w1 is not None and (w1.dtype != out.dtype or w1.numel() != C):
+        return False
     rc = lib().dg_block_in(
         o2.size(0), C, _dtype_code(o2), len(rows), ptrs, lds, _ptr(w1), _ptr(w_qkvg), w_qkvg.stride(0), _ptr(o2),
         o2.stride(0), _stream(o2),
@@ -828,6 +832,11 @@ class Tail:
         self.done = False
 
 
+def _tail_fits(tail: Tail, out: torch.Tensor) -> bool:
+    mix = tail.w_mix
+    return tail.w.dtype == out.dtype and (mix is None or (mix.dtype == out.dtype and mix.numel() == out.size(-1)))
+
+
 def block_out_(y: torch.Tensor, g: torch.Tensor, w_proj: torch.Tensor, partial_in: torch.Tensor | None,
                blocks: list[torch.Tensor], w_mix: torch.Tensor, w_up: torch.Tensor, w_down: torch.Tensor,
                alpha: float, limit: float, out: torch.Tensor, xn_out: torch.Tensor | None = None,
@@ -849,6 +858,8 @@ def block_out_(y: torch.Tensor, g: torch.Tensor, w_proj: torch.Tensor, partial_i
     ws = (w_proj, w_up, w_down)
     if any(t.stride(1) != 1 or t.dtype != out.dtype for t in ws) or o2.stride(1) != 1:
         return False
+    if any(t is not None and t.dtype != out.dtype for t in (y2, g2, p2, mix, *rows)) or mix.numel() != C:
+        return False  # the kernel reads every operand as out's type
     x2 = None
     if xn_out is not None:
         if xn_out.dtype != out.dtype or xn_out.shape != out.shape or not xn_out.is_contiguous():
@@ -860,7 +871,7 @@ def block_out_(y: torch.Tensor, g: torch.Tensor, w_proj: torch.Tensor, partial_i
         _ptr(mix), _ptr(w_up), w_up.stride(0), _ptr(w_down), w_down.stride(0),
         float(alpha), float(limit), _ptr(o2), o2.stride(0),
     ]
-    if tail is not None and tail.w.dtype == out.dtype and tail.w.stride(1) == 1 and tail.w.size(1) == C:
+    if tail is not None and _tail_fits(tail, out) and tail.w.stride(1) == 1 and tail.w.size(1) == C:
         n = tail.w.size(0)
         t_out = tail.out
         if t_out is None:

@@ -281,3 +281,26 @@ def test_tails_are_built_where_a_launch_takes_them(dtype, n_embd, vocab, layer, 
     first, last = (m._tail(i, None, None) for i in range(2))
     assert (first is not None) == layer and (last is not None) == head
     assert all(t is None or t.out is None for t in (first, last))
+
+
+def test_layer_launches_decline_mixed_types():
+    """Operands of another type than the output's (a bf16 attention output under
+    autocast around fp32 weights) are declined before any launch: the kernels read
+    every operand as the output's type."""
+    from diff_gpt import _native
+
+    C, r = 64, lambda *s: torch.zeros(*s)  # noqa: E731
+    y, g, pin, blk, mix, out = r(4, C), r(4, C), r(4, C), r(4, C), r(1, C), r(4, C)
+    for bad in range(5):
+        ts = [t.bfloat16() if i == bad else t for i, t in enumerate((y, g, pin, blk, mix))]
+        assert not _native.block_out_(ts[0], ts[1], r(C, C), ts[2], [ts[3]], ts[4], r(4 * C, C), r(C, 2 * C), 1.702, 7.0,
+                                      out)
+    assert not _native.block_out_(y, g, r(C, C), pin, [blk], r(1, C // 2), r(4 * C, C), r(C, 2 * C), 1.702, 7.0, out)
+    for mix in (r(1, C).bfloat16(), r(1, C // 2)):
+        assert not _native.block_in_([blk, blk], mix, r(4 * C, C), r(4, 4 * C))
+        with pytest.raises(ValueError, match="pseudo-query"):
+            _native.attn_res_norm_([blk, blk], mix, out)
+        assert not _native._tail_fits(_native.Tail(mix, r(4 * C, C)), out)
+    assert not _native.block_in_([blk.bfloat16(), blk], r(1, C), r(4 * C, C), r(4, 4 * C))
+    assert _native._tail_fits(_native.Tail(r(1, C), r(4 * C, C)), out)
+    assert _native._tail_fits(_native.Tail(None, r(256, C)), out)
