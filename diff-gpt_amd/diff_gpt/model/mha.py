@@ -167,7 +167,7 @@ class MultiHeadAttention(nn.Module):
         """mha.py:44-83 on the projections qkvg (B, T, 3*inner + C), whose
         column slices are q, k, v and the gate logits: RoPE, QK-norm, the
         cache append and the attention; returns y (B, T, inner) before the
-        gate, or with gated after it (mha.py:84)."""
+        gate, or with gated (a prefill: _gates_in_prefill) after it (mha.py:84)."""
         B, T, _ = qkvg.size()
         H, D = self.n_head, self.head_dim
         ops = _native.ops()
@@ -177,10 +177,7 @@ class MultiHeadAttention(nn.Module):
         v = qkvg[..., 2 * inner : 3 * inner].view(B, T, H, D)
 
         if kv_cache is not None and T == 1:
-            y = self._decode_step(q, k, v, freqs_cis, kv_cache)
-            if gated:
-                ops.gate_(y, self._gate_logits(qkvg))
-            return y
+            return self._decode_step(q, k, v, freqs_cis, kv_cache)
         assert kv_cache is None or kv_cache.pos_dev is None, "a captured decode step takes one token per row"
         # Prefills the MFMA kernel takes rotate and normalise q as they load it
         # (dg_prefill_rope); the first launch then handles k and v only.
