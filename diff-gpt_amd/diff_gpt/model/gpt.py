@@ -20,14 +20,19 @@ from diff_gpt.model.rope import precompute_freqs_cis
 from diff_gpt.sampler.sampler import Sampler
 from diff_gpt.sampler.temperature import TemperatureSampler, draw_one
 
-# n_embd -> the most rows whose launches are joined (GPT._joins).  Three layers
-# over rows of one token, us one by one -> joined: n_embd 64 in bf16, 100 rows
-# 51.7 -> 43.9, 8192 120 -> 111, 16384 193 -> 194 (32-row groups need the
-# launches of their own); in fp32, which has no 32-row form, 100 rows 59.7 ->
-# 51.4, 35328 480 -> 473, so any number.  n_embd 128 in bf16: 4096 rows 110 ->
-# 100, 8192 166 -> 178; in fp32 the embedding's launch alone joins: 100 rows
-# 99.9 -> 98.1, 16384 427 -> 430.
-JOINED_ROWS = {64: 8192, 128: 4096}
+# (n_embd, bytes of an element) -> the most rows whose launches are joined
+# (GPT._joins).  Whole forwards over a vocabulary of 256, us one by one -> joined:
+#   n_embd  64 fp32  2 layers:   100 rows 43.4 -> 35.8, 35328 245 -> 236, 41400 274 -> 271, 70656 408 -> 417
+#                    6 layers:   100 rows  118 ->  109, 35328 666 -> 669, 41400 749 -> 785, 70656 1155 -> 1269
+#   n_embd  64 bf16  2 layers:   100 rows 37.7 -> 30.8, 8192 86.8 -> 77.3, 16384 142 -> 140
+#                    6 layers:   100 rows  102 -> 90.1, 8192 243 -> 226, 16384 390 -> 395 (70656 728 -> 752)
+#   n_embd 128 bf16  2 layers:   100 rows 49.7 -> 45.1, 4096 78.0 -> 70.0, 8192 119 -> 123
+#                    6 layers:   100 rows  138 ->  141, 4096 231 -> 206, 8192 332 -> 362
+#   n_embd 128 fp32 (the embedding's launch alone joins)  2 layers: 100 rows 70.9 -> 69.1, 8192 181 -> 176
+# Beyond the lines the launches of their own take 32-row groups, which joined
+# ones have no registers for.  A vocabulary of 1024 gains more (fp32, 2 layers,
+# 70656 rows: 566 -> 542), many layers less.
+JOINED_ROWS = {(64, 4): 36864, (64, 2): 8192, (128, 4): 4096, (128, 2): 4096}
 
 
 def _ordinal_target_table(V: int, sigma: float, dtype: torch.dtype, device) -> torch.Tensor:
@@ -206,7 +211,7 @@ class GPT(BaseGPT):
         as written, since an overridden forward or a hook may read or replace what
         lies between."""
         w = self.token_embedding_table.weight
-        if rows > JOINED_ROWS.get(w.size(1), 0) and not (w.size(1) == 64 and w.dtype == torch.float32):
+        if rows > JOINED_ROWS.get((w.size(1), w.element_size()), -1):
             return False
         return all(plain_block(b) for b in self.blocks)
 

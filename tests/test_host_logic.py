@@ -304,3 +304,12 @@ def test_layer_launches_decline_mixed_types():
     assert not _native.block_in_([blk.bfloat16(), blk], r(1, C), r(4 * C, C), r(4, 4 * C))
     assert _native._tail_fits(_native.Tail(r(1, C), r(4 * C, C)), out)
     assert _native._tail_fits(_native.Tail(None, r(256, C)), out)
+
+
+@pytest.mark.parametrize("dtype,n_embd,most", [
+    (torch.float32, 64, 36864), (torch.bfloat16, 64, 8192), (torch.float16, 64, 8192), (torch.float32, 128, 4096),
+    (torch.bfloat16, 128, 4096), (torch.float64, 64, -1), (torch.float32, 32, -1), (torch.bfloat16, 256, -1),
+])
+def test_launches_are_joined_up_to_a_number_of_rows(dtype, n_embd, most):
+    m = GPT(vocab_size=64, n_embd=n_embd, block_size=16, n_head=4, n_layer=2).eval().to(dtype)
+    assert all(m._joins(rows) == (rows <= most) for rows in (1, abs(most), abs(most) + 1, 1 << 20))
