@@ -265,9 +265,10 @@ class GPT(BaseGPT):
         blocks: tuple[torch.Tensor, ...] = (x,)
         partial = x
         last = len(self.blocks) - 1
-        # the head's input rms_norm(partial), written by the last layer unless its
-        # launch goes on with the head
+        # the head's input rms_norm(partial), written by the last layer
         xn_head = None
+        if self.blocks:
+            xn_head = torch.empty((B, 1 if _last_only else T, x.size(-1)), dtype=x.dtype, device=x.device)
         advance = kv_cache.pos_dev if _advance else None
         joins = self._joins(B * T)
         joins_last = self._joins(B) if _last_only else joins
@@ -275,8 +276,6 @@ class GPT(BaseGPT):
         for i, block in enumerate(self.blocks):
             one = _last_only and i == last
             tail = self._tail(i, _argmax_out, advance) if (joins_last if one else joins) else None
-            if i == last and tail is None:
-                xn_head = torch.empty((B, 1 if one else T, x.size(-1)), dtype=x.dtype, device=x.device)
             # a Block with a forward of its own is not handed what joined launches pass on
             joined = {} if qkvg is None and tail is None else {"_qkvg": qkvg, "_tail": tail}
             blocks, partial = block(blocks, partial, freqs_cis=freqs_cis, kv_cache=kv_cache,

@@ -236,25 +236,6 @@ def test_an_overridden_layer_is_heard(dev, embd, layer, monkeypatch):
     assert torch.equal(logits(model), plain)
 
 
-def test_a_joined_head_stores_no_norm(dev, monkeypatch):
-    """The norm of the last layer's rows goes to memory for a head's launch of its
-    own only."""
-    from diff_gpt import _native
-    from diff_gpt.model import gpt
-
-    torch.manual_seed(0)
-    idx = torch.randint(0, 128, (3, 17), generator=torch.Generator().manual_seed(4)).to(dev)
-    real, norms = _native.block_out_, []
-    monkeypatch.setattr(_native, "block_out_", lambda *a, **k: (norms.append(a[11] is not None), real(*a, **k))[1])
-    for vocab, stored in ((128, False), (192, True)):
-        model = gpt.GPT(vocab_size=vocab, n_embd=64, block_size=32, n_head=4, n_layer=2).eval().to(dev)
-        for last_only in (False, True):
-            norms.clear()
-            with torch.inference_mode():
-                model(idx, _last_only=last_only)
-            assert norms == [False, stored]
-
-
 @pytest.mark.parametrize("vocab", [1536, 1024])
 def test_logits_are_allocated_once(dev, vocab, monkeypatch):
     """Peak memory of a forward with joined launches: no second (B, T, V) beside
