@@ -821,15 +821,16 @@ class Tail:
     or, with w_mix None, the head (w (V, C) the embedding table, out (..., V)
     the logits, cap, ids the int64 argmax of each row or None, advance an int32
     device position to move on by one or None).  out None: allocated for the
-    launch, and None again if it does not take the tail.  done: a launch has
-    written out (and ids, and advance)."""
+    launch, and None again if it does not take the tail.  keep_norm False: with
+    the head in the launch, nobody reads block_out_'s xn_out, and it is left
+    unwritten.  done: a launch has written out (and ids, and advance)."""
 
-    __slots__ = ("w_mix", "w", "out", "cap", "ids", "advance", "done")
+    __slots__ = ("w_mix", "w", "out", "cap", "ids", "advance", "keep_norm", "done")
 
     def __init__(self, w_mix: torch.Tensor | None, w: torch.Tensor, out: torch.Tensor | None = None, cap: float = 0.0,
-                 ids: torch.Tensor | None = None, advance: torch.Tensor | None = None) -> None:
+                 ids: torch.Tensor | None = None, advance: torch.Tensor | None = None, keep_norm: bool = True) -> None:
         self.w_mix, self.w, self.out, self.cap, self.ids, self.advance = w_mix, w, out, cap, ids, advance
-        self.done = False
+        self.keep_norm, self.done = keep_norm, False
 
 
 def _tail_fits(tail: Tail, out: torch.Tensor) -> bool:
@@ -883,7 +884,7 @@ def block_out_(y: torch.Tensor, g: torch.Tensor, w_proj: torch.Tensor, partial_i
                                      or not tail.ids.is_contiguous()):
             raise ValueError("block_out: ids must be a contiguous int64 tensor of the rows")
         if tail.w_mix is None:
-            rc = lib().dg_block_out_head(*args, _ptr(x2), C, n, _ptr(tail.w), tail.w.stride(0), float(tail.cap),
+            rc = lib().dg_block_out_head(*args, _ptr(x2 if tail.keep_norm else None), C, n, _ptr(tail.w), tail.w.stride(0), float(tail.cap),
                                          _ptr(t2), n, _ptr(tail.ids), _ptr(tail.advance), _stream(o2))
         elif x2 is None:
             t_mix = tail.w_mix.reshape(-1).contiguous()

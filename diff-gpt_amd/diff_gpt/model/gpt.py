@@ -226,7 +226,7 @@ class GPT(BaseGPT):
             return _native.Tail(block.attn_res_proj.weight, block.sa._projection_weight())
         if w.size(0) not in _native.TAIL_VOCABS or type(self)._head is not _GPT_HEAD or "_head" in self.__dict__:
             return None
-        return _native.Tail(None, w, None, float(self.logit_softcap), ids, advance)
+        return _native.Tail(None, w, None, float(self.logit_softcap), ids, advance, keep_norm=False)
 
     def forward(
         self,

@@ -236,6 +236,28 @@ def test_an_overridden_layer_is_heard(dev, embd, layer, monkeypatch):
     assert torch.equal(logits(model), plain)
 
 
+def test_a_joined_head_stores_no_norm(dev, monkeypatch):
+    """With the head in the last layer's launch the norm of its rows goes nowhere;
+    a head of its own launch reads it from memory."""
+    from diff_gpt import _native
+    from diff_gpt.model import gpt
+
+    torch.manual_seed(0)
+    idx = torch.randint(0, 128, (3, 17), generator=torch.Generator().manual_seed(4)).to(dev)
+    lib, stored = _native.lib(), []
+    for name in ("dg_block_out_head", "dg_block_out_norm"):
+        real = getattr(lib, name)
+        xn = 23  # the argument after out and its row stride
+        monkeypatch.setattr(lib, name, lambda *a, real=real: (stored.append(a[xn].value is not None), real(*a))[1])
+    for vocab, norm in ((128, False), (192, True)):
+        model = gpt.GPT(vocab_size=vocab, n_embd=64, block_size=32, n_head=4, n_layer=2).eval().to(dev)
+        for last_only in (False, True):
+            stored.clear()
+            with torch.inference_mode():
+                model(idx, _last_only=last_only)
+            assert stored == [norm]
+
+
 @pytest.mark.parametrize("vocab", [1536, 1024])
 def test_logits_are_allocated_once(dev, vocab, monkeypatch):
     """Peak memory of a forward with joined launches: no second (B, T, V) beside
