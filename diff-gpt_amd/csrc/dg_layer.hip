@@ -22,13 +22,18 @@
 // everything else the kernel reads, before the first stage, and stay in
 // registers; at more rows than fill the chip a workgroup walks several groups
 // with the same fragments, the next group's rows in flight under the current
-// one's products.  Only fp32 at n_embd 128 fetches its FFN fragments as it goes
-// (256 registers would not hold them).
+// one's products.  fp32 at n_embd 128 fetches its FFN fragments as it goes (256
+// registers would not hold them).  Instances for more than four committed blocks
+// hold eight sources: after the attention some of them keep registers in scratch,
+// with 32-row groups up to 39 of a lane's, at n_embd 64 in fp32 with the next
+// layer's projections behind them up to 19.
 //
 // RT = 1 while every group of 16 has a workgroup of its own on the chip: the
 // launch is bound by latency (one round trip to memory, the stages' chain), and
 // half the waves sit out the row work.  RT = 2 beyond: all do, and the vector
-// ALU's share (row work and SwiGLU, more than the products' in fp32) halves.
+// ALU's share (row work and SwiGLU, more than the products' in fp32) halves --
+// but for the instances whose 32-row form loses by its scratch (both sides at
+// launch_block_out_ns).
 // Measured in captured graphs, us, 3 sources, two of them the same rows
 // (before: the mixture's launch and a library GEMM; 4 waves per 16 rows after
 // the attention):
@@ -723,12 +728,24 @@ void launch_block_in(const BlockInArgs& a, hipStream_t s) {
   else launch_block_in_ns<T, C, kMaxResSources>(a, s);
 }
 
-// fp32 at n_embd 64 keeps a workgroup per 16 rows at any size: its 32-row form
-// needs more than the 128 registers of two workgroups per CU (35328 rows: 54 us
-// with the spills, 52 with one workgroup per CU, 44 so).
+// At n_embd 64 two kinds of instances keep a workgroup per 16 rows at any size,
+// their 32-row forms needing more than the 128 registers of two workgroups per
+// CU: fp32 (35328 rows: 54 us with the spills, 52 with one workgroup per CU, 44
+// so), and 16-bit types for 5 to 8 blocks.  us after the attention, 16-row ->
+// 32-row groups:
+//                 blocks   8200 rows       16384          35328
+//   n_embd  64 bf16    3    9.6 ->  9.7   12.4 -> 11.3   22.0 -> 25.3
+//                      5   11.3 -> 13.1   15.3 -> 15.6   29.0 -> 33.8
+//                      8   11.9 -> 13.6   15.8 -> 16.4   30.4 -> 36.1
+//                      9   13.7 -> 15.8   18.1 -> 19.5   36.7 -> 41.8
+//                     16   20.4 -> 21.1   28.8 -> 25.9   60.3 -> 61.1
+//                     31   37.8 -> 33.6   51.2 -> 40.4    114 ->  104
+//   n_embd 128 bf16    5   22.9 -> 19.6   43.3 -> 30.0   96.1 -> 56.6
+//                     31   61.4 -> 44.2    107 -> 74.7    275 ->  196
+//   n_embd 128 fp32    5   40.0 -> 36.5   78.6 -> 66.5    170 ->  149
 template <typename T, int C, int NS>
 void launch_block_out_ns(const BlockOutArgs& a, hipStream_t s) {
-  constexpr bool kDeep = !(C == 64 && sizeof(T) == 4);
+  constexpr bool kDeep = !(C == 64 && (sizeof(T) == 4 || NS == 8));
   const bool deep = kDeep && layer_deep(a.M, C);
   const unsigned grid = layer_grid(a.M, deep, C);
   if constexpr (kDeep) {
