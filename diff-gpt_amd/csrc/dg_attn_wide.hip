@@ -205,6 +205,12 @@ __global__ __launch_bounds__(64 * kWideWaves, 4) void attn_wide_kernel(const Wid
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         if (t0 + u * KPH >= own1) continue;
+        if (t0 + (u + 1) * KPH > own1) {  // wave-uniform: some lanes hold the last key again
+          // its value weighs 0 there, and 0 times an infinity would be a NaN
+          const bool own = t0 + u * KPH + kg < own1;
+#pragma unroll
+          for (int w = 0; w < Row::WORDS; ++w) v[u].w[w] = own ? v[u].w[w] : 0u;
+        }
         const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[u], cl, -moff));
         l += p;
 #pragma unroll

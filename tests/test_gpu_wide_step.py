@@ -135,6 +135,35 @@ def test_wide_step_values_not_finite(dev, dtype, D):
     assert torch.equal(y[:, 0][finite], clean[:, 0][finite])
 
 
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("own", [1, 41, 43, 44])  # the last slot holds one key, some or all it can
+def test_wide_step_own_values_not_finite(dev, dtype, D, own):
+    """The same for the values of a row's own keys, the newest cached one and the
+    new one among them: the infinity or NaN reaches its row and column alone."""
+    from diff_gpt import _native
+
+    case = (400, 100, 8, 1024, own, 50)
+    B, G, H, P, _, _ = case
+    pages, rows, qkv, table, pos = _case(dev, dtype, D, case)
+    clean = _step(pages, rows.clone(), qkv, table, pos, case)
+    assert _native.last_kernel() == "attn_wide_kernel"
+    inf = float("inf")
+    hit = torch.full((B, H, D), 0.0, device=dev)
+    for b, h, t, d, x in [(0, 0, own - 1, 3, inf), (17, 3, own - 1, 5, -inf), (33, 7, 0, 9, inf), (399, 1, own - 1, D - 1, inf),
+                          (200, 2, own // 2, 4, float("nan")), (55, 6, own, 7, -inf)]:
+        if t < own:
+            rows[1, b, h, t, d] = x
+        else:
+            qkv[2][b, 0, h, d] = x
+        hit[b, h, d] = x
+    y = _step(pages, rows, qkv, table, pos, case)[:, 0].float()
+    kinds = lambda t: t.nan_to_num(7.0, 8.0, 9.0)  # noqa: E731
+    bad = ~hit.isfinite()
+    assert torch.equal(kinds(y[bad]), kinds(hit[bad]))
+    assert torch.equal(y[~bad], clean[:, 0].float()[~bad])
+
+
 def test_wide_step_large_scores(dev):
     """Queries and keys that are not normalised: scores of several hundred, the
     maximum raised chunk after chunk.  Their fp32 sums are off by up to some
