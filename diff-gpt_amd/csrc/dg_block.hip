@@ -529,7 +529,17 @@ int pow2_at_least(int x) {
   return p;
 }
 
-// rows up to which wide rows (G = 64) take attn_res_norm_split_kernel
+// Rows up to which wide rows (G = 64) take attn_res_norm_split_kernel.  The line
+// is the one against attn_res_norm_kernel, a row per wave with its sources one at
+// a time, which the split form leads up to some 4096 rows (512 rows of 512 in bf16,
+// 3 / 9 sources: 6.8 -> 5.3 / 10.2 -> 7.8 us).  attn_res_norm_wave_kernel, which takes
+// aligned rows beyond the line, is ahead of the split form below it as well, where
+// its registers hold every source; us, split -> wave, two of the sources the same:
+//   bf16  512, 3 sources: 16 rows 4.7 -> 3.1, 400 5.2 -> 3.3, 4096 15.0 -> 5.9; 10 sources: 400 8.0 -> 5.1
+//   bf16 1024, 3 sources: 16 rows 4.9 -> 3.5, 400 5.6 -> 3.8, 4096 17.1 -> 8.4; 10 sources: 400 9.2 -> 6.7
+//   fp32  512, 6 sources: 16 rows 5.7 -> 3.7, 400 6.3 -> 3.9, 4096 27.5 -> 11.5
+// and behind it where they do not and the row goes to attn_res_norm_kernel:
+//   fp32 1024, 10 sources: 400 rows 9.7 -> 12.0;  fp32 2048, 6: 400 rows 11.8 -> 17.6, 2048 37.3 -> 37.3
 constexpr int64_t kResSplitRows = 4096;
 
 template <typename T, int NPAD>

@@ -38,14 +38,17 @@ from torch import nn
 from diff_gpt import _native
 from diff_gpt.model.kv_cache import KVCache
 
-# A prefill whose attention output has at least this many bytes applies the
-# sigmoid gate as the attention kernel stores it (dg_prefill_rope_gate):
-# 32 MiB, the 8 XCDs' L2s together.  Above, a gate launch of its own reads and
-# writes y through memory once more (n_embd 512 in bf16: the sub-layer over
-# 256 x 1024 rows, y 256 MiB, 1417 us apart and 1324 fused, a layer over
-# 64 x 1024, y 64 MiB, 930 and 899); below, y is still in the L2s when that
-# launch reads it, and the ungated output stays available to the launches that
-# gate it themselves.
+# A prefill whose attention output y has at least this many bytes applies the
+# sigmoid gate as the attention kernel stores it (dg_prefill_rope_gate), with the
+# bits of a gate launch of its own, which reads and writes y once more: 32 MiB,
+# the 8 XCDs' L2s together.  A layer, us, gate apart -> fused, by the size of y:
+#   n_embd  512 bf16   64 MiB  844 ->  830   48  656 ->  637
+#          below the line  31  426 ->  414   24  354 ->  341   16  241 ->  235    8  146 ->  142    1  73.1 -> 72.0
+#   n_embd  512 fp32   48 MiB 1490 -> 1479   31 1025 -> 1012   16  537 ->  527    2   165 ->  165
+#   n_embd 1024 bf16   48 MiB  784 ->  765   31  513 ->  498   16  299 ->  289    2   108 ->  106
+# So the line is a safe one, not where the two are even: below it the fused form
+# is ahead by 1 - 4 % too, down to about 1 MiB (0.25 MiB: 44.6 -> 45.4, where
+# dg_linear_rows takes the gate in front of c_proj).
 _FUSED_GATE_BYTES = 32 << 20
 
 
