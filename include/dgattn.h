@@ -307,8 +307,9 @@ DG_API int dg_decode_attention_at(int B, int H, int D, int dtype,
  * So it is in bf16 / fp16 at D 64 or 128 (group >= 16, 16-byte aligned rows)
  * where the shared key reads B * H * P repay the matrix-core kernel's fixed
  * chain: B * H >= 320, 2 P >= m and B * H * P >= 3300 m + 200000 with
- * m = max_pos - P; the probabilities enter the products there as two values of
- * the data type, so y agrees with the two calls within rounding.
+ * m = max_pos - P; the probabilities enter the products there as three values
+ * of the data type, all their fp32 bits, so y agrees with the two calls within
+ * the rounding of fp32 sums in another order.
  * Where the attention runs on the vector kernel (every other shape whose
  * rows, projections and table are aligned to its lane slices) it is one
  * launch too: each (row, head) wave rotates q and k itself, the wave whose
