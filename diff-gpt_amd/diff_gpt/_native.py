@@ -884,7 +884,8 @@ def block_out_(y: torch.Tensor, g: torch.Tensor, w_proj: torch.Tensor, partial_i
                                      or not tail.ids.is_contiguous()):
             raise ValueError("block_out: ids must be a contiguous int64 tensor of the rows")
         if tail.w_mix is None:
-            rc = lib().dg_block_out_head(*args, _ptr(x2 if tail.keep_norm else None), C, n, _ptr(tail.w), tail.w.stride(0), float(tail.cap),
+            norm = x2 if tail.keep_norm else None
+            rc = lib().dg_block_out_head(*args, _ptr(norm), C, n, _ptr(tail.w), tail.w.stride(0), float(tail.cap),
                                          _ptr(t2), n, _ptr(tail.ids), _ptr(tail.advance), _stream(o2))
         elif x2 is None:
             t_mix = tail.w_mix.reshape(-1).contiguous()

@@ -41,12 +41,12 @@ def _empty_rows(x: torch.Tensor) -> torch.Tensor:
 
 def _few_rows(x: torch.Tensor, w: torch.Tensor, tile: int, *others: torch.Tensor | None) -> bool:
     """Whether F.linear(x, w) and the elementwise work around it, with the tensors
-    ``others``, go to dg_linear_rows: where F.linear would be the plain product --
-    autograd records nothing, autocast changes no type, the weight has no class of
-    its own that would answer for it -- and for 16-bit products whose workgroups, of 32 rows and ``tile``
-    features, times K stay within 256 x 1024, K at most 1024 (512 for the FFN's
-    first product).  Beyond, its tiles read the operands too often.  us, the
-    separate launches -> one, bf16:
+    ``others``, go to dg_linear_rows: where F.linear would be the plain product
+    (autograd records nothing, autocast changes no type, the weight has no class
+    of its own that would answer for it), in 16-bit types, with workgroups, of 32
+    rows and ``tile`` features, that times K stay within 256 x 1024, K at most 1024
+    (512 for the FFN's first product).  Beyond, its tiles read the operands too
+    often.  us, the separate launches -> one, bf16:
       gate, c_proj, sum    n_embd  512: 64 rows 9.5 -> 6.2, 512 9.0 -> 6.4, 2048 10.9 -> 16.1
                            n_embd 1024: 64 rows 10.8 -> 8.9, 256 10.7 -> 9.3, 400 11.6 -> 15.9
       FFN up, SwiGLU       n_embd  512: 64 rows 7.9 -> 5.5, 512 9.2 -> 8.2, 768 11.0 -> 11.4
