@@ -47,7 +47,7 @@ def _few_rows(x: torch.Tensor, w: torch.Tensor, tile: int, *others: torch.Tensor
     rows and ``tile`` features, that times K stay within 256 x 1024, K at most 1024
     (512 for the FFN's first product).  Beyond, its tiles read the operands too
     often.  us, the separate launches -> one, bf16:
-      gate, c_proj, sum    n_embd  512: 64 rows 9.5 -> 6.2, 512 9.0 -> 6.4, 2048 10.9 -> 16.1
+      gate, c_proj, sum    n_embd  512: 64 rows 9.5 -> 6.3, 512 9.0 -> 6.5, 1024 9.9 -> 9.2, 1056 10.1 -> 12.3
                            n_embd 1024: 64 rows 10.8 -> 8.9, 256 10.7 -> 9.3, 400 11.6 -> 15.9
       FFN up, SwiGLU       n_embd  512: 64 rows 7.9 -> 5.5, 512 9.2 -> 8.2, 768 11.0 -> 11.4
                            n_embd 1024: 16 rows 6.6 -> 7.5, 200 10.8 -> 13.7
