@@ -12,14 +12,12 @@
 //     D = 128).  S^T (16 keys x 16 rows) = K Q^T on v_mfma_f32_16x16x32, lane
 //     (c, g) = (l & 15, l >> 4) getting row c's scores of keys 4g .. 4g + 3; then
 //     O^T (16 dims x 16 rows) += V^T P^T, the lane's scores of two key tiles
-//     being its operand as they stand.  P enters as three terms of the data
-//     type, each the rounding error of those before it: all 24 bits of the fp32
-//     probability (of fp16's, what lies above 2^-41), with exact products and
-//     fp32 sums.  The second and third terms have an accumulator of their own,
-//     added at the end where the first one's is finite, so an infinite V gives
-//     the infinity that an fp32 probability would.  V goes to LDS by direct
-//     copies (16-byte pieces XOR-swizzled by row, 8 KB per wave, no barrier) and
-//     comes back transposed (ds_read_b64_tr_b16).
+//     being its operand as they stand.  P enters as three terms of the data type
+//     (split_pair): all 24 bits of the fp32 probability (of fp16's, what lies above
+//     2^-41), with exact products and fp32 sums, and an infinite V gives the
+//     infinity that an fp32 probability would.  V goes to LDS by direct copies
+//     (16-byte pieces XOR-swizzled by row, 8 KB per wave, no barrier) and comes
+//     back transposed (ds_read_b64_tr_b16).
 //   * each wave first takes the own keys of two of the 16 rows, half a wave per
 //     row, as the vector kernel does (D / 8 lanes of 16 bytes per key), appends
 //     their new key and value, and adds the new key from registers at the end.
@@ -27,11 +25,11 @@
 //     merge the 8 prefix parts and the row's own part.
 //
 // All row tiles of one (group, head) run on one XCD, so its L2 holds their
-// prefix once.  Those 400 rows with 40 own keys: 56 us in the vector kernel, 15.6
+// prefix once.  Those 400 rows with 40 own keys: 56 us in the vector kernel, 15.5
 // here (15.0 with two terms of P, 19.2 with fp32 P and V on
 // v_mfma_f32_16x16x4_f32).  What bounds it then is the latency of two chains in a
 // workgroup, 64-key chunks of the prefix and 16-key trips over the own keys (48
-// own keys after a 3000-token prefix: 21 us for 100 rows, 26 for 400); from some
+// own keys after a 3000-token prefix: 21 us for 100 rows, 25 for 400); from some
 // 6000 rows of 8 heads the rows' own K/V from HBM.  The error against float64 is
 // the vector kernel's (400 rows, 1024 + 40 keys: 1.646443e-3 of the norm in bf16,
 // 2.064455e-4 in fp16, either kernel).
@@ -92,6 +90,44 @@ __device__ __forceinline__ float half_sum_groups(float v) {
   return a + b;
 }
 
+// A pair of probabilities as three terms of T whose sum they are, packed.
+// bf16: the bits in three runs of eight, none negative, and the second and third
+// at least 2^-126, so that no term of a probability above that makes a NaN of an
+// infinite value and all three go into one sum (rounded terms, some of them
+// negative, and a second sum for them took the registers of a wave's loads: 400
+// rows over 1024 + 40 keys of 8 x 128 26.9 us, 25.0 so).
+// fp16: each the rounding error of those before it, the second and third scaled by
+// kRest, since the type's exponents end at 2^-24 (a first term's rounding error is
+// at most 2^-12 of 2^kLazyLog2); they have a sum of their own.
+constexpr float kRest = 65536.0f;
+template <typename T>
+__device__ __forceinline__ void split_pair(float p0, float p1, uint32_t (&term)[3]) {
+#pragma clang fp contract(off)
+  if constexpr (__is_same(T, bf16_t)) {
+    typedef uint16_t u16x2_t __attribute__((ext_vector_type(2)));
+    auto top = [](float a, float b) __attribute__((always_inline)) {
+      return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
+    };
+    auto rest = [](float a) __attribute__((always_inline)) {
+      return a - __uint_as_float(__float_as_uint(a) & 0xffff0000u);
+    };
+    auto positive = [](uint32_t w) __attribute__((always_inline)) {
+      const u16x2_t least = {0x0080, 0x0080};
+      return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2_t, w), least));
+    };
+    const float r0 = rest(p0), r1 = rest(p1);
+    term[0] = top(p0, p1);
+    term[1] = positive(top(r0, r1));
+    term[2] = positive(top(rest(r0), rest(r1)));
+  } else {
+    RowRegs<T, 2> t0, t1;
+    t0.w[0] = term[0] = pack_pair<T>(p0, p1);
+    const float r0 = (p0 - elem<T, 2>(t0, 0)) * kRest, r1 = (p1 - elem<T, 2>(t0, 1)) * kRest;
+    t1.w[0] = term[1] = pack_pair<T>(r0, r1);
+    term[2] = pack_pair<T>(r0 - elem<T, 2>(t1, 0), r1 - elem<T, 2>(t1, 1));
+  }
+}
+
 template <typename T, typename FT, int D>
 __global__ __launch_bounds__(64 * kWideWaves, 4) void attn_wide_kernel(const WideArgs a) {
   constexpr int NC = D / 32;       // contraction steps of Q K^T
@@ -102,9 +138,8 @@ __global__ __launch_bounds__(64 * kWideWaves, 4) void attn_wide_kernel(const Wid
   constexpr int KPH = 32 / LPK;    // keys per half-wave and slot
   constexpr int U = 4;             // slots per trip
   constexpr int PPR = D / 8;       // 16-byte pieces of a V row
-  // scale of a probability's second and third terms: fp16's exponents end at
-  // 2^-24, and a first term's rounding error is at most 2^-12 of 2^kLazyLog2
-  constexpr float kRest = __is_same(T, f16_t) ? 65536.0f : 1.0f;
+  constexpr int kSums = __is_same(T, f16_t) ? 2 : 1;  // accumulators of a block of O^T
+  constexpr int NR = kSums == 2 ? NB : 1;
   using Row = RowRegs<T, 8>;
   __shared__ __attribute__((aligned(16))) uint16_t stage[kWideWaves][4096];  // V, then the part's acc
   __shared__ __attribute__((aligned(16))) float own_acc[kWideRows][D];
@@ -283,9 +318,9 @@ __global__ __launch_bounds__(64 * kWideWaves, 4) void attn_wide_kernel(const Wid
   const int t16 = lane & 15;
 
   float m = kNegInf, l = 0.f;
-  f32x4_t o[NB], rest[NB];
+  f32x4_t o[NB], rest[NR];
 #pragma unroll
-  for (int nb = 0; nb < NB; ++nb) o[nb] = rest[nb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  for (int nb = 0; nb < NB; ++nb) o[nb] = rest[nb % NR] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   for (int k0 = wv * KC; k0 < plen; k0 += kWideWaves * KC) {
     // every lane is done reading the chunk before (its products waited for
     // the reads) when the copies of this one go out
@@ -332,7 +367,7 @@ __global__ __launch_bounds__(64 * kWideWaves, 4) void attn_wide_kernel(const Wid
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           o[nb][r] *= alpha;
-          rest[nb][r] *= alpha;
+          if constexpr (kSums == 2) rest[nb][r] *= alpha;
         }
     }
     const float moff = m * cl;
@@ -345,13 +380,10 @@ __global__ __launch_bounds__(64 * kWideWaves, 4) void attn_wide_kernel(const Wid
         const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[u][2 * w + 1], cl, -moff));
         l += p0;
         l += p1;
-        RowRegs<T, 2> term[3];
-        term[0].w[0] = pack_pair<T>(p0, p1);
-        const float r0 = (p0 - elem<T, 2>(term[0], 0)) * kRest, r1 = (p1 - elem<T, 2>(term[0], 1)) * kRest;
-        term[1].w[0] = pack_pair<T>(r0, r1);
-        term[2].w[0] = pack_pair<T>(r0 - elem<T, 2>(term[1], 0), r1 - elem<T, 2>(term[1], 1));
+        uint32_t term[3];
+        split_pair<T>(p0, p1, term);
 #pragma unroll
-        for (int k = 0; k < 3; ++k) p[u / 2][k][2 * (u & 1) + w] = term[k].w[0];
+        for (int k = 0; k < 3; ++k) p[u / 2][k][2 * (u & 1) + w] = term[k];
       }
     // this wave's V copies are in LDS
     __builtin_amdgcn_s_waitcnt(0);
@@ -370,8 +402,9 @@ __global__ __launch_bounds__(64 * kWideWaves, 4) void attn_wide_kernel(const Wid
         }
         const u32x4_t vf = {vv[0].x, vv[0].y, vv[1].x, vv[1].y};
         o[nb] = wide_mma<T>(vf, p[t][0], o[nb]);
-        rest[nb] = wide_mma<T>(vf, p[t][1], rest[nb]);
-        rest[nb] = wide_mma<T>(vf, p[t][2], rest[nb]);
+        f32x4_t& low = kSums == 2 ? rest[nb % NR] : o[nb];
+        low = wide_mma<T>(vf, p[t][1], low);
+        low = wide_mma<T>(vf, p[t][2], low);
       }
   }
   float x, y;
@@ -390,10 +423,10 @@ __global__ __launch_bounds__(64 * kWideWaves, 4) void attn_wide_kernel(const Wid
     float w[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      // a value that is not finite has made the first terms' sum so, and the
-      // others' (whose terms are zero or negative for some keys) a NaN
+      // a value that is not finite has made the first terms' sum so, and a sum
+      // of the others' own (zero or negative for some keys) a NaN
       const bool finite = __builtin_fabsf(o[nb][r]) < __builtin_huge_valf();
-      w[r] = finite ? __builtin_fmaf(rest[nb][r], 1.0f / kRest, o[nb][r]) : o[nb][r];
+      w[r] = kSums == 2 && finite ? __builtin_fmaf(rest[nb % NR][r], 1.0f / kRest, o[nb][r]) : o[nb][r];
     }
     store_vec<float, 4>(part + c * D + 4 * ((4 * nb + g) ^ (c & (UPR - 1))), w);
   }
